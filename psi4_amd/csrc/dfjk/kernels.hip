@@ -108,12 +108,29 @@ __global__ __launch_bounds__(256) void k_j1(BS B, const double* __restrict__ W, 
     }
 }
 
-__global__ void k_j1_reduce(const double* __restrict__ dpart, int ntp, int naux, double* __restrict__ d) {
-    const int Q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (Q >= naux) return;
+// d_Q = sum over the tile pairs of the partials.  64 Q per workgroup, the tile pairs dealt to 16
+// waves (a wave's loads are 512 contiguous bytes, several in flight), their sums added in LDS in a
+// fixed order.  Bound by latency: one thread per Q walking every pair took 70 us at 171 pairs /
+// 2784 Q and 33 us at 78 / 1856; this takes 5 us at both.
+constexpr int kJ1Groups = 16;
+__global__ __launch_bounds__(64 * kJ1Groups) void k_j1_reduce(const double* __restrict__ dpart, int ntp, int naux,
+                                                             double* __restrict__ d) {
+    __shared__ double red[kJ1Groups][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int Q = blockIdx.x * 64 + lane;
     double s = 0.0;
-    for (int t = 0; t < ntp; ++t) s += dpart[static_cast<size_t>(t) * naux + Q];
-    d[Q] = s;
+    if (Q < naux) {
+#pragma unroll 8
+        for (int t = grp; t < ntp; t += kJ1Groups) s += dpart[static_cast<size_t>(t) * naux + Q];
+    }
+    red[grp][lane] = s;
+    __syncthreads();
+    if (grp == 0 && Q < naux) {
+        double v = red[0][lane];
+#pragma unroll
+        for (int g = 1; g < kJ1Groups; ++g) v += red[g][lane];
+        d[Q] = v;
+    }
 }
 
 // J partials over a chunk of Q: grid = (ntp, nchunk), 256 threads, 4 consecutive elements per
@@ -147,26 +164,47 @@ __global__ __launch_bounds__(256) void k_j2(BS B, const double* __restrict__ d, 
     for (int k = 0; k < 4; ++k) o[k] = a[k];
 }
 
-__global__ void k_j_unpack(const double* __restrict__ Jpart, int nchunk, int ntp, const int* __restrict__ tidx,
-                           int nT, int nbf, double* __restrict__ J, int ldJ, double alpha, int accumulate) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = blockIdx.y;
-    if (n >= nbf) return;
-    int I = m / TILE, Jt = n / TILE, r = m % TILE, c = n % TILE;
-    if (I > Jt) {
-        int tmp = I;
-        I = Jt;
-        Jt = tmp;
-        tmp = r;
-        r = c;
-        c = tmp;
-    }
-    const int t = tidx[I * nT + Jt];
+// J from the partials of every Q chunk.  A workgroup sums 128 elements (4 rows) of one tile, the
+// chunks dealt to 8 groups of threads and added in LDS in a fixed order, and writes each element
+// with its mirror image, so J is exactly symmetric.  Bound by latency at small sizes: one thread
+// per element of J walking every chunk took 145 us at nbf 96 (464 chunks) and 36 us at nbf 576
+// (24 chunks); this takes 9 us and 11 us.  Tiles that are not stored stay at the caller's zeros
+// (or are zeroed by k_j_clear when not accumulating).
+constexpr int kJuGroups = 8;
+__global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(const double* __restrict__ Jpart, int nchunk, int ntp,
+                                                             const int2* __restrict__ tiles, int nbf,
+                                                             double* __restrict__ J, int ldJ, double alpha,
+                                                             int accumulate) {
+    __shared__ double red[kJuGroups][128];
+    const int t = blockIdx.x, el = threadIdx.x & 127, grp = threadIdx.x >> 7;
+    const int e = blockIdx.y * 128 + el;
     double s = 0.0;
-    if (t >= 0)
-        for (int ch = 0; ch < nchunk; ++ch) s += Jpart[(static_cast<size_t>(ch) * ntp + t) * TILE2 + r * TILE + c];
+#pragma unroll 4
+    for (int c = grp; c < nchunk; c += kJuGroups) s += Jpart[(static_cast<size_t>(c) * ntp + t) * TILE2 + e];
+    red[grp][el] = s;
+    __syncthreads();
+    if (grp != 0) return;
+    double v = red[0][el];
+#pragma unroll
+    for (int g = 1; g < kJuGroups; ++g) v += red[g][el];
+    const int2 IJ = tiles[t];
+    const int m = IJ.x * TILE + e / TILE, n = IJ.y * TILE + e % TILE;
+    if (m >= nbf || n >= nbf || m > n) return;  // the lower triangle of a diagonal tile is its mirror image
     double* o = J + static_cast<size_t>(m) * ldJ + n;
-    *o = alpha * s + (accumulate ? *o : 0.0);
+    *o = alpha * v + (accumulate ? *o : 0.0);
+    if (m != n) {
+        double* ot = J + static_cast<size_t>(n) * ldJ + m;
+        *ot = alpha * v + (accumulate ? *ot : 0.0);
+    }
+}
+// J = 0 on the 32 x 32 blocks that have no stored tile
+__global__ void k_j_clear(const int* __restrict__ tidx, int nT, int nbf, double* __restrict__ J, int ldJ) {
+    const int I = blockIdx.y, Jt = blockIdx.x;
+    if (tidx[min(I, Jt) * nT + max(I, Jt)] >= 0) return;
+    for (int e = threadIdx.x; e < TILE2; e += blockDim.x) {
+        const int m = I * TILE + e / TILE, n = Jt * TILE + e % TILE;
+        if (m < nbf && n < nbf) J[static_cast<size_t>(m) * ldJ + n] = 0.0;
+    }
 }
 
 // ------------------------------------------------------------------ K path
@@ -239,43 +277,61 @@ __global__ __launch_bounds__(256) void k_gemm_nt_f64(const double* __restrict__ 
             }
 }
 
-__global__ void k_tile_reduce(const double* __restrict__ P, int nsplit, int ntile, const int* __restrict__ tile_of,
-                              int nB, int sym, int M, int N, double* __restrict__ out, int ldo, double alpha,
-                              int accumulate) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    const int m = blockIdx.y;
-    if (n >= N) return;
-    int Ib = m >> 7, Jb = n >> 7, r = m & 127, c = n & 127;
+// Sum of the split partials into the dense result.  A workgroup owns a 16 x 16 output block, the
+// splits dealt to 4 groups of 256 threads and added in LDS in a fixed order.  With sym only the
+// blocks on and above the diagonal run and write their mirror image too.  Bound by latency at small
+// sizes and by HBM at large ones: one thread per output element walking every split, both triangles
+// read separately, took 154 us at nbf 96 (464 splits), 301 us at nbf 576 (136 splits of 15 tiles)
+// and 360 us in the cross form there; this takes 18, 42 and 59 us.
+constexpr int kTrGroups = 4;
+__global__ __launch_bounds__(256 * kTrGroups) void k_tile_reduce(const double* __restrict__ P, int nsplit, int ntile,
+                                                                const int* __restrict__ tile_of, int nB, int sym, int M,
+                                                                int N, double* __restrict__ out, int ldo, double alpha,
+                                                                int accumulate) {
+    const int bj = blockIdx.x, bi = blockIdx.y;
+    if (sym && bi > bj) return;
+    __shared__ double s1[kTrGroups][256], s2[kTrGroups][16][17];
+    const int el = threadIdx.x & 255, grp = threadIdx.x >> 8;
+    const int r = el >> 4, c = el & 15;
+    const int t1 = tile_of[(bi >> 3) * nB + (bj >> 3)];
+    const size_t o1 = static_cast<size_t>((bi & 7) * 16 + r) * 128 + (bj & 7) * 16 + c;
+    double a = 0.0, b = 0.0;
+    if (t1 >= 0) {
+        const double* p = P + static_cast<size_t>(t1) * 16384 + o1;
+#pragma unroll 8
+        for (int sp = grp; sp < nsplit; sp += kTrGroups) a += p[static_cast<size_t>(sp) * ntile * 16384];
+    }
+    s1[grp][el] = a;
     if (sym == 2) {
-        // out = M + M^T from the partials of every tile; (m,n) and (n,m) add the same two
-        // split sums in either order, so the result is exactly symmetric
-        const int t1 = tile_of[Ib * nB + Jb], t2 = tile_of[Jb * nB + Ib];
-        double s1 = 0.0, s2 = 0.0;
-        for (int sp = 0; sp < nsplit; ++sp) {
-            if (t1 >= 0) s1 += P[(static_cast<size_t>(sp) * ntile + t1) * 16384 + r * 128 + c];
-            if (t2 >= 0) s2 += P[(static_cast<size_t>(sp) * ntile + t2) * 16384 + c * 128 + r];
+        // the mirror block of the cross form, M^T
+        const int t2 = tile_of[(bj >> 3) * nB + (bi >> 3)];
+        const size_t o2 = static_cast<size_t>((bj & 7) * 16 + r) * 128 + (bi & 7) * 16 + c;
+        if (t2 >= 0) {
+            const double* p = P + static_cast<size_t>(t2) * 16384 + o2;
+#pragma unroll 8
+            for (int sp = grp; sp < nsplit; sp += kTrGroups) b += p[static_cast<size_t>(sp) * ntile * 16384];
         }
-        double* o = out + static_cast<size_t>(m) * ldo + n;
-        const double v = m <= n ? s1 + s2 : s2 + s1;
-        *o = alpha * v + (accumulate ? *o : 0.0);
-        return;
+        s2[grp][r][c] = b;
     }
-    // symmetric: read the upper triangle only (also inside diagonal tiles), so the
-    // result is exactly symmetric whatever the accumulation order of the tile
-    if (sym && (Ib > Jb || (Ib == Jb && r > c))) {
-        int tmp = Ib;
-        Ib = Jb;
-        Jb = tmp;
-        tmp = r;
-        r = c;
-        c = tmp;
+    __syncthreads();
+    if (grp != 0) return;
+    double v = s1[0][el];
+#pragma unroll
+    for (int g = 1; g < kTrGroups; ++g) v += s1[g][el];
+    if (sym == 2) {
+        double w = s2[0][c][r];
+#pragma unroll
+        for (int g = 1; g < kTrGroups; ++g) w += s2[g][c][r];
+        v += w;
     }
-    const int t = tile_of[Ib * nB + Jb];
-    double s = 0.0;
-    if (t >= 0)
-        for (int sp = 0; sp < nsplit; ++sp) s += P[(static_cast<size_t>(sp) * ntile + t) * 16384 + r * 128 + c];
+    const int m = bi * 16 + r, n = bj * 16 + c;
+    if (m >= M || n >= N || (sym && m > n)) return;
     double* o = out + static_cast<size_t>(m) * ldo + n;
-    *o = alpha * s + (accumulate ? *o : 0.0);
+    *o = alpha * v + (accumulate ? *o : 0.0);
+    if (sym && m != n) {
+        double* ot = out + static_cast<size_t>(n) * ldo + m;
+        *ot = alpha * v + (accumulate ? *ot : 0.0);
+    }
 }
 
 // Row-major C = alpha*A*B + beta*C, 128x128 output tiles, FP64 MFMA, 4 waves of 64x64.
@@ -440,7 +496,7 @@ void launch_j1(const TileGeom& g, const JSource& B, const double* W, int naux, i
 }
 
 void launch_j1_reduce(const TileGeom& g, const double* dpart, int naux, double* d, hipStream_t s) {
-    hipLaunchKernelGGL(k_j1_reduce, grid1(naux, 256), dim3(256), 0, s, dpart, g.ntp, naux, d);
+    hipLaunchKernelGGL(k_j1_reduce, grid1(naux, 64), dim3(64 * kJ1Groups), 0, s, dpart, g.ntp, naux, d);
 }
 
 void launch_j2(const TileGeom& g, const JSource& B, const double* d, int naux, int qchunk, double* Jpart,
@@ -455,10 +511,11 @@ void launch_j2(const TileGeom& g, const JSource& B, const double* d, int naux, i
 
 void launch_j_unpack(const TileGeom& g, const double* Jpart, int nchunk, double* J, int ldJ, double alpha,
                      int accumulate, hipStream_t s) {
-    require(ldJ >= g.nbf, "j_unpack ld");
-    dim3 grid((g.nbf + 255) / 256, g.nbf);
-    hipLaunchKernelGGL(k_j_unpack, grid, dim3(256), 0, s, Jpart, nchunk, g.ntp, g.d_tidx, g.nT, g.nbf, J, ldJ, alpha,
-                       accumulate);
+    require(ldJ >= g.nbf && g.ntp > 0 && nchunk > 0, "j_unpack");
+    if (!accumulate && g.ntp < g.nT * (g.nT + 1) / 2)
+        hipLaunchKernelGGL(k_j_clear, dim3(g.nT, g.nT), dim3(256), 0, s, g.d_tidx, g.nT, g.nbf, J, ldJ);
+    hipLaunchKernelGGL(k_j_unpack, dim3(g.ntp, TILE2 / 128), dim3(128 * kJuGroups), 0, s, Jpart, nchunk, g.ntp,
+                       g.d_tiles, g.nbf, J, ldJ, alpha, accumulate);
 }
 
 void launch_pack_c(const double* Csrc, int ldsrc, int nbf, int ncol, double scale, double* Cpad, int nbfp, int ldc,
@@ -480,8 +537,8 @@ void launch_gemm_nt_f64(const double* A, size_t strideA, int lda, const double* 
 void launch_tile_reduce(const double* P, int nsplit, int ntile, const int* d_tile_of, int nB, int sym, int M, int N,
                         double* out, int ldo, double alpha, int accumulate, hipStream_t s) {
     require(M <= nB * 128 && N <= nB * 128 && ldo >= N, "tile_reduce");
-    dim3 grid((N + 255) / 256, M);
-    hipLaunchKernelGGL(k_tile_reduce, grid, dim3(256), 0, s, P, nsplit, ntile, d_tile_of, nB, sym, M, N, out, ldo,
+    dim3 grid((N + 15) / 16, (M + 15) / 16);
+    hipLaunchKernelGGL(k_tile_reduce, grid, dim3(256 * kTrGroups), 0, s, P, nsplit, ntile, d_tile_of, nB, sym, M, N, out, ldo,
                        alpha, accumulate);
 }
 
