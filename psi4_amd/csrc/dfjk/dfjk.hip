@@ -25,6 +25,7 @@
 #include "../ints/ints.hpp"
 #include "../ints/hostlinalg.hpp"
 #include "kernels.hpp"
+#include "kernels_f64.hpp"
 #include "kernels_ints.hpp"
 #include "kernels_k.hpp"
 #include "kernels_schwarz.hpp"
@@ -239,7 +240,7 @@ struct dfjk_handle {
     double bw_alpha = 1.0, bw_beta = 0.0;
     std::vector<double> fit_M;      // host metric factor, kept for rebuilding Bw after an omega change
     // workspace
-    DevBuf ws_craw, ws_cl, ws_cr, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_Pd, ws_J, ws_K, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap;
+    DevBuf ws_craw, ws_cl, ws_cr, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_Pd, ws_J, ws_K, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
     DevBuf ws_ct, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
     // column map of the half-transform: the device copy is re-uploaded (from pinned memory,
     // asynchronously) only when it changes
@@ -1228,9 +1229,14 @@ int* upload_cmap(dfjk_handle* h, const std::vector<int>& cmap, Work& wk) {
     return dmap;
 }
 
-// One density pair: Cl/Cr are device [nbf][ncol] row-major (ld = ncol).
-// Cr == nullptr: lr_symmetric.  Two structured non-symmetric forms are recognised
-// (bitwise column tests on the device) and kept symmetric:
+// One density pair: cl/cr are device [nbf][ncol] row-major (ld = ncol); cr == nullptr: lr_symmetric.
+struct PairIn {
+    const double *cl = nullptr, *cr = nullptr;
+    int ncol = 0;
+    double *D = nullptr, *J = nullptr, *K = nullptr;
+};
+// Two structured non-symmetric forms are recognised (bitwise column tests on the device) and kept
+// symmetric:
 //  * signed: every column of Cr is +/- the same column of Cl (the incremental
 //    C_left=[C_new,C_old], C_right=[C_new,-C_old] form).  K = sum_Q X_Q diag(s) X_Q^T:
 //    the columns are regrouped (+ first, then -), one half-transform is run and the
@@ -1238,11 +1244,407 @@ int* upload_cmap(dfjk_handle* h, const std::vector<int>& cmap, Work& wk) {
 //  * cross: Cl = [A, V], Cr = [V, A] (ncol even; dD = A V^T + V A^T, the form
 //    A = (C_new + C_old)/2, V = C_new - C_old of a density change, in which every
 //    product carries the small factor V).  K = sum_Q X_A X_V^T + X_V X_A^T: one
-//    half-transform of [A, V], two contractions of the upper block-triangle with the
-//    column halves swapped between the operands.
+//    half-transform of [A, V] and one contraction M = X_A X_V^T over every output block;
+//    the reduction forms M + M^T.
 // The cross form can also be declared (dfjk_set_pair_form), which skips the test.
-void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol, double* dD, double* dJ, double* dK,
-                  int accumulate, Work& wk) {
+struct PairForm {
+    bool sym = true, cross = false;
+    std::vector<int> plus, minus;  // symmetric pairs: columns with Cr = +Cl and Cr = -Cl
+    bool general() const { return !sym && !cross; }
+    bool is_signed() const { return sym && !minus.empty(); }
+};
+
+// Classify pairs (or take the declared form); the column tests of all pairs share one round trip.
+std::vector<PairForm> classify_pairs(dfjk_handle* h, const PairIn* pr, int np, Work& wk) {
+    const hipStream_t s = h->stream;
+    std::vector<PairForm> form(np);
+    size_t ntot = 0;
+    auto tested = [&](int p) { return pr[p].cr && h->pair_form == DFJK_FORM_DETECT; };
+    for (int p = 0; p < np; ++p) {
+        form[p].sym = pr[p].cr == nullptr;
+        if (pr[p].cr && h->pair_form == DFJK_FORM_CROSS) {
+            if (pr[p].ncol % 2) fail(DFJK_ERR_ARG, "JK: the cross pair form needs an even column count");
+            form[p].cross = true;
+        }
+        if (tested(p)) ntot += 2 * static_cast<size_t>(pr[p].ncol);
+    }
+    int8_t* sg = nullptr;
+    if (ntot) {
+        // shift 0 (signed form) and shift ncol/2 (cross form)
+        sg = wk.get<int8_t>(h->ws_sign, ntot);
+        size_t o = 0;
+        for (int p = 0; p < np; ++p) {
+            if (!tested(p)) continue;
+            const int nc = pr[p].ncol;
+            launch_column_signs(pr[p].cl, pr[p].cr, nc, h->nbf, nc, 0, sg + o, s);
+            if (nc % 2 == 0) launch_column_signs(pr[p].cl, pr[p].cr, nc, h->nbf, nc, nc / 2, sg + o + nc, s);
+            o += 2 * static_cast<size_t>(nc);
+        }
+        if (h->sign_pin_cap < ntot) {
+            if (wk.fixed()) fail(DFJK_ERR_MEMORY, "dfjk_compute_device_noalloc: too many columns for the structure test");
+            if (h->sign_pin) hcheck(hipHostFree(h->sign_pin), "hipHostFree");
+            h->sign_pin = nullptr;
+            h->sign_pin_cap = 0;
+            const size_t cap = std::max<size_t>(ntot, 4096);
+            hcheck(hipHostMalloc(reinterpret_cast<void**>(&h->sign_pin), cap, 0), "hipHostMalloc");
+            h->sign_pin_cap = cap;
+        }
+        hcheck(hipMemcpyAsync(h->sign_pin, sg, ntot, hipMemcpyDeviceToHost, s), "signs");
+        hcheck(hipStreamSynchronize(s), "signs");
+    }
+    size_t o = 0;
+    for (int p = 0; p < np; ++p) {
+        const int nc = pr[p].ncol;
+        PairForm& f = form[p];
+        std::vector<int> hs(nc, 1);
+        if (tested(p)) {
+            const int8_t* h8 = h->sign_pin + o;
+            o += 2 * static_cast<size_t>(nc);
+            f.sym = true;
+            for (int i = 0; i < nc; ++i) {
+                hs[i] = h8[i];
+                f.sym &= h8[i] != 0;
+            }
+            if (!f.sym && nc % 2 == 0) {
+                f.cross = true;
+                for (int i = 0; i < nc; ++i) f.cross &= h8[nc + i] == 1;
+            }
+        }
+        if (f.sym)
+            for (int i = 0; i < nc; ++i) (hs[i] >= 0 ? f.plus : f.minus).push_back(i);
+    }
+    return form;
+}
+
+// dfjk_compute_device_noalloc, before any launch: the buffers of fixed size, one K split and one
+// auxiliary function's X must fit the scratch array (X blocks and splits then adapt to the rest).
+void require_scratch(const dfjk_handle* h, int ncol, const Work& wk) {
+    if (h->ooc) fail(DFJK_ERR_STATE, "dfjk_compute_device_noalloc needs B in core");
+    const int nbf = h->nbf, xrows = (h->nT + 3) / 4 * 128;
+    auto r = [](size_t b) { return (std::max<size_t>(b, 256) + 255) / 256 * 256; };
+    int nbw_b, np_b, ldc_b;
+    ht_panel_shape(ncol + 64, &nbw_b, &np_b, &ldc_b);  // column groups are padded to 32 each
+    const size_t ldcb = static_cast<size_t>(ldc_b) + 320;
+    const size_t qsb = static_cast<size_t>(h->ntp) * TILE2, cszb = static_cast<size_t>(h->nbfp) * ldcb;
+    const size_t tiles = static_cast<size_t>(h->ntile_all) * 16384 * sizeof(double);
+    const size_t need = r(2 * static_cast<size_t>(ncol)) + r(ldcb * sizeof(int)) + 2 * r(cszb * 8) +
+                        r(static_cast<size_t>(nbf) * nbf * 8) + r(tiles) +                       // D
+                        r(qsb * 8) + r(static_cast<size_t>(h->naux) * 8) +                       // J: W, d
+                        r(static_cast<size_t>(h->ntp) * h->naux * 8) + r(qsb * 8) +             // J partials
+                        r(tiles) + r(8 * cszb) +                                                  // K split, C copies
+                        2 * r(static_cast<size_t>(xrows) * ldcb * 8) + 1024;                     // one Q of X
+    if (need > wk.cap)
+        fail(DFJK_ERR_MEMORY, "dfjk_compute_device_noalloc: nbf " + std::to_string(nbf) + ", naux " +
+                                  std::to_string(h->naux) + " and " + std::to_string(ncol) +
+                                  " columns need about " + std::to_string(need >> 20) + " MiB, beyond the " +
+                                  std::to_string(wk.cap >> 20) + " MiB scratch array");
+}
+
+ColGroups one_group(const double* src, int ncol, const double* partner) {
+    ColGroups cg;
+    cg.n = 1;
+    cg.ncb = (ncol + 15) / 16;
+    cg.g[0] = ColGroup{src, partner, nullptr, ncol, ncol, 0, cg.ncb};
+    return cg;
+}
+
+// D = Cl Cr^T (jk.cc:314-354), FP64: the contraction kernel over the columns of the packed C
+void compute_D(dfjk_handle* h, const double* dCl, const double* dCr, int ncol, double* D, Work& wk) {
+    const hipStream_t s = h->stream;
+    const bool sym = dCr == nullptr || dCr == dCl;
+    const int ncb = (ncol + 15) / 16, nk = (ncol + 7) / 8;
+    const size_t csz = static_cast<size_t>(h->nbfp) * 16 * ncb;
+    double* DL = wk.get<double>(h->ws_cl, csz);
+    launch_pack_frag(one_group(dCl, ncol, dCl), h->nbf, h->nbfp, nullptr, DL, s);
+    double* DR = DL;
+    if (!sym) {
+        DR = wk.get<double>(h->ws_cr, csz);
+        launch_pack_frag(one_group(dCr, ncol, dCr), h->nbf, h->nbfp, nullptr, DR, s);
+    }
+    const int nblk = kc_blocks(h->nT, sym);
+    int nsp = kc_choose_splits(h->nT, sym, nk, 1, 64);
+    if (wk.fixed()) nsp = 1;
+    double* P = wk.get<double>(h->ws_Pd, static_cast<size_t>(nsp) * nblk * 4096);
+    KcSegs sg;
+    sg.n = 1;
+    sg.nsplit = nsp;
+    sg.s[0] = KcSeg{0, nsp, 0, 0, nk, 1.0};
+    launch_kc_f64(DL, DR, 0, 2 * ncb, h->nT, 1, sg, sym, P, 0, s);
+    KcOuts o;
+    o.n = 1;
+    o.o[0] = KcOut{0, nsp, D};
+    launch_kc_reduce(P, h->nT, h->nbf, sym, o, 0, s);
+}
+
+// Chunks of the second J pass over nq auxiliary functions: about 4096 workgroups, at least four Q each
+// (a chunk's partial J is as large as one Q's tile).
+int j2_chunks(const dfjk_handle* h, int nq, int want_wg = 4096) {
+    return std::max(1, std::min((nq + 3) / 4, (want_wg + h->ntp - 1) / h->ntp));
+}
+
+int kc_steps(int nq, int nk) {
+    return static_cast<int>(std::min<long long>(static_cast<long long>(nq) * nk, 1 << 30));
+}
+// The K partials take at most a quarter of the X budget, but 256 MiB in any case
+int kc_most_splits(int nblk, size_t budget) {
+    const size_t room = std::max<size_t>(budget / 4, size_t(256) << 20);
+    return static_cast<int>(std::min<size_t>(1 << 20, std::max<size_t>(1, room / (static_cast<size_t>(nblk) * 4096 * 8))));
+}
+
+// out of core: host block blk (of qblk Q) -> stage buffer blk & 1
+void stage_block(dfjk_handle* h, int blk, int qblk) {
+    const size_t qs = static_cast<size_t>(h->ntp) * TILE2;
+    const int qa = h->aux_q0 + blk * qblk, nq = std::min(qblk, h->aux_q1 - qa);
+    double* dst = h->ws_stage[blk & 1].get<double>(qs * qblk);
+    hcheck(hipStreamWaitEvent(h->cstream, h->ev_free[blk & 1], 0), "wait stage");
+    hcheck(hipMemcpyAsync(dst, h->hB + static_cast<size_t>(qa) * qs, qs * nq * sizeof(double), hipMemcpyHostToDevice,
+                          h->cstream),
+           "stage B");
+    hcheck(hipEventRecord(h->ev_copied[blk & 1], h->cstream), "record");
+}
+
+// FP64 J and K of up to kMaxPairs pairs (every pair wants K; ncol > 0).  The columns of all pairs
+// lie side by side in one half-transform per Q-block, so B is read once for all of them, left
+// matrices that several pairs share (the same array) are transformed once, and d_Q = <B_Q, Cl Cr^T>
+// = <B_Q Cl, Cr> comes from X in the half-transform's epilogue instead of a pass over B: at nbf 576 /
+// naux 2784 that pass took 0.65 of 9.9 ms.  J's second pass and the contraction take all pairs in
+// one launch.
+void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& form, int np, int accumulate,
+                 Work& wk) {
+    const TileGeom g = h->geom();
+    const hipStream_t s = h->stream;
+    const int q0 = h->aux_q0, q1 = h->aux_q1, nq_total = q1 - q0;
+    const int nT = h->nT, nbf = h->nbf, nbfp = h->nbfp;
+    EventTimer& tm = h->timer;
+    for (int p = 0; p < np; ++p)
+        if (pr[p].D) {
+            hipEvent_t e0 = tm.begin();
+            const size_t mark = wk.used;
+            compute_D(h, pr[p].cl, pr[p].cr, pr[p].ncol, pr[p].D, wk);
+            wk.used = mark;  // D's operands are dead before the next kernel of this stream
+            tm.end(T_OTHER, e0);
+        }
+    // column groups, contraction passes and output blocks
+    ColGroups cg;
+    auto add = [&](const double* src, int ld, int ncol, const int* cmap, int ncolp, const double* partner) {
+        ColGroup& G = cg.g[cg.n];
+        G = ColGroup{src, partner, cmap, ld, ncol, cg.ncb, (ncolp + 15) / 16};
+        cg.ncb += G.ncb;
+        return cg.n++;
+    };
+    struct Pass {
+        int pair, ka, kb, nk;
+        double alpha;
+    };
+    std::vector<Pass> pass[2];  // [0]: upper blocks (symmetric results), [1]: every block
+    DRanges dr;
+    for (int p = 0; p < np; ++p) {
+        const PairIn& P = pr[p];
+        const PairForm& f = form[p];
+        const int nc = P.ncol;
+        int g0, dcb = 0;
+        if (f.is_signed()) {
+            const int kp = round_up(static_cast<int>(f.plus.size()), 8), km = round_up(static_cast<int>(f.minus.size()), 8);
+            std::vector<int> cmap(round_up(kp + km, 16), -1);
+            for (size_t i = 0; i < f.plus.size(); ++i) cmap[i] = f.plus[i];
+            for (size_t i = 0; i < f.minus.size(); ++i) cmap[kp + i] = f.minus[i];
+            g0 = add(P.cl, nc, nc, upload_cmap(h, cmap, wk), kp + km, P.cr);
+            const int k0 = 2 * cg.g[g0].cb0;
+            if (kp) pass[0].push_back({p, k0, k0, kp / 8, 1.0});
+            pass[0].push_back({p, k0 + kp / 8, k0 + kp / 8, km / 8, -1.0});
+            dcb = cg.g[g0].ncb;
+        } else if (f.sym) {
+            g0 = add(P.cl, nc, nc, nullptr, nc, P.cl);
+            const int k0 = 2 * cg.g[g0].cb0;
+            pass[0].push_back({p, k0, k0, (nc + 7) / 8, 1.0});
+            dcb = cg.g[g0].ncb;
+        } else if (f.cross) {
+            // [A, V] against [V, A]: the halves as two groups
+            const int half = nc / 2;
+            g0 = add(P.cl, nc, half, nullptr, half, P.cr);
+            const int g1 = add(P.cl + half, nc, half, nullptr, half, P.cr + half);
+            pass[1].push_back({p, 2 * cg.g[g0].cb0, 2 * cg.g[g1].cb0, (half + 7) / 8, 1.0});
+            dcb = cg.g[g0].ncb + cg.g[g1].ncb;
+        } else {
+            int gl = -1;
+            for (int i = 0; i < cg.n; ++i)
+                if (cg.g[i].src == P.cl && cg.g[i].ld == nc && cg.g[i].ncol == nc && !cg.g[i].cmap) gl = i;
+            if (gl < 0) gl = add(P.cl, nc, nc, nullptr, nc, nullptr);
+            g0 = add(P.cr, nc, nc, nullptr, nc, P.cl);
+            pass[1].push_back({p, 2 * cg.g[gl].cb0, 2 * cg.g[g0].cb0, (nc + 7) / 8, 1.0});
+            dcb = cg.g[g0].ncb;
+        }
+        dr.cb0[p] = cg.g[g0].cb0;
+        dr.ncb[p] = dcb;
+    }
+    dr.n = np;
+    int njp = 0;  // pairs whose J is wanted: all or none of a batch
+    for (int p = 0; p < np; ++p) njp += h->do_J && pr[p].J ? 1 : 0;
+    const bool doJ = njp > 0;
+    if (doJ && njp != np) fail(DFJK_ERR_INTERNAL, "J wanted for some pairs of a batch only");
+    const int ncb = cg.ncb, nkx = 2 * ncb;
+    const size_t csz = static_cast<size_t>(nbfp) * 16 * ncb, xq = csz, qs = static_cast<size_t>(h->ntp) * TILE2;
+    double* CA = wk.get<double>(h->ws_CA, csz);
+    double* CD = doJ ? wk.get<double>(h->ws_CD, csz) : nullptr;
+    launch_pack_frag(cg, nbf, nbfp, CA, CD, s);
+
+    double *dvec = nullptr, *Jpart = nullptr;
+    const int ldd = h->naux;
+    int jn = 0, jchunk = 0;
+    size_t jstride = 0;
+    auto size_j2 = [&](int nq, int want_wg) {
+        jn = j2_chunks(h, nq, want_wg);
+        jchunk = (nq + jn - 1) / jn;
+        jn = (nq + jchunk - 1) / jchunk;
+        jstride = static_cast<size_t>(jn) * qs;
+        Jpart = wk.get<double>(h->ws_Jpart, np * jstride);
+    };
+    if (doJ) {
+        dvec = wk.get<double>(h->ws_d, static_cast<size_t>(np) * ldd);  // at absolute Q (the adjoint reads it)
+        if (!h->ooc)
+            size_j2(nq_total, wk.fixed() ? static_cast<int>(std::max<size_t>(
+                                               h->ntp, std::min<size_t>(4096, wk.left() / 8 / (TILE2 * sizeof(double)))))
+                                         : 4096);
+    }
+    // Q-blocks
+    const size_t per_q = xq * sizeof(double);
+    int qblk = std::min(nq_total, 65535);
+    size_t budget = 0;
+    if (!wk.fixed()) {
+        budget = memory_limited(h, g_x_budget, ((h->ooc ? 0 : b_doubles(h)) + static_cast<size_t>(h->naux) * h->naux) *
+                                                   sizeof(double));
+        qblk = static_cast<int>(std::min<size_t>(qblk, std::max<size_t>(1, budget / per_q)));
+        if (h->ooc) {
+            // two stage buffers share the budget with X
+            const size_t pq = qs * 2 * sizeof(double);
+            const size_t stage_budget = std::max<size_t>(pq, std::min<size_t>(size_t(8) << 30, budget / 2));
+            qblk = std::min<int>(qblk, static_cast<int>(std::max<size_t>(1, stage_budget / pq)));
+        }
+    }
+    auto even_blocks = [&] {
+        const int nb = (nq_total + qblk - 1) / qblk;
+        qblk = (nq_total + nb - 1) / nb;
+    };
+    even_blocks();
+    // splits of every pass; a launch's splits are numbered through its passes
+    KcSegs segs[2];
+    size_t poff[2] = {0, 0}, psize = 0;
+    for (int k = 0; k < 2; ++k) {
+        const int nseg = static_cast<int>(pass[k].size());
+        const int nblk = kc_blocks(nT, k == 0);
+        poff[k] = psize;
+        for (const Pass& ps : pass[k]) {
+            int nsp = kc_choose_splits(nT, k == 0, kc_steps(qblk, ps.nk), nseg, kc_most_splits(nblk * nseg, budget));
+            if (wk.fixed())
+                nsp = static_cast<int>(std::max<size_t>(
+                    1, std::min<size_t>(nsp, wk.left() / 4 / (static_cast<size_t>(nblk) * 4096 * sizeof(double) * nseg))));
+            segs[k].s[segs[k].n++] = KcSeg{segs[k].nsplit, nsp, ps.ka, ps.kb, ps.nk, ps.alpha};
+            segs[k].nsplit += nsp;
+        }
+        psize += static_cast<size_t>(segs[k].nsplit) * nblk * 4096;
+    }
+    double* P = wk.get<double>(h->ws_P, psize);
+    int ncross = 0;
+    for (int p = 0; p < np; ++p) ncross += form[p].cross ? 1 : 0;
+    const size_t nn = static_cast<size_t>(nbf) * nbf;
+    double* M = ncross ? wk.get<double>(h->ws_M, ncross * nn) : nullptr;
+    int rt = ht_row_tiles(nT, qblk, ncb);
+    const size_t dq = static_cast<size_t>(ht_row_groups(nT, 1)) * ncb;  // d partials per Q, at most
+    if (wk.fixed()) {
+        const size_t room = wk.left() > 1024 ? wk.left() - 1024 : 0;  // alignment of X and the d partials
+        qblk = static_cast<int>(std::min<size_t>(qblk, room / (per_q + dq * sizeof(double))));
+        if (qblk < 1)
+            fail(DFJK_ERR_MEMORY, "dfjk_compute_device_noalloc: one auxiliary function's half-transform does not "
+                                  "fit the " + std::to_string(wk.cap >> 20) + " MiB scratch array");
+        even_blocks();
+        rt = ht_row_tiles(nT, qblk, ncb);
+    }
+    const int nrg = ht_row_groups(nT, rt);
+    double* X = wk.get<double>(h->ws_XL, xq * qblk);
+    double* dpart = doJ ? wk.get<double>(h->ws_dpart, dq * qblk) : nullptr;
+    const int nblocks = (nq_total + qblk - 1) / qblk;
+    if (doJ && h->ooc) size_j2(qblk, 4096);
+    JOut jout{};
+    for (int p = 0; p < np; ++p) jout.J[p] = pr[p].J;
+    if (h->ooc) {
+        // both stage buffers start free
+        for (int i = 0; i < 2; ++i) hcheck(hipEventRecord(h->ev_free[i], s), "record");
+        stage_block(h, 0, qblk);
+    }
+    for (int blk = 0; blk < nblocks; ++blk) {
+        const int qa = q0 + blk * qblk, nq = std::min(qblk, q1 - qa);
+        const double* b64;
+        if (!h->ooc) {
+            b64 = h->dB.as<double>() + static_cast<size_t>(qa) * qs;
+        } else {
+            if (blk + 1 < nblocks) stage_block(h, blk + 1, qblk);
+            hcheck(hipStreamWaitEvent(s, h->ev_copied[blk & 1], 0), "wait copy");
+            b64 = h->ws_stage[blk & 1].as<double>();
+        }
+        hipEvent_t e0 = tm.begin();
+        launch_ht_f64(g, b64, nq, CA, CD, ncb, rt, X, dpart, h->dZero.p, s);
+        tm.end(T_HT, e0);
+        h->n_ht += 1;
+        if (doJ) {
+            hipEvent_t ej = tm.begin();
+            launch_dpart_reduce(dpart, nq, nrg, ncb, dr, dvec + qa, ldd, s);
+            if (h->ooc) {
+                const int nch = (nq + jchunk - 1) / jchunk;
+                launch_j2(g, JSource{JSource::F64, b64}, dvec + qa, ldd, np, nq, jchunk, Jpart, jstride, s);
+                launch_j_unpack(g, Jpart, jstride, nch, jout, np, nbf, 1.0, (blk > 0 || accumulate) ? 1 : 0, s);
+            }
+            tm.end(T_J, ej);
+        }
+        hipEvent_t e1 = tm.begin();
+        for (int k = 0; k < 2; ++k)
+            if (segs[k].n) {
+                launch_kc_f64(X, X, xq, nkx, nT, nq, segs[k], k == 0, P + poff[k], blk > 0 ? 1 : 0, s);
+                h->n_kgemm += 1;
+            }
+        tm.end(T_KGEMM, e1);
+        if (h->ooc) hcheck(hipEventRecord(h->ev_free[blk & 1], s), "record");
+    }
+    if (doJ && !h->ooc) {
+        hipEvent_t ej = tm.begin();
+        launch_j2(g, JSource{JSource::F64, h->dB.as<double>() + static_cast<size_t>(q0) * qs}, dvec + q0, ldd, np,
+                  nq_total, jchunk, Jpart, jstride, s);
+        launch_j_unpack(g, Jpart, jstride, jn, jout, np, nbf, 1.0, accumulate, s);
+        tm.end(T_J, ej);
+    }
+    hipEvent_t e2 = tm.begin();
+    for (int k = 0; k < 2; ++k) {
+        if (!segs[k].n) continue;
+        KcOuts outs;
+        int im = 0;
+        for (int i = 0; i < segs[k].n; ++i) {
+            const int p = pass[k][i].pair;
+            if (i > 0 && pass[k][i - 1].pair == p) {  // a signed pair's second pass: the same output
+                outs.o[outs.n - 1].nsp += segs[k].s[i].nsp;
+                continue;
+            }
+            double* out = form[p].cross ? M + nn * im++ : pr[p].K;
+            outs.o[outs.n++] = KcOut{segs[k].s[i].sp0, segs[k].s[i].nsp, out};
+        }
+        // the cross form's M is complete before it is added to K with its transpose
+        KcOuts cross, plain;
+        for (int i = 0, j = 0; i < segs[k].n; ++i) {
+            const int p = pass[k][i].pair;
+            if (i > 0 && pass[k][i - 1].pair == p) continue;
+            (form[p].cross ? cross : plain).o[(form[p].cross ? cross : plain).n++] = outs.o[j++];
+        }
+        if (plain.n) launch_kc_reduce(P + poff[k], nT, nbf, k == 0, plain, accumulate, s);
+        if (cross.n) launch_kc_reduce(P + poff[k], nT, nbf, k == 0, cross, 0, s);
+    }
+    for (int p = 0, im = 0; p < np; ++p)
+        if (form[p].cross) launch_add_transpose(M + nn * im++, nbf, pr[p].K, accumulate, s);
+    tm.end(T_OTHER, e2);
+}
+
+// One density pair in the mixed precisions, or J alone in FP64.
+void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int accumulate, Work& wk) {
+    const double *dCl = in.cl, *dCr = in.cr;
+    const int ncol = in.ncol;
+    double *dJ = in.J, *dK = in.K;
     const TileGeom g = h->geom();
     const hipStream_t s = h->stream;
     const int q0 = h->aux_q0, q1 = h->aux_q1;
@@ -1250,113 +1652,16 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
     const int nbf = h->nbf, nbfp = h->nbfp;
     const int xrows = (h->nT + 3) / 4 * 128;
     EventTimer& tm = h->timer;
-    if (wk.fixed() && h->ooc) fail(DFJK_ERR_STATE, "dfjk_compute_device_noalloc needs B in core");
-    if (wk.fixed()) {
-        // Before any launch: the buffers of fixed size, one K split and one auxiliary
-        // function's X must fit the scratch array (X blocks and splits then adapt to the rest).
-        auto r = [](size_t b) { return (std::max<size_t>(b, 256) + 255) / 256 * 256; };
-        int nbw_b, np_b, ldc_b;
-        ht_panel_shape(ncol + 64, &nbw_b, &np_b, &ldc_b);  // column groups are padded to 32 each
-        const size_t ldcb = static_cast<size_t>(ldc_b) + 320;
-        const size_t qsb = static_cast<size_t>(h->ntp) * TILE2, cszb = static_cast<size_t>(nbfp) * ldcb;
-        const size_t tiles = static_cast<size_t>(h->ntile_all) * 16384 * sizeof(double);
-        const size_t need = r(2 * static_cast<size_t>(ncol)) + r(ldcb * sizeof(int)) + 2 * r(cszb * 8) +
-                            r(static_cast<size_t>(nbf) * nbf * 8) + r(tiles) +                       // D
-                            r(qsb * 8) + r(static_cast<size_t>(h->naux) * 8) +                       // J: W, d
-                            r(static_cast<size_t>(h->ntp) * h->naux * 8) + r(qsb * 8) +             // J partials
-                            r(tiles) + r(8 * cszb) +                                                  // K split, C copies
-                            2 * r(static_cast<size_t>(xrows) * ldcb * 8) + 1024;                     // one Q of X
-        if (need > wk.cap)
-            fail(DFJK_ERR_MEMORY, "dfjk_compute_device_noalloc: nbf " + std::to_string(nbf) + ", naux " +
-                                      std::to_string(h->naux) + " and " + std::to_string(ncol) +
-                                      " columns need about " + std::to_string(need >> 20) + " MiB, beyond the " +
-                                      std::to_string(wk.cap >> 20) + " MiB scratch array");
-    }
-
-    // classify the pair (or take the declared form) and build the column map
-    bool sym = (dCr == nullptr), cross = false;
-    std::vector<int> hs(ncol, 1);
-    if (!sym && h->pair_form == DFJK_FORM_CROSS) {
-        if (ncol % 2) fail(DFJK_ERR_ARG, "JK: the cross pair form needs an even column count");
-        cross = true;
-    } else if (!sym && h->pair_form == DFJK_FORM_DETECT) {
-        // both column tests in one round trip: shift 0 (signed form), shift ncol/2 (cross form)
-        const int ntest = ncol % 2 == 0 ? 2 : 1;
-        int8_t* sg = wk.get<int8_t>(h->ws_sign, 2 * static_cast<size_t>(ncol));
-        launch_column_signs(dCl, dCr, ncol, nbf, ncol, 0, sg, s);
-        if (ntest == 2) launch_column_signs(dCl, dCr, ncol, nbf, ncol, ncol / 2, sg + ncol, s);
-        if (h->sign_pin_cap < 2 * static_cast<size_t>(ncol)) {
-            if (wk.fixed()) fail(DFJK_ERR_MEMORY, "dfjk_compute_device_noalloc: too many columns for the structure test");
-            if (h->sign_pin) hcheck(hipHostFree(h->sign_pin), "hipHostFree");
-            h->sign_pin = nullptr;
-            h->sign_pin_cap = 0;
-            const size_t cap = std::max<size_t>(2 * static_cast<size_t>(ncol), 4096);
-            hcheck(hipHostMalloc(reinterpret_cast<void**>(&h->sign_pin), cap, 0), "hipHostMalloc");
-            h->sign_pin_cap = cap;
-        }
-        hcheck(hipMemcpyAsync(h->sign_pin, sg, static_cast<size_t>(ntest) * ncol, hipMemcpyDeviceToHost, s), "signs");
-        hcheck(hipStreamSynchronize(s), "signs");
-        const int8_t* h8 = h->sign_pin;
-        bool allpm = true;
-        for (int i = 0; i < ncol; ++i) {
-            hs[i] = h8[i];
-            allpm &= h8[i] != 0;
-        }
-        sym = allpm;
-        if (!sym && ntest == 2) {
-            cross = true;
-            for (int i = 0; i < ncol; ++i) cross &= h8[ncol + i] == 1;
-            if (cross) std::fill(hs.begin(), hs.end(), 1);
-        }
-    }
-    const bool general = !sym && !cross;
-    std::vector<int> plus, minus;
-    for (int i = 0; i < ncol; ++i) (hs[i] >= 0 ? plus : minus).push_back(i);
-    const bool signed_sym = sym && !minus.empty();
-    int ncol_eff = ncol, kplus = 0, half = 0, wcross = 0;
-    std::vector<int> cmap;
-    if (signed_sym) {
-        kplus = round_up(static_cast<int>(plus.size()), 32);
-        ncol_eff = kplus + round_up(static_cast<int>(minus.size()), 32);
-    } else if (cross) {
-        half = ncol / 2;
-        wcross = round_up(half, 32);
-        ncol_eff = 2 * wcross;
-    }
-    int nbw, npanel, ldc;
-    ht_panel_shape(ncol_eff, &nbw, &npanel, &ldc);
-    cmap.assign(ldc, -1);
-    if (signed_sym) {
-        for (size_t i = 0; i < plus.size(); ++i) cmap[i] = plus[i];
-        for (size_t i = 0; i < minus.size(); ++i) cmap[kplus + i] = minus[i];
-    } else if (cross) {
-        for (int i = 0; i < half; ++i) {
-            cmap[i] = i;
-            cmap[wcross + i] = half + i;
-        }
-    } else {
-        for (int i = 0; i < ncol; ++i) cmap[i] = i;
-    }
-    int* dmap = upload_cmap(h, cmap, wk);
-
-    double* cl = wk.get<double>(h->ws_cl, static_cast<size_t>(nbfp) * ldc);
-    launch_pack_cmap_f64(dCl, ncol, nbf, dmap, cl, nbfp, ldc, s);
-    double* cr = cl;
-    if (dCr) {
-        cr = wk.get<double>(h->ws_cr, static_cast<size_t>(nbfp) * ldc);
-        launch_pack_cmap_f64(dCr, ncol, nbf, dmap, cr, nbfp, ldc, s);
-    }
+    const bool sym = form.sym, cross = form.cross, general = form.general(), signed_sym = form.is_signed();
+    const std::vector<int>&plus = form.plus, &minus = form.minus;
 
     // D = Cl Cr^T (jk.cc:314-354), FP64
-    const bool need_D = (dD != nullptr) || (h->do_J && dJ != nullptr);
-    double* Dm = dD;
+    const bool need_D = (in.D != nullptr) || (h->do_J && dJ != nullptr);
+    double* Dm = in.D;
     if (need_D) {
         hipEvent_t e0 = tm.begin();
         if (!Dm) Dm = wk.get<double>(h->ws_D, static_cast<size_t>(nbf) * nbf);
-        double* P = wk.get<double>(h->ws_Pd, static_cast<size_t>(h->ntile_all) * 16384);
-        launch_gemm_nt_f64(cl, 0, ldc, cr, 0, ldc, nbf, nbf, ldc, 1, 1, h->d_otiles_all.as<int2>(), h->ntile_all, P, 0,
-                           s);
-        launch_tile_reduce(P, 1, h->ntile_all, h->d_otile_of_all.as<int>(), h->nB, 0, nbf, nbf, Dm, nbf, 1.0, 0, s);
+        compute_D(h, dCl, dCr, ncol, Dm, wk);
         tm.end(T_OTHER, e0);
     }
 
@@ -1370,6 +1675,36 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
     const bool doK = h->do_K && dK;
     if (!doJ && !doK) return;
     const int prec = h->precision;
+    if (doK && prec == DFJK_PREC_FP64) fail(DFJK_ERR_INTERNAL, "FP64 K outside compute_f64");
+
+    // column map of the half-transform
+    int ncol_eff = ncol, kplus = 0, half = 0, wcross = 0;
+    if (signed_sym) {
+        kplus = round_up(static_cast<int>(plus.size()), 32);
+        ncol_eff = kplus + round_up(static_cast<int>(minus.size()), 32);
+    } else if (cross) {
+        half = ncol / 2;
+        wcross = round_up(half, 32);
+        ncol_eff = 2 * wcross;
+    }
+    int nbw, npanel, ldc;
+    ht_panel_shape(ncol_eff, &nbw, &npanel, &ldc);
+    int* dmap = nullptr;
+    if (doK) {
+        std::vector<int> cmap(ldc, -1);
+        if (signed_sym) {
+            for (size_t i = 0; i < plus.size(); ++i) cmap[i] = plus[i];
+            for (size_t i = 0; i < minus.size(); ++i) cmap[kplus + i] = minus[i];
+        } else if (cross) {
+            for (int i = 0; i < half; ++i) {
+                cmap[i] = i;
+                cmap[wcross + i] = half + i;
+            }
+        } else {
+            for (int i = 0; i < ncol; ++i) cmap[i] = i;
+        }
+        dmap = upload_cmap(h, cmap, wk);
+    }
     const size_t qs = static_cast<size_t>(h->ntp) * TILE2;  // elements per Q
     const size_t xq = static_cast<size_t>(xrows) * ldc;      // X elements per Q
     const size_t esz = prec == DFJK_PREC_FP64 ? 8 : 4;       // FP64, FP32, or BF16 hi+lo
@@ -1403,7 +1738,7 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
             if (wk.fixed())
                 want_wg = static_cast<int>(std::max<size_t>(
                     h->ntp, std::min<size_t>(4096, wk.left() / 8 / (TILE2 * sizeof(double)))));
-            jnchunk = std::max(1, std::min(nq_total, (want_wg + h->ntp - 1) / h->ntp));
+            jnchunk = j2_chunks(h, nq_total, want_wg);
             qchunk = (h->naux + jnchunk - 1) / jnchunk;
             jnchunk = (h->naux + qchunk - 1) / qchunk;
             Jpart = wk.get<double>(h->ws_Jpart, static_cast<size_t>(jnchunk) * qs);
@@ -1511,8 +1846,7 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
     if (doJ && h->ooc) {
         // out of core: d_Q partials and J partials per streamed block
         dpart = wk.get<double>(h->ws_dpart, static_cast<size_t>(h->ntp) * qblk);
-        const int want_wg = 4096;
-        jnchunk = std::max(1, std::min(qblk, (want_wg + h->ntp - 1) / h->ntp));
+        jnchunk = j2_chunks(h, qblk);
         jchunk = (qblk + jnchunk - 1) / jnchunk;
         jnchunk = (qblk + jchunk - 1) / jchunk;
         Jpart = wk.get<double>(h->ws_Jpart, static_cast<size_t>(jnchunk) * qs);
@@ -1537,24 +1871,14 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
         if (q0 > 0 || q1 < h->naux) launch_zero(dpart, static_cast<size_t>(h->ntp) * h->naux, s);
         launch_j1(g, js, W, h->naux, q0, q1, dpart, s);
         launch_j1_reduce(g, dpart, h->naux, dvec, s);
-        launch_j2(g, js, dvec, h->naux, qchunk, Jpart, s);
-        launch_j_unpack(g, Jpart, jnchunk, dJ, nbf, 1.0, accumulate, s);
+        launch_j2(g, js, dvec, h->naux, 1, h->naux, qchunk, Jpart, 0, s);
+        launch_j_unpack(g, Jpart, 0, jnchunk, JOut{{dJ}}, 1, nbf, 1.0, accumulate, s);
         tm.end(T_J, e0);
     }
-    auto stage_copy = [&](int blk) {  // out of core: host block -> stage buffer blk & 1
-        const int qa = q0 + blk * qblk;
-        const int nq = std::min(qblk, q1 - qa);
-        double* dst = wk.get<double>(h->ws_stage[blk & 1], qs * qblk);
-        hcheck(hipStreamWaitEvent(h->cstream, h->ev_free[blk & 1], 0), "wait stage");
-        hcheck(hipMemcpyAsync(dst, h->hB + static_cast<size_t>(qa) * qs, qs * nq * sizeof(double),
-                              hipMemcpyHostToDevice, h->cstream),
-               "stage B");
-        hcheck(hipEventRecord(h->ev_copied[blk & 1], h->cstream), "record");
-    };
     if (h->ooc) {
         // both stage buffers start free
         for (int i = 0; i < 2; ++i) hcheck(hipEventRecord(h->ev_free[i], s), "record");
-        stage_copy(0);
+        stage_block(h, 0, qblk);
     }
 
     for (int blk = 0; blk < nblocks; ++blk) {
@@ -1570,7 +1894,7 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
             if (prec != DFJK_PREC_FP64) b32 = h->dB32.as<float>() + off;
             if (prec == DFJK_PREC_BF16X3 && doK) b32t = h->dB32T.as<float>() + off;
         } else {
-            if (blk + 1 < nblocks) stage_copy(blk + 1);
+            if (blk + 1 < nblocks) stage_block(h, blk + 1, qblk);
             hcheck(hipStreamWaitEvent(s, h->ev_copied[blk & 1], 0), "wait copy");
             double* st = h->ws_stage[blk & 1].as<double>();
             b64 = st;
@@ -1600,21 +1924,15 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
             const int nch = (nq + jchunk - 1) / jchunk;
             launch_j1(g, js, W, nq, 0, nq, dpart, s);
             launch_j1_reduce(g, dpart, nq, dvec + qa, s);
-            launch_j2(g, js, dvec + qa, nq, jchunk, Jpart, s);
-            launch_j_unpack(g, Jpart, nch, dJ, nbf, 1.0, (blk > 0 || accumulate) ? 1 : 0, s);
+            launch_j2(g, js, dvec + qa, h->naux, 1, nq, jchunk, Jpart, 0, s);
+            launch_j_unpack(g, Jpart, 0, nch, JOut{{dJ}}, 1, nbf, 1.0, (blk > 0 || accumulate) ? 1 : 0, s);
             tm.end(T_J, e0);
         }
 
         if (doK) {
             const int nsp = std::min(nsplit, nq);
             hipEvent_t e0 = tm.begin();
-            if (prec == DFJK_PREC_FP64) {
-                launch_ht2_f64(g, b64, 0, nq, cl, ldc, nbw, npanel, reinterpret_cast<double*>(XL), xrows, h->dZero.p,
-                               s);
-                if (general)
-                    launch_ht2_f64(g, b64, 0, nq, cr, ldc, nbw, npanel, reinterpret_cast<double*>(XR), xrows,
-                                   h->dZero.p, s);
-            } else if (prec == DFJK_PREC_FP32) {
+            if (prec == DFJK_PREC_FP32) {
                 launch_ht2_f32(g, b32, 0, nq, c32l, ldc, nbw, npanel, reinterpret_cast<float*>(XL), xrows, h->dZero.p,
                                s);
                 if (general)
@@ -1634,12 +1952,7 @@ void compute_pair(dfjk_handle* h, const double* dCl, const double* dCr, int ncol
             for (size_t ip = 0; ip < passes.size(); ++ip) {
                 const Pass& pp = passes[ip];
                 const int acc = (blk > 0 || ip > 0) ? 1 : 0;
-                if (prec == DFJK_PREC_FP64) {
-                    double* xl = reinterpret_cast<double*>(XL) + pp.offl;
-                    double* xr = reinterpret_cast<double*>(XR) + pp.offr;
-                    launch_kgemm2_f64(xl, xr, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp, otiles, ntile, P, pp.alpha,
-                                      acc, upper ? 1 : 0, s);
-                } else if (prec == DFJK_PREC_FP32) {
+                if (prec == DFJK_PREC_FP32) {
                     float* xl = reinterpret_cast<float*>(XL) + pp.offl;
                     float* xr = reinterpret_cast<float*>(XR) + pp.offr;
                     launch_kgemm2_f32(xl, xr, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp, otiles, ntile, P, pp.alpha,
@@ -1677,22 +1990,13 @@ void compute_wk_pair(dfjk_handle* h, const double* dCl, const double* dCr, int n
     const int q0 = h->aux_q0, q1 = h->aux_q1;
     const int nq_total = q1 - q0;
     const int nbf = h->nbf, nbfp = h->nbfp;
-    const int xrows = (h->nT + 3) / 4 * 128;
     EventTimer& tm = h->timer;
-    int nbw, npanel, ldc;
-    ht_panel_shape(ncol, &nbw, &npanel, &ldc);
-    std::vector<int> cmap(ldc, -1);
-    for (int i = 0; i < ncol; ++i) cmap[i] = i;
-    Work alloc_wk;
-    int* dmap = upload_cmap(h, cmap, alloc_wk);
-    double* cl = h->ws_cl.get<double>(static_cast<size_t>(nbfp) * ldc);
-    launch_pack_cmap_f64(dCl, ncol, nbf, dmap, cl, nbfp, ldc, s);
-    double* cr = cl;
-    if (dCr) {
-        cr = h->ws_cr.get<double>(static_cast<size_t>(nbfp) * ldc);
-        launch_pack_cmap_f64(dCr, ncol, nbf, dmap, cr, nbfp, ldc, s);
-    }
-    const size_t xq = static_cast<size_t>(xrows) * ldc;
+    const int ncb = (ncol + 15) / 16, nk = (ncol + 7) / 8, nT = h->nT;
+    const size_t xq = static_cast<size_t>(nbfp) * 16 * ncb, qs = static_cast<size_t>(h->ntp) * TILE2;
+    double* cl = h->ws_CA.get<double>((dCr ? 2 : 1) * xq);
+    double* cr = dCr ? cl + xq : cl;
+    launch_pack_frag(one_group(dCl, ncol, nullptr), nbf, nbfp, cl, nullptr, s);
+    if (dCr) launch_pack_frag(one_group(dCr, ncol, nullptr), nbf, nbfp, cr, nullptr, s);
     const size_t budget = memory_limited(
         h, g_x_budget, (2 * b_doubles(h) + static_cast<size_t>(h->naux) * h->naux) * sizeof(double));
     const size_t per_q = 2 * xq * sizeof(double);
@@ -1700,34 +2004,35 @@ void compute_wk_pair(dfjk_handle* h, const double* dCl, const double* dCr, int n
     qblk = std::min(qblk, 65535);
     const int nblocks = (nq_total + qblk - 1) / qblk;
     qblk = (nq_total + nblocks - 1) / nblocks;
-    const int ntile = h->ntile_all;
-    const int2* otiles = h->d_otiles_all.as<int2>();
-    const int nsplit = choose_nsplit(ntile, qblk);
-    double* P = h->ws_P.get<double>(static_cast<size_t>(nsplit) * ntile * 16384);
-    const int kend = std::min(ldc, round_up(ncol, 16));
+    const int nsp = kc_choose_splits(nT, false, kc_steps(qblk, nk), 1, kc_most_splits(kc_blocks(nT, false), budget));
+    double* P = h->ws_P.get<double>(static_cast<size_t>(nsp) * kc_blocks(nT, false) * 4096);
     double* XL = h->ws_XL.get<double>(xq * qblk);
     double* XR = h->ws_XR.get<double>(xq * qblk);
+    const int rt = ht_row_tiles(nT, qblk, ncb);
+    KcSegs sg;
+    sg.n = 1;
+    sg.nsplit = nsp;
+    sg.s[0] = KcSeg{0, nsp, 0, 0, nk, 1.0};
     for (int blk = 0; blk < nblocks; ++blk) {
         const int qa = q0 + blk * qblk;
         const int nq = std::min(qblk, q1 - qa);
-        const int nsp = std::min(nsplit, nq);
         hipEvent_t e0 = tm.begin();
-        launch_ht2_f64(g, h->dB.as<double>(), qa, nq, cl, ldc, nbw, npanel, XL, xrows, h->dZero.p, s);
-        launch_ht2_f64(g, h->dBw.as<double>(), qa, nq, cr, ldc, nbw, npanel, XR, xrows, h->dZero.p, s);
+        launch_ht_f64(g, h->dB.as<double>() + static_cast<size_t>(qa) * qs, nq, cl, nullptr, ncb, rt, XL, nullptr,
+                      h->dZero.p, s);
+        launch_ht_f64(g, h->dBw.as<double>() + static_cast<size_t>(qa) * qs, nq, cr, nullptr, ncb, rt, XR, nullptr,
+                      h->dZero.p, s);
         tm.end(T_HT, e0);
         h->n_ht += 2;
         hipEvent_t e1 = tm.begin();
-        launch_kgemm2_f64(XL, XR, xq, xrows, nbf, ldc, 0, kend, nq, nsp, otiles, ntile, P, 1.0, blk > 0 ? 1 : 0, 0, s);
+        launch_kc_f64(XL, XR, xq, 2 * ncb, nT, nq, sg, false, P, blk > 0 ? 1 : 0, s);
         h->n_kgemm += 1;
-        if (nsp < nsplit && blk == 0)
-            hcheck(hipMemsetAsync(P + static_cast<size_t>(nsp) * ntile * 16384, 0,
-                                  sizeof(double) * static_cast<size_t>(nsplit - nsp) * ntile * 16384, s),
-                   "memset");
         tm.end(T_KGEMM, e1);
     }
     hipEvent_t e2 = tm.begin();
-    launch_tile_reduce(P, nsplit, ntile, h->d_otile_of_all.as<int>(), h->nB, 0, nbf, nbf, dwK, nbf, 1.0, accumulate,
-                       s);
+    KcOuts out;
+    out.n = 1;
+    out.o[0] = KcOut{0, nsp, dwK};
+    launch_kc_reduce(P, nT, nbf, false, out, accumulate, s);
     tm.end(T_OTHER, e2);
 }
 
@@ -1750,6 +2055,74 @@ void reset_timers(dfjk_handle* h) {
     ensure_stream(h);
 }
 
+// J, K (and D) of a batch of pairs whose pointers are the caller's (device or host).
+void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool device, char* arena,
+               size_t arena_bytes) {
+    const size_t nn = static_cast<size_t>(h->nbf) * h->nbf;
+    const int np = static_cast<int>(batch.size());
+    std::vector<PairIn> pr(batch);
+    if (!device) {
+        // operands to the device, an array that several pairs share once
+        size_t csum = 0;
+        for (const PairIn& p : batch) csum += (p.cr ? 2 : 1) * static_cast<size_t>(h->nbf) * p.ncol;
+        double* raw = h->ws_craw.get<double>(csum);
+        std::vector<std::pair<std::pair<const double*, int>, double*>> seen;
+        auto up = [&](const double* c, int ncol, const char* what) -> const double* {
+            for (const auto& e : seen)
+                if (e.first.first == c && e.first.second == ncol) return e.second;
+            const size_t csz = static_cast<size_t>(h->nbf) * ncol;
+            copy_settled(raw, c, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, what);
+            seen.push_back({{c, ncol}, raw});
+            raw += csz;
+            return seen.back().second;
+        };
+        double* gD = h->ws_D.get<double>(nn * np);
+        double* gJ = h->ws_J.get<double>(nn * np);
+        double* gK = h->ws_K.get<double>(nn * np);
+        for (int i = 0; i < np; ++i) {
+            pr[i].cl = up(batch[i].cl, batch[i].ncol, "upload C_left");
+            if (batch[i].cr) pr[i].cr = up(batch[i].cr, batch[i].ncol, "upload C_right");
+            if (batch[i].D) pr[i].D = gD + nn * i;
+            if (batch[i].J) pr[i].J = gJ + nn * i;
+            if (batch[i].K) pr[i].K = gK + nn * i;
+            if (accumulate) {
+                if (batch[i].J) copy_settled(pr[i].J, batch[i].J, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
+                if (batch[i].K) copy_settled(pr[i].K, batch[i].K, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
+            }
+        }
+    }
+    Work wk;  // per batch: the batches run in stream order, so a fixed arena is reused
+    wk.base = arena;
+    wk.cap = arena_bytes;
+    if (wk.fixed())
+        for (const PairIn& p : pr) require_scratch(h, p.ncol, wk);
+    const std::vector<PairForm> form = classify_pairs(h, pr.data(), np, wk);
+    const bool f64 = h->precision == DFJK_PREC_FP64 && h->do_K && pr[0].K;
+    if (f64) {
+        // a signed pair's column map is the handle's: such a pair runs alone
+        for (int i = 0; i < np;) {
+            int j = i + 1;
+            if (!form[i].is_signed())
+                while (j < np && !form[j].is_signed()) ++j;
+            compute_f64(h, pr.data() + i, std::vector<PairForm>(form.begin() + i, form.begin() + j), j - i, accumulate,
+                        wk);
+            i = j;
+        }
+    } else {
+        for (int i = 0; i < np; ++i) compute_pair(h, pr[i], form[i], accumulate, wk);
+    }
+    if (!device) {
+        for (int i = 0; i < np; ++i) {
+            if (batch[i].D) copy_settled(batch[i].D, pr[i].D, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download D");
+            if (batch[i].J && h->do_J)
+                copy_settled(batch[i].J, pr[i].J, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download J");
+            if (batch[i].K && h->do_K)
+                copy_settled(batch[i].K, pr[i].K, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download K");
+        }
+        hcheck(hipStreamSynchronize(h->stream), "compute");
+    }
+}
+
 // arena: null for the allocating entry points, else the device address of this device's
 // static scratch array (dfjk_compute_device_noalloc; device pointers only, no timing events)
 void compute_impl(dfjk_handle* h, int n, const double* const* Cl, const double* const* Cr, const int* ncol,
@@ -1766,6 +2139,14 @@ void compute_impl(dfjk_handle* h, int n, const double* const* Cl, const double* 
     } restore{h, timing};
     reset_timers(h);
     const size_t nn = static_cast<size_t>(h->nbf) * h->nbf;
+    // The pairs in order, in batches of up to kMaxPairs.  Pairs of a batch share the passes over B
+    // (FP64 with K; the fixed workspace takes them one by one).
+    std::vector<PairIn> batch;   // caller's pointers
+    auto flush = [&] {
+        if (batch.empty()) return;
+        run_batch(h, batch, accumulate, device, arena, arena_bytes);
+        batch.clear();
+    };
     for (int i = 0; i < n; ++i) {
         if (ncol[i] < 0) fail(DFJK_ERR_ARG, "JK: negative column count");
         if (!Cl[i] && ncol[i] > 0) fail(DFJK_ERR_ARG, "JK: null C_left matrix");
@@ -1785,6 +2166,7 @@ void compute_impl(dfjk_handle* h, int n, const double* const* Cl, const double* 
             dK = nullptr;
         }
         if (ncol[i] == 0) {
+            flush();  // outputs are written in the order of the pairs
             // psi4: D = 0, J += 0, K skipped for nocc == 0 (dfhelper.cc:3355-3358)
             if (device) {
                 if (dD) launch_zero(dD, nn, h->stream);
@@ -1797,39 +2179,24 @@ void compute_impl(dfjk_handle* h, int n, const double* const* Cl, const double* 
             }
             continue;
         }
-        const size_t csz = static_cast<size_t>(h->nbf) * ncol[i];
-        const double* cl = Cl[i];
-        const double* cr = Cr ? Cr[i] : nullptr;
-        double *gD = dD, *gJ = dJ, *gK = dK;
-        if (!device) {
-            double* raw = h->ws_craw.get<double>(2 * csz);
-            copy_settled(raw, cl, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload C_left");
-            cl = raw;
-            if (cr) {
-                copy_settled(raw + csz, cr, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload C_right");
-                cr = raw + csz;
-            }
-            gD = dD ? h->ws_D.get<double>(nn) : nullptr;
-            gJ = dJ ? h->ws_J.get<double>(nn) : nullptr;
-            gK = dK ? h->ws_K.get<double>(nn) : nullptr;
-            if (accumulate) {
-                if (gJ) copy_settled(gJ, dJ, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
-                if (gK) copy_settled(gK, dK, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
-            }
-        }
-        Work wk;  // per pair: the pairs run in stream order, so a fixed arena is reused
-        wk.base = arena;
-        wk.cap = arena_bytes;
-        compute_pair(h, cl, cr, ncol[i], gD, gJ, gK, accumulate, wk);
-        if (!device) {
-            if (dD) copy_settled(dD, gD, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download D");
-            if (dJ && h->do_J)
-                copy_settled(dJ, gJ, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download J");
-            if (dK && h->do_K)
-                copy_settled(dK, gK, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download K");
-            hcheck(hipStreamSynchronize(h->stream), "compute");
-        }
+        PairIn p;
+        p.cl = Cl[i];
+        p.cr = Cr ? Cr[i] : nullptr;
+        p.ncol = ncol[i];
+        p.D = dD;
+        p.J = dJ;
+        p.K = dK;
+        // a pair that reads or writes what an earlier one of its batch writes waits for it
+        bool clash = false;
+        for (const PairIn& o : batch)
+            for (const double* w : {o.D, o.J, o.K})
+                clash |= w && (w == p.cl || w == p.cr || w == p.D || w == p.J || w == p.K);
+        const bool alone = arena || h->precision != DFJK_PREC_FP64 || !h->do_K || !p.K;
+        if (alone || clash || (!batch.empty() && (p.J == nullptr) != (batch[0].J == nullptr))) flush();
+        batch.push_back(p);
+        if (alone || static_cast<int>(batch.size()) == kMaxPairs) flush();
     }
+    flush();
     finish_timers(h);
 }
 
@@ -1916,7 +2283,13 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
     h->do_J = h->do_K = true;
     try {
         Work wk;
-        compute_pair(h, dC, nullptr, nocc, D, Jm, Km, 0, wk);
+        PairIn in;
+        in.cl = dC;
+        in.ncol = nocc;
+        in.D = D;
+        in.J = Jm;
+        in.K = Km;
+        compute_f64(h, &in, classify_pairs(h, &in, 1, wk), 1, 0, wk);
     } catch (...) {
         h->aux_q0 = uq0, h->aux_q1 = uq1, h->precision = prec, h->do_J = dj, h->do_K = dk;
         throw;
@@ -2485,7 +2858,7 @@ int dfjk_finalize(dfjk_handle* h) {
                         &h->ws_Jpart, &h->ws_XL, &h->ws_XR,  &h->ws_P,    &h->ws_Pd, &h->ws_J,     &h->ws_K,
                         &h->ws_G,    &h->ws_sign, &h->ws_c32, &h->ws_cbf, &h->ws_cmap, &h->ws_ct,   &h->ws_red,
                         &h->ws_Y,    &h->ws_PC,  &h->ws_gam, &h->ws_dc, &h->ws_stage[0], &h->ws_stage[1],
-                        &h->ws_stage32, &h->ws_stage32t};
+                        &h->ws_stage32, &h->ws_stage32t, &h->ws_CA, &h->ws_CD, &h->ws_M};
         for (DevBuf* b : ws) b->release();
         h->cmap_dev.clear();
         h->dM_ready = false;

@@ -134,34 +134,44 @@ __global__ __launch_bounds__(64 * kJ1Groups) void k_j1_reduce(const double* __re
 }
 
 // J partials over a chunk of Q: grid = (ntp, nchunk), 256 threads, 4 consecutive elements per
-// thread (vector loads), two Q per pass.
-template <class BS>
-__global__ __launch_bounds__(256) void k_j2(BS B, const double* __restrict__ d, int ntp, int naux, int qchunk,
-                                            double* __restrict__ Jpart) {
+// thread (vector loads), two Q per pass.  NP densities share the pass over B (d[p * ldd + Q], partials
+// at Jpart + p * pstride): bound by reading B, so a second density costs next to nothing.
+template <class BS, int NP>
+__global__ __launch_bounds__(256) void k_j2(BS B, const double* __restrict__ d, int ldd, int ntp, int naux, int qchunk,
+                                            double* __restrict__ Jpart, size_t pstride) {
     const int t = blockIdx.x, c = blockIdx.y;
     const int qa = c * qchunk, qb = min(naux, qa + qchunk);
     const int e0 = 4 * threadIdx.x;
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    double a[NP][4] = {};
     int Q = qa;
     for (; Q + 1 < qb; Q += 2) {
-        const double d0 = d[Q], d1 = d[Q + 1];
         const size_t base = (static_cast<size_t>(Q) * ntp + t) * TILE2 + e0;
         double v0[4], v1[4];
         B.load4(base, v0);
         B.load4(base + static_cast<size_t>(ntp) * TILE2, v1);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = fma(v1[k], d1, fma(v0[k], d0, a[k]));
+        for (int p = 0; p < NP; ++p) {
+            const double d0 = d[static_cast<size_t>(p) * ldd + Q], d1 = d[static_cast<size_t>(p) * ldd + Q + 1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) a[p][k] = fma(v1[k], d1, fma(v0[k], d0, a[p][k]));
+        }
     }
     if (Q < qb) {
-        const double d0 = d[Q];
         double v0[4];
         B.load4((static_cast<size_t>(Q) * ntp + t) * TILE2 + e0, v0);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = fma(v0[k], d0, a[k]);
-    }
-    double* o = Jpart + (static_cast<size_t>(c) * ntp + t) * TILE2 + e0;
+        for (int p = 0; p < NP; ++p) {
+            const double d0 = d[static_cast<size_t>(p) * ldd + Q];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = a[k];
+            for (int k = 0; k < 4; ++k) a[p][k] = fma(v0[k], d0, a[p][k]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        double* o = Jpart + p * pstride + (static_cast<size_t>(c) * ntp + t) * TILE2 + e0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = a[p][k];
+    }
 }
 
 // J from the partials of every Q chunk.  A workgroup sums 128 elements (4 rows) of one tile, the
@@ -171,11 +181,12 @@ __global__ __launch_bounds__(256) void k_j2(BS B, const double* __restrict__ d, 
 // (24 chunks); this takes 9 us and 11 us.  Tiles that are not stored stay at the caller's zeros
 // (or are zeroed by k_j_clear when not accumulating).
 constexpr int kJuGroups = 8;
-__global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(const double* __restrict__ Jpart, int nchunk, int ntp,
-                                                             const int2* __restrict__ tiles, int nbf,
-                                                             double* __restrict__ J, int ldJ, double alpha,
-                                                             int accumulate) {
+__global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(const double* __restrict__ Jpart, size_t pstride,
+                                                             int nchunk, int ntp, const int2* __restrict__ tiles,
+                                                             int nbf, JOut out, int ldJ, double alpha, int accumulate) {
     __shared__ double red[kJuGroups][128];
+    Jpart += blockIdx.z * pstride;
+    double* __restrict__ J = out.J[blockIdx.z];
     const int t = blockIdx.x, el = threadIdx.x & 127, grp = threadIdx.x >> 7;
     const int e = blockIdx.y * 128 + el;
     double s = 0.0;
@@ -198,7 +209,8 @@ __global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(const double* __re
     }
 }
 // J = 0 on the 32 x 32 blocks that have no stored tile
-__global__ void k_j_clear(const int* __restrict__ tidx, int nT, int nbf, double* __restrict__ J, int ldJ) {
+__global__ void k_j_clear(const int* __restrict__ tidx, int nT, int nbf, JOut out, int ldJ) {
+    double* __restrict__ J = out.J[blockIdx.z];
     const int I = blockIdx.y, Jt = blockIdx.x;
     if (tidx[min(I, Jt) * nT + max(I, Jt)] >= 0) return;
     for (int e = threadIdx.x; e < TILE2; e += blockDim.x) {
@@ -208,75 +220,6 @@ __global__ void k_j_clear(const int* __restrict__ tidx, int nT, int nbf, double*
 }
 
 // ------------------------------------------------------------------ K path
-__global__ void k_pack_c(const double* __restrict__ src, int ldsrc, int nbf, int ncol, double scale,
-                         double* __restrict__ dst, int nbfp, int ldc) {
-    const size_t idx = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= static_cast<size_t>(nbfp) * ldc) return;
-    const int m = static_cast<int>(idx / ldc), i = static_cast<int>(idx % ldc);
-    dst[idx] = (m < nbf && i < ncol) ? scale * src[static_cast<size_t>(m) * ldsrc + i] : 0.0;
-}
-
-// Batched NT product into 128x128 tiles, FP64 MFMA.  4 waves in a 2x2 grid,
-// each wave a 64x64 sub-tile (4x4 MFMA blocks).  grid = (ntile, nsplit).
-__global__ __launch_bounds__(256) void k_gemm_nt_f64(const double* __restrict__ A, size_t strideA, int lda,
-                                                     const double* __restrict__ Bm, size_t strideB, int ldb, int M,
-                                                     int N, int K, int nbatch, const int2* __restrict__ tiles,
-                                                     int ntile, double* __restrict__ P, int accumulate) {
-    __shared__ double As[128][17];
-    __shared__ double Bs[128][17];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const int tile = blockIdx.x, split = blockIdx.y, nsplit = gridDim.y;
-    const int2 tb = tiles[tile];
-    const int m0 = tb.x * 128, n0 = tb.y * 128;
-    const int b0 = static_cast<int>((static_cast<long long>(nbatch) * split) / nsplit);
-    const int b1 = static_cast<int>((static_cast<long long>(nbatch) * (split + 1)) / nsplit);
-    d4_t acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = d4_t{0.0, 0.0, 0.0, 0.0};
-    for (int b = b0; b < b1; ++b) {
-        const double* Ab = A + static_cast<size_t>(b) * strideA;
-        const double* Bb = Bm + static_cast<size_t>(b) * strideB;
-        for (int k0 = 0; k0 < K; k0 += 16) {
-            __syncthreads();
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                const int e = tid + 256 * it;
-                const int r = e >> 4, kk = e & 15;
-                const bool kin = (k0 + kk) < K;
-                As[r][kk] = (kin && m0 + r < M) ? Ab[static_cast<size_t>(m0 + r) * lda + k0 + kk] : 0.0;
-                Bs[r][kk] = (kin && n0 + r < N) ? Bb[static_cast<size_t>(n0 + r) * ldb + k0 + kk] : 0.0;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int ks = 0; ks < 16; ks += 4) {
-                double a[4], bv[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = As[wr * 64 + i * 16 + (lane & 15)][ks + (lane >> 4)];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) bv[j] = Bs[wc * 64 + j * 16 + (lane & 15)][ks + (lane >> 4)];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i * 4 + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i * 4 + j], 0, 0, 0);
-            }
-        }
-    }
-    double* Pt = P + (static_cast<size_t>(split) * ntile + tile) * 16384;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wr * 64 + i * 16 + 4 * r + (lane >> 4);
-                const int col = wc * 64 + j * 16 + (lane & 15);
-                double* o = Pt + row * 128 + col;
-                *o = acc[i * 4 + j][r] + (accumulate ? *o : 0.0);
-            }
-}
-
 // Sum of the split partials into the dense result.  A workgroup owns a 16 x 16 output block, the
 // splits dealt to 4 groups of 256 threads and added in LDS in a fixed order.  With sym only the
 // blocks on and above the diagonal run and write their mirror image too.  Bound by latency at small
@@ -499,39 +442,30 @@ void launch_j1_reduce(const TileGeom& g, const double* dpart, int naux, double* 
     hipLaunchKernelGGL(k_j1_reduce, grid1(naux, 64), dim3(64 * kJ1Groups), 0, s, dpart, g.ntp, naux, d);
 }
 
-void launch_j2(const TileGeom& g, const JSource& B, const double* d, int naux, int qchunk, double* Jpart,
-               hipStream_t s) {
+void launch_j2(const TileGeom& g, const JSource& B, const double* d, int ldd, int np, int naux, int qchunk,
+               double* Jpart, size_t pstride, hipStream_t s) {
     require(qchunk > 0, "j2 qchunk");
-    require(B.a != nullptr, "j2 source");
+    require(B.a != nullptr && np >= 1 && np <= 4 && (np == 1 || ldd >= naux), "j2 source");
     dim3 grid(g.ntp, (naux + qchunk - 1) / qchunk);
+    require(np == 1 || pstride >= static_cast<size_t>(grid.y) * g.q_stride(), "j2 partials");
     with_bsrc(B, [&](auto src) {
-        hipLaunchKernelGGL(k_j2<decltype(src)>, grid, dim3(256), 0, s, src, d, g.ntp, naux, qchunk, Jpart);
+#define P4A_J2(N)                                                                                                    \
+    case N:                                                                                                          \
+        hipLaunchKernelGGL((k_j2<decltype(src), N>), grid, dim3(256), 0, s, src, d, ldd, g.ntp, naux, qchunk, Jpart, \
+                           pstride);                                                                                 \
+        break;
+        switch (np) { P4A_J2(1) P4A_J2(2) P4A_J2(3) P4A_J2(4) }
+#undef P4A_J2
     });
 }
 
-void launch_j_unpack(const TileGeom& g, const double* Jpart, int nchunk, double* J, int ldJ, double alpha,
-                     int accumulate, hipStream_t s) {
-    require(ldJ >= g.nbf && g.ntp > 0 && nchunk > 0, "j_unpack");
+void launch_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np, int ldJ,
+                     double alpha, int accumulate, hipStream_t s) {
+    require(ldJ >= g.nbf && g.ntp > 0 && nchunk > 0 && np >= 1 && np <= 4, "j_unpack");
     if (!accumulate && g.ntp < g.nT * (g.nT + 1) / 2)
-        hipLaunchKernelGGL(k_j_clear, dim3(g.nT, g.nT), dim3(256), 0, s, g.d_tidx, g.nT, g.nbf, J, ldJ);
-    hipLaunchKernelGGL(k_j_unpack, dim3(g.ntp, TILE2 / 128), dim3(128 * kJuGroups), 0, s, Jpart, nchunk, g.ntp,
-                       g.d_tiles, g.nbf, J, ldJ, alpha, accumulate);
-}
-
-void launch_pack_c(const double* Csrc, int ldsrc, int nbf, int ncol, double scale, double* Cpad, int nbfp, int ldc,
-                   hipStream_t s) {
-    require(nbfp >= nbf && ldc >= ncol && ldsrc >= ncol, "pack_c");
-    const size_t n = static_cast<size_t>(nbfp) * ldc;
-    hipLaunchKernelGGL(k_pack_c, grid1(n, 256), dim3(256), 0, s, Csrc, ldsrc, nbf, ncol, scale, Cpad, nbfp, ldc);
-}
-
-void launch_gemm_nt_f64(const double* A, size_t strideA, int lda, const double* B, size_t strideB, int ldb, int M,
-                        int N, int K, int nbatch, int nsplit, const int2* d_tiles, int ntile, double* P, int accumulate,
-                        hipStream_t s) {
-    require(ntile > 0 && nsplit > 0 && nbatch >= nsplit && lda >= K && ldb >= K, "gemm_nt_f64");
-    dim3 grid(ntile, nsplit);
-    hipLaunchKernelGGL(k_gemm_nt_f64, grid, dim3(256), 0, s, A, strideA, lda, B, strideB, ldb, M, N, K, nbatch,
-                       d_tiles, ntile, P, accumulate);
+        hipLaunchKernelGGL(k_j_clear, dim3(g.nT, g.nT, np), dim3(256), 0, s, g.d_tidx, g.nT, g.nbf, out, ldJ);
+    hipLaunchKernelGGL(k_j_unpack, dim3(g.ntp, TILE2 / 128, np), dim3(128 * kJuGroups), 0, s, Jpart, pstride, nchunk,
+                       g.ntp, g.d_tiles, g.nbf, out, ldJ, alpha, accumulate);
 }
 
 void launch_tile_reduce(const double* P, int nsplit, int ntile, const int* d_tile_of, int nB, int sym, int M, int N,

@@ -33,24 +33,18 @@ struct JSource {
 void launch_j1(const TileGeom& g, const JSource& B, const double* W, int naux, int q0, int q1, double* dpart,
                hipStream_t s);
 void launch_j1_reduce(const TileGeom& g, const double* dpart, int naux, double* d, hipStream_t s);
-// Jpart[c][t][e] = sum_{Q in chunk c} B[Q][t][e] d[Q]   (chunks of qchunk over [0,naux))
-void launch_j2(const TileGeom& g, const JSource& B, const double* d, int naux, int qchunk, double* Jpart,
-               hipStream_t s);
-// J[m][n] = alpha * sum_c Jpart[c][tile(m,n)] (+ J if accumulate)
-void launch_j_unpack(const TileGeom& g, const double* Jpart, int nchunk, double* J, int ldJ, double alpha,
-                     int accumulate, hipStream_t s);
+// Jpart[p][c][t][e] = sum_{Q in chunk c} B[Q][t][e] d[p * ldd + Q]   (chunks of qchunk over [0,naux); np <= 4
+// densities in one pass over B, density p's partials at Jpart + p * pstride)
+void launch_j2(const TileGeom& g, const JSource& B, const double* d, int ldd, int np, int naux, int qchunk,
+               double* Jpart, size_t pstride, hipStream_t s);
+struct JOut {
+    double* J[4];
+};
+// J_p[m][n] = alpha * sum_c Jpart[p][c][tile(m,n)] (+ J_p if accumulate)
+void launch_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np, int ldJ,
+                     double alpha, int accumulate, hipStream_t s);
 
 // ---- K path ----
-// Pack a dense row-major nbf x ncol matrix (any leading dim) into [nbfp][ldc] zero-padded.
-void launch_pack_c(const double* Csrc, int ldsrc, int nbf, int ncol, double scale, double* Cpad, int nbfp, int ldc,
-                   hipStream_t s);
-// Batched NT product accumulated into 128x128 output tiles:
-//   P[split][tile] (+)= sum_{b in split} A_b[m][:K] . B_b[n][:K]
-// A_b = A + b*strideA (row-major, lda), rows < M; likewise B (rows < N).
-// tiles: list of (Ib, Jb) 128-blocks, ntile entries.
-void launch_gemm_nt_f64(const double* A, size_t strideA, int lda, const double* B, size_t strideB, int ldb, int M,
-                        int N, int K, int nbatch, int nsplit, const int2* d_tiles, int ntile, double* P, int accumulate,
-                        hipStream_t s);
 // out[m][n] = alpha * sum_split P[split][tile(m,n)][..] (+ out if accumulate).  sym 1: only
 // tiles Ib<=Jb exist and the lower triangle is read transposed; sym 2: every tile exists and
 // out = alpha * (P + P^T), exactly symmetric.  tile_of: [nB*nB] -> tile index.
