@@ -84,10 +84,12 @@ class _SCFEnergy2e(torch.autograd.Function):
         _sync()
         jk.energy_adjoint_device(C.data_ptr(), C.shape[1], dC.data_ptr() if want_C else 0,
                                  dB.data_ptr() if want_B else 0)
-        if want_C:
-            dC.mul_(gE)
-        if want_B:
-            dB.mul_(gE)
+        # E.backward() passes 1: no pass over dE/dB (as large as B) for that
+        if float(gE) != 1.0:
+            if want_C:
+                dC.mul_(gE)
+            if want_B:
+                dB.mul_(gE)
         return dC, dB, None
 
 

@@ -2257,101 +2257,108 @@ void compute_wk_impl(dfjk_handle* h, int n, const double* const* Cl, const doubl
 }
 
 // Adjoint of E = tr(D(2J - K)), D = C C^T, at FP64 (the DF gradient terms of
-// scfgrad/jk_grad.cc:294-475 contract the same c_Q = d_Q and (Q|ij) = C^T B_Q C):
-//   dE/dC = 4 (2J - K) C,   Gamma_Qmn = dE/dB_Qmn = 4 d_Q D_mn - 2 (C (C^T X_Q) C^T)_mn, X_Q = B_Q C.
+// scfgrad/jk_grad.cc:294-475 contract the same c_Q = d_Q and (Q|ij) = C^T B_Q C).  With X_Q = B_Q C,
+// Y_Q = C^T X_Q and Z_Q = 2 d_Q 1 - Y_Q:
+//   E = sum_Q tr(Y_Q Z_Q), dE/dC = 4 (2J - K) C = 4 sum_Q X_Q Z_Q,
+//   Gamma_Q = dE/dB_Q = 4 d_Q D - 2 C Y_Q C^T = 2 C Z_Q C^T.
 // E and dE/dC use the whole auxiliary range; Gamma is produced for the configured range
-// [q0, q1), in blocks of Q.  dC is a device [nbf][nocc] matrix.  Gamma blocks go to
-// gam_dev (device, [q1-q0][nbf][nbf]) or, when gam_host is set, are copied to host memory.
+// [q0, q1).  Q-blocks are streamed from host memory out of core.  dC is a device [nbf][nocc] matrix.
+// Gamma blocks go to gam_dev (device, [q1-q0][nbf][nbf]) or, when gam_host is set, are copied to host
+// memory.
 void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double* dEdC, double* gam_dev,
                   double* gam_host) {
-    // E and dE/dC come from J and K, which stream B out of core too; Gamma needs B in core
-    if (h->ooc && (gam_dev || gam_host))
+    // E and dE/dC stream B out of core too; Gamma needs B in core
+    const bool gam = gam_dev || gam_host;
+    if (h->ooc && gam)
         fail(DFJK_ERR_STATE, "DFJK: dE/dB of the energy adjoint needs B in core (subalgorithm INCORE)");
     const hipStream_t s = h->stream;
-    const int nbf = h->nbf, nbfp = h->nbfp;
-    const size_t nn = static_cast<size_t>(nbf) * nbf;
-    const int uq0 = h->aux_q0, uq1 = h->aux_q1;
-    const int prec = h->precision;
-    const bool dj = h->do_J, dk = h->do_K;
-    double* D = h->ws_D.get<double>(nn);
-    double* Jm = h->ws_J.get<double>(nn);
-    double* Km = h->ws_K.get<double>(nn);
-    // full-range FP64 J and K (this also leaves d_Q for every Q in ws_d)
-    h->aux_q0 = 0;
-    h->aux_q1 = h->naux;
-    h->precision = DFJK_PREC_FP64;
-    h->do_J = h->do_K = true;
-    try {
-        Work wk;
-        PairIn in;
-        in.cl = dC;
-        in.ncol = nocc;
-        in.D = D;
-        in.J = Jm;
-        in.K = Km;
-        compute_f64(h, &in, classify_pairs(h, &in, 1, wk), 1, 0, wk);
-    } catch (...) {
-        h->aux_q0 = uq0, h->aux_q1 = uq1, h->precision = prec, h->do_J = dj, h->do_K = dk;
-        throw;
-    }
-    h->aux_q0 = uq0, h->aux_q1 = uq1, h->precision = prec, h->do_J = dj, h->do_K = dk;
-    const double* dvec = h->ws_d.as<double>();
-
-    // G = 2J - K; E = <D, G> (fixed-order reduction); dE/dC = 4 G C
-    h->dM_ready = false;
-    double* G = h->ws_G.get<double>(nn);
-    launch_axpby_mat(Jm, 2.0, Km, -1.0, G, nn, s);
-    if (E) {
-        constexpr int kRed = 256;
-        double* part = h->ws_red.get<double>(kRed);
-        launch_dot_partial(D, G, nn, part, kRed, s);
-        std::vector<double> hp(kRed);
-        copy_settled(hp.data(), part, kRed * sizeof(double), hipMemcpyDeviceToHost, s, "energy");
-        double e = 0.0;
-        for (double v : hp) e += v;
-        *E = e;
-    }
-    if (dEdC) launch_gemm_nn_f64(G, nbf, dC, nocc, dEdC, nocc, nbf, nocc, nbf, 4.0, 0.0, s);
-    if (!gam_dev && !gam_host) return;
-
-    // Gamma over [uq0, uq1) in blocks: X_Q = B_Q C (half-transform), Y_Q = C^T X_Q,
-    // P_Q = C Y_Q, Gamma_Q = 4 d_Q D - 2 P_Q C^T.
     const TileGeom g = h->geom();
-    const int xrows = (h->nT + 3) / 4 * 128;
-    int nbw, npanel, ldc;
-    ht_panel_shape(nocc, &nbw, &npanel, &ldc);
-    std::vector<int> cmap(ldc, -1);
-    for (int i = 0; i < nocc; ++i) cmap[i] = i;
-    Work alloc_wk;
-    int* dmap = upload_cmap(h, cmap, alloc_wk);
-    double* cl = h->ws_cl.get<double>(static_cast<size_t>(nbfp) * ldc);
-    launch_pack_cmap_f64(dC, nocc, nbf, dmap, cl, nbfp, ldc, s);
-    double* CT = h->ws_ct.get<double>(static_cast<size_t>(nocc) * nbf);
-    launch_transpose(dC, nbf, nocc, nocc, CT, nbf, s);
+    const int nbf = h->nbf, nbfp = h->nbfp, nT = h->nT;
+    const size_t nn = static_cast<size_t>(nbf) * nbf, qs = static_cast<size_t>(h->ntp) * TILE2;
+    const int uq0 = h->aux_q0, uq1 = h->aux_q1;
+    // E and dE/dC take every Q, Gamma alone its own range
+    const int q0 = E || dEdC ? 0 : uq0, q1 = E || dEdC ? h->naux : uq1;
+    if (!E && !dEdC && !gam) return;
+    const int ncb = (nocc + 15) / 16, nk = (nocc + 7) / 8;
+    const size_t csz = static_cast<size_t>(nbfp) * 16 * ncb, xq = csz, zq = static_cast<size_t>(256) * ncb * ncb;
+    double* CA = h->ws_CA.get<double>(csz);
+    double* CD = h->ws_CD.get<double>(csz);
+    double* CB = h->ws_cl.get<double>(csz);
+    launch_pack_frag(one_group(dC, nocc, dC), nbf, nbfp, CA, CD, s);
+    launch_pack_rows(dC, nocc, nocc, nbf, nbfp, ncb, CB, s);
 
-    const size_t xq = static_cast<size_t>(xrows) * ldc;
-    const size_t yq = static_cast<size_t>(nocc) * nocc, pq = static_cast<size_t>(nbf) * nocc;
-    const size_t per_q = (xq + yq + pq + (gam_host ? nn : 0)) * sizeof(double);
-    const size_t budget = memory_limited(h, size_t(2) << 30, (b_doubles(h) + 4 * nn) * sizeof(double));
-    const int nq_total = uq1 - uq0;
-    int qblk = static_cast<int>(std::min<size_t>(nq_total, std::max<size_t>(1, budget / per_q)));
+    const int nzw = adj_z_waves(ncb);
+    const size_t dq = static_cast<size_t>(ht_row_groups(nT, 1)) * ncb;
+    const size_t per_q = (xq * (gam ? 2 : 1) + zq + dq + (gam_host ? nn : 0)) * sizeof(double);
+    const size_t budget =
+        memory_limited(h, size_t(2) << 30, ((h->ooc ? 0 : b_doubles(h)) + 4 * nn) * sizeof(double));
+    int qblk = static_cast<int>(std::min<size_t>(q1 - q0, std::max<size_t>(1, budget / per_q)));
     qblk = std::min(qblk, 65535);
+    if (h->ooc) {
+        const size_t pq = qs * 2 * sizeof(double);
+        const size_t stage_budget = std::max<size_t>(pq, std::min<size_t>(size_t(8) << 30, budget / 2));
+        qblk = std::min<int>(qblk, static_cast<int>(std::max<size_t>(1, stage_budget / pq)));
+    }
+    const int nblocks = (q1 - q0 + qblk - 1) / qblk;
+    qblk = (q1 - q0 + nblocks - 1) / nblocks;
+    const int rt = ht_row_tiles(nT, qblk, ncb), nrg = ht_row_groups(nT, rt);
+    const int nsp = adj_dc_splits(nT, ncb, kc_steps(qblk, nk));
     double* X = h->ws_XL.get<double>(xq * qblk);
-    double* Y = h->ws_Y.get<double>(yq * qblk);
-    double* P = h->ws_PC.get<double>(pq * qblk);
+    double* dpart = h->ws_dpart.get<double>(dq * qblk);
+    double* dvec = h->ws_d.get<double>(h->naux);
+    double* Z = h->ws_Y.get<double>(zq * qblk);
+    double* epart = h->ws_red.get<double>(static_cast<size_t>(q1 - q0) * nzw);
+    double* P = gam ? h->ws_PC.get<double>(xq * qblk) : nullptr;
+    double* part = dEdC ? h->ws_P.get<double>(nsp * adj_dc_partial(nT, ncb)) : nullptr;
     double* Gb = gam_host ? h->ws_gam.get<double>(nn * qblk) : nullptr;
-    for (int qa = uq0; qa < uq1; qa += qblk) {
-        const int nq = std::min(qblk, uq1 - qa);
-        double* out = gam_host ? Gb : gam_dev + static_cast<size_t>(qa - uq0) * nn;
-        launch_ht2_f64(g, h->dB.as<double>(), qa, nq, cl, ldc, nbw, npanel, X, xrows, h->dZero.p, s);
-        launch_gemm_nn_f64(CT, nbf, X, ldc, Y, nocc, nocc, nocc, nbf, 1.0, 0.0, s, nq, 0, xq, yq);
-        launch_gemm_nn_f64(dC, nocc, Y, nocc, P, nocc, nbf, nocc, nocc, 1.0, 0.0, s, nq, 0, yq, pq);
-        launch_fill_scaled(dvec, qa, nq, 4.0, D, nbf, out, s);
-        launch_gemm_nn_f64(P, nocc, CT, nbf, out, nbf, nbf, nbf, nocc, -2.0, 1.0, s, nq, pq, 0, nn);
-        if (gam_host) {
-            copy_settled(gam_host + static_cast<size_t>(qa - uq0) * nn, Gb, nn * nq * sizeof(double),
-                         hipMemcpyDeviceToHost, s, "download dE/dB");
+    DRanges dr;
+    dr.n = 1;
+    dr.cb0[0] = 0;
+    dr.ncb[0] = ncb;
+    // out-of-core blocks are laid over the aux range of the handle
+    struct RangeRestore {
+        dfjk_handle* h;
+        int q0, q1;
+        ~RangeRestore() { h->aux_q0 = q0, h->aux_q1 = q1; }
+    } restore{h, uq0, uq1};
+    h->aux_q0 = q0;
+    h->aux_q1 = q1;
+    if (h->ooc) {
+        for (int i = 0; i < 2; ++i) hcheck(hipEventRecord(h->ev_free[i], s), "record");
+        stage_block(h, 0, qblk);
+    }
+    for (int blk = 0; blk < nblocks; ++blk) {
+        const int qa = q0 + blk * qblk, nq = std::min(qblk, q1 - qa);
+        const double* b64;
+        if (!h->ooc) {
+            b64 = h->dB.as<double>() + static_cast<size_t>(qa) * qs;
+        } else {
+            if (blk + 1 < nblocks) stage_block(h, blk + 1, qblk);
+            hcheck(hipStreamWaitEvent(s, h->ev_copied[blk & 1], 0), "wait copy");
+            b64 = h->ws_stage[blk & 1].as<double>();
         }
+        launch_ht_f64(g, b64, nq, CA, CD, ncb, rt, X, dpart, h->dZero.p, s);
+        if (h->ooc) hcheck(hipEventRecord(h->ev_free[blk & 1], s), "record");
+        launch_dpart_reduce(dpart, nq, nrg, ncb, dr, dvec + qa, h->naux, s);
+        launch_adj_z(CB, X, nT, ncb, nq, dvec + qa, Z, epart + static_cast<size_t>(qa - q0) * nzw, s);
+        if (dEdC) launch_adj_dc(X, Z, nT, ncb, nk, nq, nsp, part, blk > 0 ? 1 : 0, s);
+        const int ga = std::max(qa, uq0), gb = std::min(qa + nq, uq1);
+        if (gam && ga < gb) {
+            double* out = gam_host ? Gb : gam_dev + static_cast<size_t>(ga - uq0) * nn;
+            launch_adj_p(Z + (ga - qa) * zq, CD, nT, ncb, gb - ga, P, s);
+            launch_adj_g(P, CD, nT, ncb, nk, gb - ga, nbf, out, s);
+            if (gam_host)
+                copy_settled(gam_host + static_cast<size_t>(ga - uq0) * nn, Gb, nn * (gb - ga) * sizeof(double),
+                             hipMemcpyDeviceToHost, s, "download dE/dB");
+        }
+    }
+    if (dEdC) launch_adj_dc_reduce(part, nsp, nT, ncb, nbf, nocc, 4.0, dEdC, s);
+    if (E) {
+        std::vector<double> hp(static_cast<size_t>(q1 - q0) * nzw);
+        copy_settled(hp.data(), epart, hp.size() * sizeof(double), hipMemcpyDeviceToHost, s, "energy");
+        long double e = 0.0L;  // naux * nzw terms in sequence
+        for (double v : hp) e += v;
+        *E = static_cast<double>(e);
     }
 }
 

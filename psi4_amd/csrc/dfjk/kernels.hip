@@ -503,37 +503,11 @@ __global__ void k_hermitivitize(double* __restrict__ A, int n, int lda) {
         A[cr] = v;
     }
 }
-// partial[b] = sum over the block's slice of X.*Y (fixed tree, deterministic)
-__global__ __launch_bounds__(256) void k_dot_partial(const double* __restrict__ X, const double* __restrict__ Y,
-                                                     size_t n, double* __restrict__ partial) {
-    __shared__ double red[256];
-    double s = 0.0;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * 256)
-        s = fma(X[i], Y[i], s);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
 __global__ void k_transpose(const double* __restrict__ A, int rows, int cols, int lda, double* __restrict__ AT,
                             int ldt) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
     if (c < cols) AT[static_cast<size_t>(c) * ldt + r] = A[static_cast<size_t>(r) * lda + c];
 }
-// G[q][m][n] = a * d[q0+q] * D[m][n]
-__global__ void k_fill_scaled(const double* __restrict__ d, int q0, double a, const double* __restrict__ D, int n,
-                              double* __restrict__ G) {
-    const size_t nn = static_cast<size_t>(n) * n;
-    const int q = blockIdx.y;
-    const double f = a * d[q0 + q];
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < nn;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        G[q * nn + i] = f * D[i];
-}
-
 // p[0..n) = 0 (a kernel, not hipMemsetAsync: a caller may capture this work in a graph)
 __global__ void k_zero(double* __restrict__ p, size_t n) {
     for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
@@ -565,18 +539,10 @@ void launch_hermitivitize(double* A, int n, int lda, hipStream_t s) {
     require(n >= 1 && n <= 65535 && lda >= n, "hermitivitize");
     hipLaunchKernelGGL(k_hermitivitize, dim3((n + 255) / 256, n), dim3(256), 0, s, A, n, lda);
 }
-void launch_dot_partial(const double* X, const double* Y, size_t n, double* partial, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_dot_partial, dim3(nblocks), dim3(256), 0, s, X, Y, n, partial);
-}
 void launch_transpose(const double* A, int rows, int cols, int lda, double* AT, int ldt, hipStream_t s) {
     require(lda >= cols && ldt >= rows, "transpose");
     hipLaunchKernelGGL(k_transpose, dim3((cols + 255) / 256, rows), dim3(256), 0, s, A, rows, cols, lda, AT, ldt);
 }
-void launch_fill_scaled(const double* d, int q0, int nq, double a, const double* D, int n, double* G, hipStream_t s) {
-    require(nq >= 1 && nq <= 65535, "fill_scaled");
-    hipLaunchKernelGGL(k_fill_scaled, dim3(64, nq), dim3(256), 0, s, d, q0, a, D, n, G);
-}
-
 // Dense [nq][nbf][nbf] -> stored tiles of Q = q0 .. q0+nq-1; pairs outside the Schwarz mask are zero.
 __global__ __launch_bounds__(256) void k_pack_dense(const double* __restrict__ src, const int2* __restrict__ tiles,
                                                     int ntp, int nbf, const uint8_t* __restrict__ mask, int q0,

@@ -63,17 +63,12 @@ void launch_gemm_nn_f64(const double* A, int lda, const double* B, int ldb, doub
 void launch_axpby_mat(const double* X, double a, const double* Y, double b, double* Z, size_t n, hipStream_t s);
 // A = (A + A^T) / 2 in place (n x n, leading dimension lda)
 void launch_hermitivitize(double* A, int n, int lda, hipStream_t s);
-// partial[0..nblocks) = block sums of X.*Y (deterministic; sum the partials on the host)
-void launch_dot_partial(const double* X, const double* Y, size_t n, double* partial, int nblocks, hipStream_t s);
 // p[0..n) = 0 by a kernel (graph-capturable, unlike hipMemsetAsync)
 void launch_zero(double* p, size_t n, hipStream_t s);
 // out[r][c] = f[r] * A[r][c] (rows x cols, dense row-major)
 void launch_scale_rows(const double* A, int rows, int cols, const double* f, double* out, hipStream_t s);
 // AT[c][r] = A[r][c]
 void launch_transpose(const double* A, int rows, int cols, int lda, double* AT, int ldt, hipStream_t s);
-// G[q][:][:] = a * d[q0+q] * D for q < nq (D n x n)
-void launch_fill_scaled(const double* d, int q0, int nq, double a, const double* D, int n, double* G, hipStream_t s);
-
 // ---- synthetic tensor-level workload ----
 // B_Qmn = s_Q * decay[|m-n|] * (G_Qmn + G_Qnm)/2, G from Philox4x32-10 keyed by seed, Q in [q0,q1).
 // Stored tiles of Q = q0 .. q0+nq-1 from a dense device [nq][nbf][nbf] tensor; mask is nbf x nbf (0 = screened).

@@ -458,6 +458,362 @@ __global__ __launch_bounds__(256) void k_add_transpose(const double* __restrict_
     *o = a + b + (accumulate ? *o : 0.0);
 }
 
+// ------------------------------------------------------------------ adjoint
+// With X_Q = B_Q C, Y_Q = C^T X_Q (o x o) and d_Q = tr Y_Q, every term of the adjoint of
+// E = tr(D (2J - K)) comes from X and Z_Q = 2 d_Q 1 - Y_Q, with neither J, K nor D:
+//   E = sum_Q tr(Y_Q Z_Q), dE/dC = 4 sum_Q X_Q Z_Q, dE/dB_Q = 2 C Z_Q C^T.
+// For o = n/5 that is 0.4 of the products that J, K, (2J - K) C and 4 d D - 2 (C Y) C^T take, and B
+// is read once.  All operands are again register images of the kernel before.
+__global__ __launch_bounds__(256) void k_pack_rows(const double* __restrict__ C, int ld, int ncol, int nbf, int n,
+                                                   int ncb, double* __restrict__ CB) {
+    for (int idx = blockIdx.x * 256 + threadIdx.x; idx < n; idx += gridDim.x * 256) {
+        const int e = idx & 1, lane = (idx >> 1) & 63, rest = idx >> 7;
+        const int kb = rest / ncb, cb = rest % ncb;
+        const int m = 8 * kb + 4 * e + (lane >> 4), c = 16 * cb + (lane & 15);
+        CB[idx] = (m < nbf && c < ncol) ? C[static_cast<size_t>(m) * ld + c] : 0.0;
+    }
+}
+
+// NC-wide groups of ncb blocks: the first ncb - ng (NC - 1) are NC wide, the others NC - 1
+__device__ inline int group_start(int g, int ncb, int ng, int NC) {
+    return g * NC - max(0, g - (ncb - ng * (NC - 1)));
+}
+
+// Y and Z of one q: blocks [i0, i0 + NI) x [j0, j0 + NJ).  X is gathered 8 bytes per lane in the
+// transposed sense (rows along the sum); each 16 x 16 piece feeds NI MFMA steps, so the gather (32
+// cache cycles) hides under them.
+template <int NI, int NJ>
+__device__ __forceinline__ void adj_z_body(const double* __restrict__ CB, const double* __restrict__ Xq, int nkb, int ncb,
+                                           int i0, int j0, double dq, double* __restrict__ Zq,
+                                           double* __restrict__ ep) {
+    const int lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
+    const unsigned off_c = lane * 16;
+    const unsigned off_x = ((lj >> 3) * 128 + (lj & 3) * 32 + ((lj >> 2) & 1) + lg * 2) * 8;
+    const int nkx = 2 * ncb;
+    d4_t acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = d4_t{0.0, 0.0, 0.0, 0.0};
+    d2_t a0[NI], a1[NI], b0[NJ], b1[NJ];
+    auto load = [&](int kb, d2_t* a, d2_t* b) {
+        kb = min(kb, nkb - 1);
+        const double* ca = CB + (static_cast<size_t>(kb) * ncb + i0) * 128;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[i] = ld2(ca + 128 * i, off_c);
+        const double* x = Xq + (static_cast<size_t>(kb >> 1) * nkx + 2 * j0) * 128 + 16 * (kb & 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            b[j].x = ld1(x + 256 * j, off_x);
+            b[j].y = ld1(x + 256 * j + 8, off_x);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mul = [&](const d2_t* a, const d2_t* b) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0, a0, b0);
+    for (int kb = 0; kb < nkb; kb += 2) {  // nkb is even
+        load(kb + 1, a1, b1);
+        mul(a0, b0);
+        load(kb + 2, a0, b0);
+        mul(a1, b1);
+    }
+    double es = 0.0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                d2_t z;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const double y = acc[i][j][2 * h + e];
+                    const bool diag = 16 * (i0 + i) + 8 * h + 4 * e + lg == 16 * (j0 + j) + lj;
+                    z[e] = (diag ? 2.0 * dq : 0.0) - y;
+                    es = fma(y, z[e], es);
+                }
+                *reinterpret_cast<d2_t*>(reinterpret_cast<char*>(
+                                             Zq + (static_cast<size_t>(2 * (i0 + i) + h) * ncb + j0 + j) * 128) + off_c) = z;
+            }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o);
+    if (lane == 0) *ep = es;
+}
+
+constexpr int kZ = 4;  // column blocks per side of a wave's part of Y
+__global__ __launch_bounds__(256, 2) void k_adj_z(const double* __restrict__ CB, const double* __restrict__ X, int nT,
+                                                  int ncb, int ng, int nc, int nq, const double* __restrict__ d,
+                                                  double* __restrict__ Z, double* __restrict__ epart) {
+    const WaveItem w = wave_item(ng * ng);
+    if (w.group >= nq) return;
+    const int q = w.group, gi = w.item / ng, gj = w.item % ng;
+    const int i0 = group_start(gi, ncb, ng, nc), j0 = group_start(gj, ncb, ng, nc);
+    const int ni = group_start(gi + 1, ncb, ng, nc) - i0, nj = group_start(gj + 1, ncb, ng, nc) - j0;
+    const double* Xq = X + static_cast<size_t>(q) * nT * 4 * ncb * 128;
+    double* Zq = Z + static_cast<size_t>(q) * 2 * ncb * ncb * 128;
+    double* ep = epart + static_cast<size_t>(q) * ng * ng + w.item;
+    const double dq = d[q];
+#define P4A_Z(NI, NJ) \
+    if (ni == NI && nj == NJ) return adj_z_body<NI, NJ>(CB, Xq, 4 * nT, ncb, i0, j0, dq, Zq, ep)
+    P4A_Z(4, 4);
+    P4A_Z(4, 3);
+    P4A_Z(3, 4);
+    P4A_Z(3, 3);
+    P4A_Z(3, 2);
+    P4A_Z(2, 3);
+    P4A_Z(2, 2);
+    P4A_Z(1, 1);
+#undef P4A_Z
+}
+
+// One wave of a product whose right operand is shared or not: NF row fragments x NC column blocks of
+// the transposed product, summed over steps; the caller gives the operand addresses of a step.
+template <int NF, int NC, class LA, class LC>
+__device__ __forceinline__ void frag_product(d4_t (&acc)[NF][NC], int steps, LA&& la, LC&& lc) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[f][c] = d4_t{0.0, 0.0, 0.0, 0.0};
+    if (steps <= 0) return;
+    d2_t a0[NF], a1[NF], c0[NC], c1[NC];
+    auto load = [&](int st, d2_t* a, d2_t* c) {
+        st = min(st, steps - 1);
+        la(st, a);
+        lc(st, c);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mul = [&](const d2_t* a, const d2_t* c) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int i = 0; i < NC; ++i)
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+                    acc[f][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(c[i][e], a[f][e], acc[f][i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0, a0, c0);
+    int st = 0;
+    for (; st + 1 < steps; st += 2) {
+        load(st + 1, a1, c1);
+        mul(a0, c0);
+        load(st + 2, a0, c0);
+        mul(a1, c1);
+    }
+    if (st < steps) mul(a0, c0);
+}
+
+// P_q^T = Z_q C^T: rows of C as the row operand, Z as the column operand
+template <int NF, int NC>
+__device__ __forceinline__ void adj_p_body(const double* __restrict__ Zq, const double* __restrict__ CD, int ncb, int rb0,
+                                           int cb0, double* __restrict__ Pq) {
+    const unsigned off = (threadIdx.x & 63) * 16;
+    const int nkx = 2 * ncb;
+    d4_t acc[NF][NC];
+    frag_product<NF, NC>(
+        acc, nkx,
+        [&](int st, d2_t* a) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) a[f] = ld2(CD + (static_cast<size_t>(rb0 + f) * nkx + st) * 128, off);
+        },
+        [&](int st, d2_t* c) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i) c[i] = ld2(Zq + (static_cast<size_t>(st) * ncb + cb0 + i) * 128, off);
+        });
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 0; i < 2 * NC; ++i)
+            *reinterpret_cast<d2_t*>(reinterpret_cast<char*>(
+                                         Pq + (static_cast<size_t>(rb0 + f) * nkx + 2 * cb0 + i) * 128) + off) =
+                d2_t{acc[f][i >> 1][2 * (i & 1)], acc[f][i >> 1][2 * (i & 1) + 1]};
+}
+template <int NC>
+__global__ __launch_bounds__(256, 2) void k_adj_p(const double* __restrict__ Z, const double* __restrict__ CD, int nT,
+                                                  int ncb, int ng, int nq, double* __restrict__ P) {
+    const int nrg = (nT + 1) / 2;
+    const WaveItem w = wave_item(nrg * ng);
+    if (w.group >= nq) return;
+    const int q = w.group, rg = w.item / ng, gc = w.item % ng;
+    const int cb0 = group_start(gc, ncb, ng, NC);
+    const bool wide = group_start(gc + 1, ncb, ng, NC) - cb0 == NC;
+    const double* Zq = Z + static_cast<size_t>(q) * 2 * ncb * ncb * 128;
+    double* Pq = P + static_cast<size_t>(q) * nT * 4 * ncb * 128;
+    const bool full = 2 * rg + 2 <= nT;
+    if (full) {
+        if (wide)
+            adj_p_body<4, NC>(Zq, CD, ncb, 4 * rg, cb0, Pq);
+        else if constexpr (NC > 1)
+            adj_p_body<4, NC - 1>(Zq, CD, ncb, 4 * rg, cb0, Pq);
+    } else {
+        if (wide)
+            adj_p_body<2, NC>(Zq, CD, ncb, 4 * rg, cb0, Pq);
+        else if constexpr (NC > 1)
+            adj_p_body<2, NC - 1>(Zq, CD, ncb, 4 * rg, cb0, Pq);
+    }
+}
+
+// G_q = 2 P_q C^T, a 64 x 64 block on or above the diagonal, written with its mirror image.  Bound
+// by writing G (8 n^2 bytes per q).
+template <int NI, int NJ, bool DIAG>
+__device__ __forceinline__ void adj_g_body(const double* __restrict__ Pq, const double* __restrict__ CD, int nkx, int nk,
+                                           int rb0, int cb0, int n, double* __restrict__ G) {
+    const int lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
+    const unsigned off = lane * 16;
+    d4_t acc[NJ][NI];
+    // the transposed product: rows of G along the MFMA rows, columns along its columns
+    frag_product<NJ, NI>(
+        acc, nk,
+        [&](int st, d2_t* a) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) a[j] = ld2(CD + (static_cast<size_t>(cb0 + j) * nkx + st) * 128, off);
+        },
+        [&](int st, d2_t* c) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) c[i] = ld2(Pq + (static_cast<size_t>(rb0 + i) * nkx + st) * 128, off);
+        });
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if (DIAG && i > j) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = 16 * (rb0 + i) + 4 * r + lg, c = 16 * (cb0 + j) + lj;
+                if (m >= n || c >= n || (DIAG && m > c)) continue;
+                const double v = 2.0 * acc[j][i][r];
+                G[static_cast<size_t>(m) * n + c] = v;
+                G[static_cast<size_t>(c) * n + m] = v;
+            }
+        }
+}
+__global__ __launch_bounds__(256, 2) void k_adj_g(const double* __restrict__ P, const double* __restrict__ CD, int nT,
+                                                  int ncb, int nk, int nq, int n, int nbr, int nblk,
+                                                  double* __restrict__ G) {
+    const WaveItem w = wave_item(nblk);
+    if (w.group >= nq) return;
+    int I = 0, r = w.item;
+    while (r >= nbr - I) {
+        r -= nbr - I;
+        ++I;
+    }
+    const int J = I + r, nkx = 2 * ncb;
+    const double* Pq = P + static_cast<size_t>(w.group) * nT * 4 * ncb * 128;
+    double* Gq = G + static_cast<size_t>(w.group) * n * n;
+    const bool fj = 4 * J + 4 <= 2 * nT;
+    if (I == J) {
+        if (fj)
+            adj_g_body<4, 4, true>(Pq, CD, nkx, nk, 4 * I, 4 * J, n, Gq);
+        else
+            adj_g_body<2, 2, true>(Pq, CD, nkx, nk, 4 * I, 4 * J, n, Gq);
+    } else if (fj) {
+        adj_g_body<4, 4, false>(Pq, CD, nkx, nk, 4 * I, 4 * J, n, Gq);
+    } else {
+        adj_g_body<4, 2, false>(Pq, CD, nkx, nk, 4 * I, 4 * J, n, Gq);
+    }
+}
+
+// sum over (q, k) of X_q Z_q: one wave takes 4 (or 2) row fragments x NC column blocks of one split
+template <int NF, int NC>
+__device__ __forceinline__ void adj_dc_body(const double* __restrict__ X, const double* __restrict__ Z, size_t xq,
+                                            size_t zq, int ncb, int nk, int rb0, int cb0, int s0, int s1,
+                                            double* __restrict__ part, int accumulate) {
+    const int lane = threadIdx.x & 63;
+    const unsigned off = lane * 16;
+    const int nkx = 2 * ncb;
+    d4_t acc[NF][NC];
+    // steps are taken in order: (q, k) of the step being loaded
+    int q = s0 / nk, k = s0 % nk, at = 0;
+    auto advance = [&](int st) {
+        if (st > at) {
+            at = st;
+            if (++k == nk) {
+                k = 0;
+                ++q;
+            }
+        }
+    };
+    frag_product<NF, NC>(
+        acc, s1 - s0,
+        [&](int st, d2_t* a) {
+            advance(st);
+            const double* p = X + q * xq + (static_cast<size_t>(rb0) * nkx + k) * 128;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) a[f] = ld2(p + static_cast<size_t>(f) * nkx * 128, off);
+        },
+        [&](int, d2_t* c) {
+            const double* p = Z + q * zq + (static_cast<size_t>(k) * ncb + cb0) * 128;
+#pragma unroll
+            for (int i = 0; i < NC; ++i) c[i] = ld2(p + 128 * i, off);
+        });
+    // acc holds the transposed product: lane m + 16 (column % 4), register column / 4
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double* o = part + (static_cast<size_t>(rb0 + f) * ncb + cb0 + i) * 256 + r * 64 + lane;
+                *o = acc[f][i][r] + (accumulate ? *o : 0.0);
+            }
+}
+template <int NC>
+__global__ __launch_bounds__(64, 2) void k_adj_dc(const double* __restrict__ X, const double* __restrict__ Z, int nT,
+                                                  int ncb, int ng, int nk, int nq, int nsplit,
+                                                  double* __restrict__ partial, int accumulate) {
+    const int nrg = (nT + 1) / 2;
+    const WaveItem w = wave_item(nrg * ng);
+    if (w.group >= nsplit) return;
+    const int sp = w.group, rg = w.item / ng, gc = w.item % ng;
+    const int cb0 = group_start(gc, ncb, ng, NC);
+    const bool wide = group_start(gc + 1, ncb, ng, NC) - cb0 == NC;
+    const long long steps = static_cast<long long>(nq) * nk;
+    const int s0 = uni(static_cast<int>(steps * sp / nsplit)), s1 = uni(static_cast<int>(steps * (sp + 1) / nsplit));
+    const size_t xq = static_cast<size_t>(nT) * 4 * ncb * 128, zq = static_cast<size_t>(2) * ncb * ncb * 128;
+    double* part = partial + static_cast<size_t>(sp) * 2 * nT * ncb * 256;
+#define P4A_DC(NF, N) adj_dc_body<NF, N>(X, Z, xq, zq, ncb, nk, 4 * rg, cb0, s0, s1, part, accumulate)
+    if (2 * rg + 2 <= nT) {
+        if (wide)
+            P4A_DC(4, NC);
+        else if constexpr (NC > 1)
+            P4A_DC(4, NC - 1);
+    } else {
+        if (wide)
+            P4A_DC(2, NC);
+        else if constexpr (NC > 1)
+            P4A_DC(2, NC - 1);
+    }
+#undef P4A_DC
+}
+__global__ __launch_bounds__(256 * kRedGroups) void k_adj_dc_reduce(const double* __restrict__ partial, int nsplit,
+                                                                   size_t stride, int ncb, int n, int ncol, double alpha,
+                                                                   double* __restrict__ out) {
+    __shared__ double red[kRedGroups][256];
+    const int cb = blockIdx.x, rb = blockIdx.y;
+    const int el = threadIdx.x & 255, grp = threadIdx.x >> 8;
+    const double* p = partial + (static_cast<size_t>(rb) * ncb + cb) * 256 + el;
+    double a = 0.0;
+#pragma unroll 8
+    for (int sp = grp; sp < nsplit; sp += kRedGroups) a += p[sp * stride];
+    red[grp][el] = a;
+    __syncthreads();
+    if (grp) return;
+    double v = red[0][el];
+#pragma unroll
+    for (int g = 1; g < kRedGroups; ++g) v += red[g][el];
+    const int m = 16 * rb + (el & 15), c = 16 * cb + 4 * (el >> 6) + ((el & 63) >> 4);
+    if (m < n && c < ncol) out[static_cast<size_t>(m) * ncol + c] = alpha * v;
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------ launchers
@@ -523,19 +879,19 @@ void launch_dpart_reduce(const double* dpart, int nq, int nrg, int ncb, const DR
 
 int kc_block_rows(int nT) { return (nT + 1) / 2; }
 
-// Splits of a pass of `steps` (q, k) steps that shares its launch with nseg - 1 others, at most max_splits.
-// Large passes: about 320 steps a split keep the split's waves within 8 Q of one another (see k_kc_f64),
-// or 7 rounds of the chip's 2048 wave slots if that is more splits (the waves of a launch are of uneven
-// length: nbf 576 / 120 columns / 2784 Q takes 2.43, 2.23, 2.17, 2.19 ms with 2.1, 3.2, 6.3, 8.4
-// rounds).  Not shorter than 16 steps, a split's 32 KB of partial sums costing about as much as 10, unless the
-// launch would then have fewer than 512 waves (4 steps at least).  Multiples of 8, one split per XCD, from 8 on.
+// Splits of `steps` steps when a split is nw waves.  A wave's partial sums (32 KB written and read
+// again) cost about as much as 10 steps, and the waves of a launch end unevenly, which costs about half a
+// round of the chip's 2048 wave slots: 10 ns / steps + 1024 / (ns nw) is least at ns = sqrt(102 steps / nw)
+// (nbf 576 / 120 columns / 2784 Q: 307; measured 2.43, 2.23, 2.17, 2.19 ms with 96, 144, 288, 384).
+// Where the launch streams more X than the L2s hold, about 320 steps a split keep a split's waves
+// within 8 Q of one another (see k_kc_f64).  At least 4 steps; multiples of 8, one split per XCD.
+static int balanced_splits(long long nw, int steps, int max_splits) {
+    long long ns = std::max<long long>(steps / 320, std::llround(std::sqrt(102.0 * steps / nw)));
+    ns = std::max<long long>(1, std::min<long long>({ns, steps / 4, max_splits}));
+    return static_cast<int>(ns >= 8 ? ns / 8 * 8 : ns);
+}
 int kc_choose_splits(int nT, bool upper, int steps, int nseg, int max_splits) {
-    const long long nw = static_cast<long long>(kc_blocks(nT, upper)) * nseg;  // waves per split
-    const long long big = std::max<long long>(steps / 320, 7 * kXCD * kSlots / nw);
-    long long ns = std::max(std::min<long long>(steps / 16, big), std::min<long long>(steps / 4, 512 / nw));
-    ns = std::max<long long>(1, std::min<long long>(ns, max_splits));
-    if (ns >= 8) ns = ns / 8 * 8;
-    return static_cast<int>(ns);
+    return balanced_splits(static_cast<long long>(kc_blocks(nT, upper)) * nseg, steps, max_splits);
 }
 
 void launch_kc_f64(const double* XA, const double* XB, size_t qstride, int nkx, int nT, int nq, const KcSegs& segs,
@@ -569,6 +925,70 @@ void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& 
 void launch_add_transpose(const double* M, int n, double* K, int accumulate, hipStream_t s) {
     const int nb = (n + 15) / 16;
     hipLaunchKernelGGL(k_add_transpose, dim3(nb, nb), dim3(256), 0, s, M, n, K, accumulate);
+}
+
+// ---- adjoint ----
+void launch_pack_rows(const double* C, int ld, int ncol, int nbf, int nbfp, int ncb, double* CB, hipStream_t s) {
+    require(ncol > 0 && ld >= ncol && ncol <= 16 * ncb && nbfp >= nbf && nbfp % TILE == 0 &&
+                static_cast<long long>(nbfp) * 16 * ncb < (1LL << 31),
+            "pack_rows");
+    const int n = nbfp * 16 * ncb;
+    hipLaunchKernelGGL(k_pack_rows, dim3(std::min(4096, (n + 255) / 256)), dim3(256), 0, s, C, ld, ncol, nbf, n, ncb, CB);
+}
+
+static int z_groups(int ncb) { return (ncb + kZ - 1) / kZ; }
+int adj_z_waves(int ncb) { return z_groups(ncb) * z_groups(ncb); }
+void launch_adj_z(const double* CB, const double* X, int nT, int ncb, int nq, const double* d, double* Z, double* epart,
+                  hipStream_t s) {
+    require(nT > 0 && ncb > 0 && nq > 0, "adj_z");
+    const int ng = z_groups(ncb), nc = (ncb + ng - 1) / ng;
+    // groups are nc or nc - 1 wide: 1 (one block), 2, 3 or 4, and 2 beside 1 never occurs
+    hipLaunchKernelGGL(k_adj_z, dim3(wave_grid(nq, ng * ng, 4)), dim3(256), 0, s, CB, X, nT, ncb, ng, nc, nq, d, Z, epart);
+}
+
+template <class F>
+static void with_groups(int ncb, F&& f) {
+    const int ng = (ncb + 4) / 5, nc = (ncb + ng - 1) / ng;
+    switch (nc) {
+        case 1: f(std::integral_constant<int, 1>{}, ng); break;
+        case 2: f(std::integral_constant<int, 2>{}, ng); break;
+        case 3: f(std::integral_constant<int, 3>{}, ng); break;
+        case 4: f(std::integral_constant<int, 4>{}, ng); break;
+        default: f(std::integral_constant<int, 5>{}, ng); break;
+    }
+}
+void launch_adj_p(const double* Z, const double* CD, int nT, int ncb, int nq, double* P, hipStream_t s) {
+    require(nT > 0 && ncb > 0 && nq > 0, "adj_p");
+    with_groups(ncb, [&](auto nc, int ng) {
+        constexpr int NC = decltype(nc)::value;
+        hipLaunchKernelGGL((k_adj_p<NC>), dim3(wave_grid(nq, kc_block_rows(nT) * ng, 4)), dim3(256), 0, s, Z, CD, nT, ncb,
+                           ng, nq, P);
+    });
+}
+void launch_adj_g(const double* P, const double* CD, int nT, int ncb, int nk, int nq, int n, double* G, hipStream_t s) {
+    require(nT > 0 && nk > 0 && nk <= 2 * ncb && nq > 0 && n <= nT * TILE, "adj_g");
+    const int nblk = kc_blocks(nT, true);
+    hipLaunchKernelGGL(k_adj_g, dim3(wave_grid(nq, nblk, 4)), dim3(256), 0, s, P, CD, nT, ncb, nk, nq, n,
+                       kc_block_rows(nT), nblk, G);
+}
+int adj_dc_splits(int nT, int ncb, int steps) {
+    return balanced_splits(kc_block_rows(nT) * ((ncb + 4) / 5), steps, 4096);
+}
+void launch_adj_dc(const double* X, const double* Z, int nT, int ncb, int nk, int nq, int nsplit, double* partial,
+                   int accumulate, hipStream_t s) {
+    require(nT > 0 && nk > 0 && nk <= 2 * ncb && nq > 0 && nsplit > 0 && static_cast<long long>(nq) * nk < (1LL << 31),
+            "adj_dc");
+    with_groups(ncb, [&](auto nc, int ng) {
+        constexpr int NC = decltype(nc)::value;
+        hipLaunchKernelGGL((k_adj_dc<NC>), dim3(wave_grid(nsplit, kc_block_rows(nT) * ng, 1)), dim3(64), 0, s, X, Z, nT,
+                           ncb, ng, nk, nq, nsplit, partial, accumulate);
+    });
+}
+void launch_adj_dc_reduce(const double* partial, int nsplit, int nT, int ncb, int n, int ncol, double alpha, double* out,
+                          hipStream_t s) {
+    require(nsplit > 0 && n <= nT * TILE && ncol <= 16 * ncb, "adj_dc_reduce");
+    hipLaunchKernelGGL(k_adj_dc_reduce, dim3(ncb, 2 * nT), dim3(256 * kRedGroups), 0, s, partial, nsplit,
+                       adj_dc_partial(nT, ncb), ncb, n, ncol, alpha, out);
 }
 
 }  // namespace p4a

@@ -85,4 +85,25 @@ void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& 
 // K (+)= M + M^T (n x n)
 void launch_add_transpose(const double* M, int n, double* K, int accumulate, hipStream_t s);
 
+
+// ---- adjoint of E = tr(D (2J - K)), D = C C^T, with ncb 16-column blocks of C ----
+// CB [nbfp/8][ncb][64][2]: C in the row order of X's fragments (rows 8 kb + 4 e + lane / 16)
+void launch_pack_rows(const double* C, int ld, int ncol, int nbf, int nbfp, int ncb, double* CB, hipStream_t s);
+// Y_q = C^T X_q, Z_q = 2 d_q 1 - Y_q as [2 ncb][ncb][64][2]; epart[q][adj_z_waves(ncb)] sums Y Z
+int adj_z_waves(int ncb);
+void launch_adj_z(const double* CB, const double* X, int nT, int ncb, int nq, const double* d, double* Z, double* epart,
+                  hipStream_t s);
+// P_q = C Z_q in X's layout
+void launch_adj_p(const double* Z, const double* CD, int nT, int ncb, int nq, double* P, hipStream_t s);
+// G_q = 2 P_q C^T, dense [nq][n][n], exactly symmetric; nk: k8 steps (ceil(ncol / 8))
+void launch_adj_g(const double* P, const double* CD, int nT, int ncb, int nk, int nq, int n, double* G, hipStream_t s);
+// partial[split][row block][column block][4][64] (+)= sum_{q, k} X_q[rows][k] Z_q[k][columns]
+int adj_dc_splits(int nT, int ncb, int steps);
+inline size_t adj_dc_partial(int nT, int ncb) { return static_cast<size_t>(2) * nT * ncb * 256; }  // doubles per split
+void launch_adj_dc(const double* X, const double* Z, int nT, int ncb, int nk, int nq, int nsplit, double* partial,
+                   int accumulate, hipStream_t s);
+// out[n][ncol] = alpha * sum over splits
+void launch_adj_dc_reduce(const double* partial, int nsplit, int nT, int ncb, int n, int ncol, double alpha, double* out,
+                          hipStream_t s);
+
 }  // namespace p4a

@@ -1133,10 +1133,6 @@ static void ht_mfma(const TileGeom& g, const T* B, int q0, int nq, const T* C, i
         ht_mfma_wm<T, 2>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
 }
 
-void launch_ht2_f64(const TileGeom& g, const double* B, int q0, int nq, const double* C, int ldc, int nbw, int npanel,
-                    double* X, int xrows, const void* zt, hipStream_t s) {
-    ht_mfma<double>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
-}
 void launch_ht2_f32(const TileGeom& g, const float* B, int q0, int nq, const float* C, int ldc, int nbw, int npanel,
                     float* X, int xrows, const void* zt, hipStream_t s) {
     ht_mfma<float>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
@@ -1190,14 +1186,6 @@ static void kgemm_check(int xrows, int ld, int kbeg, int kend, int nbatch, int n
             "kgemm shape");
 }
 
-void launch_kgemm2_f64(const double* A, const double* B, size_t stride, int xrows, int nvalid, int ld, int kbeg,
-                       int kend, int nbatch, int nsplit, const int2* tiles, int ntile, double* P, double alpha,
-                       int accumulate, int upper, hipStream_t s) {
-    kgemm_check(xrows, ld, kbeg, kend, nbatch, nsplit, ntile, 16);
-    require(nvalid > 0 && nvalid <= xrows, "kgemm valid rows");
-    hipLaunchKernelGGL((k_kgemm_mfma<double>), dim3(xcd_grid(nsplit, ntile)), dim3(256), 0, s, A, stride, B, stride, ld,
-                       kbeg, kend, nbatch, nsplit, tiles, ntile, P, alpha, accumulate, upper, nvalid);
-}
 void launch_kgemm2_f32(const float* A, const float* B, size_t stride, int xrows, int nvalid, int ld, int kbeg, int kend,
                        int nbatch, int nsplit, const int2* tiles, int ntile, double* P, double alpha, int accumulate,
                        int upper, hipStream_t s) {
@@ -1221,12 +1209,6 @@ void launch_to_f32(const double* src, float* dst, size_t n, hipStream_t s) {
 void launch_to_f32_t(const double* src, float* dst, size_t n, hipStream_t s) {
     require(n % TILE2 == 0, "to_f32_t");
     hipLaunchKernelGGL(k_to_f32_t, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
-}
-void launch_pack_cmap_f64(const double* src, int ldsrc, int nbf, const int* cmap, double* dst, int nbfp, int ldc,
-                          hipStream_t s) {
-    const size_t n = static_cast<size_t>(nbfp) * ldc;
-    hipLaunchKernelGGL((k_pack_cmap<double>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, src, ldsrc,
-                       nbf, cmap, dst, nbfp, ldc);
 }
 void launch_pack_cmap_f32(const double* src, int ldsrc, int nbf, const int* cmap, float* dst, int nbfp, int ldc,
                           hipStream_t s) {

@@ -125,3 +125,35 @@ def test_partial_auxiliary_range(gpu_available):
     jk.set_aux_range(7, 31)
     D, J, K = _compute(jk, [C])
     _check(B[7:31], C, C, D[0], J[0], K[0])
+
+
+@pytest.mark.parametrize("nbf,naux,nocc", [(1, 1, 1), (33, 7, 5), (64, 12, 16), (70, 20, 33), (97, 9, 65), (100, 31, 81),
+                                           (129, 6, 100), (40, 11, 60)])
+def test_adjoint_sizes(gpu_available, nbf, naux, nocc):
+    """E, dE/dC = 4 (2J - K) C and dE/dB = 4 d D - 2 D B D at block edges and for more columns than rows.
+    The tolerance is that of the chains the device sums (rows, columns and auxiliary functions in
+    turn) on the sums of absolute values; dE/dB is exactly symmetric, and a partial auxiliary range
+    gives the same slice."""
+    announce(f"adjoint, nbf {nbf} naux {naux} columns {nocc}")
+    jk, B = _tensor(nbf, naux, 11)
+    C = np.random.default_rng(nocc).standard_normal((nbf, nocc)) / np.sqrt(nbf)
+
+    def ref(B, C):
+        D = C @ C.T
+        d = np.einsum("qmn,mn->q", B, D)
+        DBD = D @ B @ D
+        ej, ek = 2 * np.sum(d * d), np.einsum("qmn,qmn->", DBD, B)
+        J, K = np.einsum("q,qmn->mn", d, B), np.einsum("qmk,qnk->mn", B @ C, B @ C)
+        return ej, ek, 8 * (J @ C), 4 * (K @ C), 4 * d[:, None, None] * D, 2 * DBD
+
+    E, dC, dB = jk.energy_adjoint(C, True)
+    r, a = ref(B, C), ref(np.abs(B), np.abs(C))
+    c = 4 * (2 * nbf * nbf + 2 * nbf + nocc + naux * nocc + 8) * EPS
+    assert abs(E - (r[0] - r[1])) <= c * (a[0] + a[1])
+    assert np.all(np.abs(dC - (r[2] - r[3])) <= c * (a[2] + a[3]))
+    assert np.all(np.abs(dB - (r[4] - r[5])) <= c * (a[4] + a[5]))
+    assert np.array_equal(dB, dB.transpose(0, 2, 1))
+    if naux > 6:
+        jk.set_aux_range(2, 5)
+        E2, dC2, dB2 = jk.energy_adjoint(C, True)
+        assert E2 == E and np.array_equal(dC2, dC) and np.array_equal(dB2, dB[2:5])
