@@ -81,7 +81,8 @@ constexpr int kFold32 = 512;
 
 template <int RT>
 struct StepList {
-    int off[kMaxColTiles * RT];
+    int off[kMaxColTiles * RT];    // by column tile
+    int soff[kMaxColTiles * RT];   // by step
     int J[kMaxColTiles];
     int cnt[kMaxColTiles];
     int n;
@@ -110,10 +111,14 @@ __device__ inline void build_steps(StepList<RT>& sl, const int* __restrict__ tid
         if (tid < kMaxColTiles) sl.cnt[tid] += v;
         __syncthreads();
     }
-    // compact: step k -> J (offsets are kept indexed by J)
+    // compact: step k -> J and its block offsets
     if (tid < kMaxColTiles) {
         const int prev = tid ? sl.cnt[tid - 1] : 0;
-        if (sl.cnt[tid] != prev) sl.J[prev] = tid;
+        if (sl.cnt[tid] != prev) {
+            sl.J[prev] = tid;
+#pragma unroll
+            for (int s = 0; s < RT; ++s) sl.soff[prev * RT + s] = sl.off[tid * RT + s];
+        }
         if (tid == kMaxColTiles - 1) sl.n = sl.cnt[tid];
     }
     __syncthreads();
@@ -351,6 +356,23 @@ __device__ inline void wait_vmem() {
     __builtin_amdgcn_s_waitcnt(wait_vm(N));
 #endif
 }
+// Workgroup barrier that publishes this wave's LDS stores and the direct loads older than its n
+// youngest vector-memory operations, and leaves those n in flight (__syncthreads waits for all).
+template <int N>
+__device__ inline void barrier_vmem() {
+    fence_compiler();
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_s_waitcnt(wait_vm(N) & ~0x0F00);
+    __builtin_amdgcn_s_barrier();
+#endif
+    fence_compiler();
+}
+template <int P>
+__device__ inline void set_priority() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_s_setprio(P);
+#endif
+}
 // 16 bytes per lane from global memory straight into LDS: lane L of the wave writes
 // lds + 16 L bytes (lds is wave-uniform)
 __device__ inline void load_lds16(const uint16_t* src, uint16_t* lds) {
@@ -429,32 +451,45 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
     constexpr int NRG = PAN / 16;
     constexpr int NLD = 2 * NRG / NWAVE;
     static_assert(!DC || NLD * NWAVE == 2 * NRG, "whole direct loads per wave");
-    auto issueC = [&](int st, int buf) {
-        const size_t kb = static_cast<size_t>(jof(st)) * TILE;
-        const int w = __builtin_amdgcn_readfirstlane(wave);
-        const int r0 = lane >> 2, pc = lane & 3;
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    const uint16_t* csrc[NLD];  // wave-uniform: the group's first row
+    int cdst[NLD];
 #pragma unroll
-        for (int i = 0; i < NLD; ++i) {
-            const int idx = w + NWAVE * i, arr = idx / NRG, rg = idx % NRG;
-            const int r = rg * 16 + r0;
-            const uint16_t* src = (arr ? CTl : CTh) + static_cast<size_t>(col0 + r) * nbfp + kb + 8 * (pc ^ ((r >> 1) & 3));
-            load_lds16(src, lbuf(buf) + 2 * A_SZ + arr * C_SZ + rg * 512);
-        }
+    for (int i = 0; i < NLD; ++i) {
+        const int idx = w + NWAVE * i, arr = idx / NRG, rg = idx % NRG;
+        csrc[i] = (arr ? CTl : CTh) + static_cast<size_t>(col0 + rg * 16) * nbfp;
+        cdst[i] = 2 * A_SZ + arr * C_SZ + rg * 512;
+    }
+    const unsigned coff = ((lane >> 2) * nbfp + 8 * ((lane & 3) ^ ((lane >> 3) & 3))) * 2;  // bytes
+    auto issueC = [&](int J, int buf) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i)
+            load_lds16(reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(csrc[i] + J * TILE) + coff),
+                       lbuf(buf) + cdst[i]);
     };
-    // vector f = v & 127 covers row (f>>2) of its row tile's block, k = 8*(f&3)..+7
-    auto gloadA = [&](int st, v4f_t(&a)[2 * NAV]) {
-        const int J = jof(st);
+    // vector f = v & 127 covers row (f>>2) of its row tile's block, k = 8*(f&3)..+7.  The block's tile
+    // and offset are wave-uniform.  A block stored as (J, I) (below the diagonal) is read from the
+    // tile-transposed copy, so the vector is always a row segment of this row tile's block.
+    const unsigned aoff = ((tid & 127) >> 2) * TILE * 4 + 32 * (tid & 3);  // bytes
+    auto gloadA_at = [&](int J, const int* off, v4f_t(&a)[2 * NAV]) {
 #pragma unroll
         for (int n = 0; n < NAV; ++n) {
-            const int v = tid + NTHR * n, sub = v >> 7, f = v & 127;
-            const int off = sl.off[J * RT + sub];
-            // a block stored as (J, I) (below the diagonal) is read from the tile-transposed
-            // copy, so the vector is always a row segment of this row tile's block
-            const bool tr = (I0 + sub > J);
-            const float* t = off >= 0 ? (tr ? BT : B) + qoff + off : ztile;
-            a[2 * n] = *reinterpret_cast<const v4f_t*>(t + (f >> 2) * TILE + 8 * (f & 3));
-            a[2 * n + 1] = *reinterpret_cast<const v4f_t*>(t + (f >> 2) * TILE + 8 * (f & 3) + 4);
+            const int sub = (w * 64 + NTHR * n) >> 7;
+            const float* t = off[n] >= 0 ? (I0 + sub > J ? BT : B) + qoff + off[n] : ztile;
+            const char* t8 = reinterpret_cast<const char*>(t) + aoff;
+            a[2 * n] = *reinterpret_cast<const v4f_t*>(t8);
+            a[2 * n + 1] = *reinterpret_cast<const v4f_t*>(t8 + 16);
         }
+    };
+    auto offs = [&](int st, int* off) {
+#pragma unroll
+        for (int n = 0; n < NAV; ++n)
+            off[n] = __builtin_amdgcn_readfirstlane(sl.soff[min(st, nsteps - 1) * RT + ((w * 64 + NTHR * n) >> 7)]);
+    };
+    auto gloadA = [&](int st, v4f_t(&a)[2 * NAV]) {
+        int off[NAV];
+        offs(st, off);
+        gloadA_at(__builtin_amdgcn_readfirstlane(jof(st)), off, a);
     };
     // the A vectors split into hi/lo (done while the previous step's MFMAs run)
     v4u_t sah[NAV], sal[NAV];
@@ -508,83 +543,93 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
         if (NSLOT > 3) cstore(3, c3h, c3l);
         if (NSLOT > 4) cstore(4, c4h, c4l);
     };
-    // One step's products: all fragments first (one LDS wait), then the MFMAs product by
-    // product (consecutive updates of one accumulator are 4*NBW MFMAs apart), then the next
-    // step's staging into the other buffer.
+    // One step's products, column block by column block: the A fragments and the first C fragments are
+    // read first, then each block's C fragments while the block before it is multiplied, so the LDS
+    // reads of a step are spread over its MFMAs (an accumulator's three updates are 4 MFMAs apart).  pre
+    // (the next steps' operands) runs after the first block's MFMAs are issued.
     // A wave whose 16-row fragments lie past the last row tile (last row block only) skips
     // their fragment reads and MFMAs; their accumulators stay zero.
     const int nfr = __builtin_amdgcn_readfirstlane(min(4, max(0, 2 * (nT - I0 - 2 * wm))));
-    auto compute = [&](int buf, auto ni, auto&& pre, auto&& mid, auto&& store_next) {
+    auto compute = [&](int buf, auto ni, auto&& pre) {
         constexpr int NI = decltype(ni)::value;
         const uint16_t* Ah = lbuf(buf);
         const uint16_t* Al = Ah + A_SZ;
         const uint16_t* Ch = Al + A_SZ;
         const uint16_t* Cl = Ch + C_SZ;
         const int fc = lane >> 4;
-        bf8_t ah[4], al[4], bh[NBW], bl[NBW];
-        // hi fragments first; the lo fragments are read while the hi x hi MFMAs run
+        bf8_t ah[4], al[4], bh[2], bl[2];
+        auto frag = [&](const uint16_t* L, int row) {
+            return __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + kg_swz(row + (lane & 15), fc)));
+        };
+        auto cread = [&](int j) {
+            bh[j & 1] = frag(Ch, wn * NBW * 16 + j * 16);
+            bl[j & 1] = frag(Cl, wn * NBW * 16 + j * 16);
+        };
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
-            ah[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(Ah + kg_swz(wm * 64 + i * 16 + (lane & 15), fc)));
+        for (int i = 0; i < NI; ++i) ah[i] = frag(Ah, wm * 64 + i * 16);
+        if constexpr (NI > 0) cread(0);
 #pragma unroll
-        for (int j = 0; j < NBW; ++j)
-            bh[j] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(Ch + kg_swz(wn * NBW * 16 + j * 16 + (lane & 15), fc)));
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < NI; ++i) al[i] = frag(Al, wm * 64 + i * 16);
 #pragma unroll
-        for (int j = 0; j < NBW; ++j)
-            bl[j] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(Cl + kg_swz(wn * NBW * 16 + j * 16 + (lane & 15), fc)));
+        for (int j = 0; j < NBW; ++j) {
+            if constexpr (NI > 0)
+                if (j + 1 < NBW) cread(j + 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
-            al[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(Al + kg_swz(wm * 64 + i * 16 + (lane & 15), fc)));
-        __builtin_amdgcn_sched_barrier(0);
-        pre();
-        __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j & 1], acc[i][j], 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < NBW; ++j)
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j & 1], acc[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-        // the next A vectors' hi/lo split (24 VALU ops per vector) runs between the MFMAs below
-        __builtin_amdgcn_sched_barrier(0);
-        mid();
-#pragma unroll
-        for (int j = 0; j < NBW; ++j)
-#pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < NBW; ++j)
-#pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        if constexpr (NI > 0) {
-            // one MFMA, then two VALU ops, 12 times per A vector; then the remaining MFMAs
-            constexpr int NG = 12 * NAV < 2 * NI * NBW ? 12 * NAV : 2 * NI * NBW;
-#pragma unroll
-            for (int k = 0; k < NG; ++k) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j & 1], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j == 0) {
+                pre();
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (2 * NI * NBW > NG) __builtin_amdgcn_sched_group_barrier(0x008, 2 * NI * NBW - NG, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        store_next();
     };
     // Steps run in pairs so the two A sets are named statically; the loop body has no
     // branches around its loads and stores (loads past the last step re-read it, and their
     // stores land in a buffer no later compute reads).
     auto mainloop = [&](auto ni) {
-        // Staged C: the step's C and A loads are issued before its fragment reads, and the A
-        // split runs between its MFMAs.  Direct C: the A loads first; the split and the direct
-        // loads after the fragment reads (a fragment read or split that follows a direct load
-        // in program order is made to wait for it), and the step ends by waiting for all its
-        // loads, which have had the step's MFMAs to land.
-        auto loads = [&](int st, v4f_t(&a)[2 * NAV]) {
-            if constexpr (!DC) gloadC(st);
-            gloadA(st + 1, a);
-        };
-        auto waitC = [&] {
-            if constexpr (DC) wait_vmem<0>();
+        // Staged C: the step's C and A loads are issued before its fragment reads.  Direct C: the A
+        // vectors that arrived are split and stored to the other buffer, then the next step's C goes
+        // there (a store that follows a direct load to its buffer would wait for it), then the A loads
+        // of the step after next; the wait that closes the step leaves those in flight, so a block of
+        // B has two steps to arrive from HBM.  The tiles and offsets of those loads are looked up a
+        // step ahead.
+        int J1 = 0, J2 = 0, off2[NAV] = {};
+        auto half = [&](int cur, int st, v4f_t(&have)[2 * NAV], v4f_t(&next)[2 * NAV]) {
+            if constexpr (DC) {
+                const int jn = sl.J[min(st + 3, nsteps - 1)];
+                int on[NAV];
+#pragma unroll
+                for (int n = 0; n < NAV; ++n) on[n] = sl.soff[min(st + 3, nsteps - 1) * RT + ((w * 64 + NTHR * n) >> 7)];
+                compute(cur, ni, [&] {
+                    splitA(have);
+                    lstore(cur ^ 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    issueC(J1, cur ^ 1);
+                    fence_compiler();
+                    __builtin_amdgcn_sched_barrier(0);
+                    gloadA_at(J2, off2, next);
+                });
+                J1 = J2;
+                J2 = __builtin_amdgcn_readfirstlane(jn);
+#pragma unroll
+                for (int n = 0; n < NAV; ++n) off2[n] = __builtin_amdgcn_readfirstlane(on[n]);
+                barrier_vmem<2 * NAV>();
+            } else {
+                gloadC(st + 1);
+                gloadA(st + 2, next);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(cur, ni, [&] { splitA(have); });
+                lstore(cur ^ 1);
+                __syncthreads();
+            }
         };
         if constexpr (DC) {
-            issueC(0, 0);
+            issueC(__builtin_amdgcn_readfirstlane(jof(0)), 0);
             fence_compiler();
         } else {
             gloadC(0);
@@ -593,39 +638,156 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
         splitA(a0);
         lstore(0);
         gloadA(1, a1);
-        waitC();
+        J1 = __builtin_amdgcn_readfirstlane(jof(1));
+        J2 = __builtin_amdgcn_readfirstlane(jof(2));
+        offs(2, off2);
+        if constexpr (DC) wait_vmem<0>();
         __syncthreads();
         int st = 0;
-        // (scheduling fences keep the loads ahead of the MFMAs they are meant to overlap)
         for (; st + 1 < nsteps; st += 2) {
-            loads(st + 1, a0);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (DC)
-                compute(0, ni, [&] { splitA(a1); __builtin_amdgcn_sched_barrier(0); issueC(st + 1, 1); }, [] {}, [&] { lstore(1); });
-            else
-                compute(0, ni, [] {}, [&] { splitA(a1); }, [&] { lstore(1); });
-            waitC();
-            __syncthreads();
-            loads(st + 2, a1);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (DC)
-                compute(1, ni, [&] { splitA(a0); __builtin_amdgcn_sched_barrier(0); issueC(st + 2, 0); }, [] {}, [&] { lstore(0); });
-            else
-                compute(1, ni, [] {}, [&] { splitA(a0); }, [&] { lstore(0); });
-            waitC();
-            __syncthreads();
+            half(0, st, a1, a0);
+            half(1, st + 1, a0, a1);
         }
-        if (st < nsteps) compute(0, ni, [] {}, [] {}, [] {});  // odd step count: the last step is in buffer 0
+        if (st < nsteps) compute(0, ni, [] {});  // odd step count: the last step is in buffer 0
         // direct loads still in flight (steps past the end) land before the LDS is released
         if constexpr (DC) wait_vmem<0>();
     };
+    // The 8-wave shape.  With all waves at the same point of a step, the fragment reads, the split and
+    // the barrier (1870 of 3790 cycles per step at nbf 1500) left the MFMA pipes idle: 50 % busy, 8.49 ms
+    // per 1000 Q at 600 columns.  Taking turns keeps them 62 % busy and takes 7.45 ms, now against the
+    // power limit (the clock falls from 1.97 to 1.78 GHz; MFMAs alone on random data reach 2113 TFLOP/s).
+    // Two groups of four waves (one wave per SIMD each) take turns: while one group multiplies a step
+    // whose fragments it holds in registers, the other reads its fragments of a step from LDS, splits and
+    // stores A and starts its loads.  Slots are separated by barriers; group 0 reads step s in slot 2s
+    // and multiplies it in slot 2s + 1, group 1 one slot later.  The buffer of step s + 1 was last
+    // read in slot 2s - 1 and is first read in slot 2s + 2: both groups start their direct loads to
+    // it in slot 2s (group 0 while reading, group 1 before multiplying) and have waited for them
+    // by the end of slot 2s + 1.
+    auto mainloop_pp = [&](auto ni, auto grp) {
+        constexpr int NI = decltype(ni)::value;
+        constexpr bool G1 = decltype(grp)::value;
+        bf8_t ah[4], al[4], bh[NBW], bl[NBW];
+        const int fc = lane >> 4;
+        auto frags = [&](int buf) {
+            const uint16_t* Ah = lbuf(buf);
+            const uint16_t* Al = Ah + A_SZ;
+            const uint16_t* Ch = Al + A_SZ;
+            const uint16_t* Cl = Ch + C_SZ;
+            auto frag = [&](const uint16_t* L, int row) {
+                return __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + kg_swz(row + (lane & 15), fc)));
+            };
+            if constexpr (NI > 0) {
+#pragma unroll
+                for (int i = 0; i < NI; ++i) ah[i] = frag(Ah, wm * 64 + i * 16);
+#pragma unroll
+                for (int j = 0; j < NBW; ++j) bh[j] = frag(Ch, wn * NBW * 16 + j * 16);
+#pragma unroll
+                for (int j = 0; j < NBW; ++j) bl[j] = frag(Cl, wn * NBW * 16 + j * 16);
+#pragma unroll
+                for (int i = 0; i < NI; ++i) al[i] = frag(Al, wm * 64 + i * 16);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto mul = [&] {
+            __builtin_amdgcn_sched_barrier(0);
+            set_priority<1>();
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < NBW; ++j)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
+            set_priority<0>();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // tiles and offsets of the loads, looked up a step ahead: J1 = tile of step s + 1 (group 1's
+        // multiply phase: s + 2), J2 and off2 of step s + 2
+        int J1, J2, off2[NAV];
+        issueC(__builtin_amdgcn_readfirstlane(jof(0)), 0);
+        fence_compiler();
+        gloadA(0, a0);
+        splitA(a0);
+        lstore(0);
+        gloadA(1, a1);
+        J1 = __builtin_amdgcn_readfirstlane(jof(1));
+        J2 = __builtin_amdgcn_readfirstlane(jof(2));
+        offs(2, off2);
+        wait_vmem<0>();
+        __syncthreads();
+        auto read_phase = [&](int cur, int st, v4f_t(&have)[2 * NAV], v4f_t(&next)[2 * NAV]) {
+            const int jn = sl.J[min(st + 3, nsteps - 1)];
+            int on[NAV];
+#pragma unroll
+            for (int n = 0; n < NAV; ++n) on[n] = sl.soff[min(st + 3, nsteps - 1) * RT + ((w * 64 + NTHR * n) >> 7)];
+            frags(cur);
+            splitA(have);
+            lstore(cur ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!G1) {
+                issueC(J1, cur ^ 1);
+                fence_compiler();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            gloadA_at(J2, off2, next);
+            __builtin_amdgcn_sched_barrier(0);
+            J1 = J2;
+            J2 = __builtin_amdgcn_readfirstlane(jn);
+#pragma unroll
+            for (int n = 0; n < NAV; ++n) off2[n] = __builtin_amdgcn_readfirstlane(on[n]);
+            // group 1's direct loads to the other buffer (started a slot ago) have landed; group 0's
+            // have another slot
+            barrier_vmem < G1 ? 2 * NAV : 63 > ();
+        };
+        auto mul_phase = [&](int cur, bool last) {
+            if constexpr (G1) {
+                // J1 is already the tile of step st + 2, whose buffer is the one just read
+                issueC(J1, cur);
+                fence_compiler();
+            }
+            mul();
+            if (!last) barrier_vmem < G1 ? 63 : 2 * NAV > ();
+        };
+        if constexpr (G1) {
+            issueC(J1, 1);
+            fence_compiler();
+            barrier_vmem<63>();
+        }
+        int st = 0;
+        for (; st + 1 < nsteps; st += 2) {
+            read_phase(0, st, a1, a0);
+            mul_phase(0, false);
+            read_phase(1, st + 1, a0, a1);
+            mul_phase(1, G1 && st + 2 >= nsteps);
+        }
+        if (st < nsteps) {
+            read_phase(0, st, a1, a0);
+            mul_phase(0, G1);
+        }
+        wait_vmem<0>();  // direct loads of steps past the end land before the LDS is released
+    };
     if (nsteps > 0) {
+        auto go = [&](auto ni) {
+            if constexpr (DC && NWAVE == 8) {
+                if (w < 4)
+                    mainloop_pp(ni, std::false_type{});
+                else
+                    mainloop_pp(ni, std::true_type{});
+            } else {
+                mainloop(ni);
+            }
+        };
         if (nfr == 4)
-            mainloop(std::integral_constant<int, 4>{});
+            go(std::integral_constant<int, 4>{});
         else if (nfr == 2)
-            mainloop(std::integral_constant<int, 2>{});
+            go(std::integral_constant<int, 2>{});
         else
-            mainloop(std::integral_constant<int, 0>{});
+            go(std::integral_constant<int, 0>{});
     }
     const size_t xq = static_cast<size_t>(q) * xrows * ldc;
 #pragma unroll
