@@ -26,6 +26,7 @@
 #include "../ints/hostlinalg.hpp"
 #include "kernels.hpp"
 #include "kernels_f64.hpp"
+#include "kernels_fit.hpp"
 #include "kernels_ints.hpp"
 #include "kernels_k.hpp"
 #include "kernels_schwarz.hpp"
@@ -92,7 +93,8 @@ void copy2d_settled(void* dst, size_t dpitch, const void* src, size_t spitch, si
     hcheck(hipDeviceSynchronize(), what);
 }
 
-// Growable device buffer.
+// Growable device buffer.  At least 1 MiB: the builds of a small system then fit what the first one
+// allocated, whatever their precision and form (an allocation costs as much as such a build).
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -107,7 +109,7 @@ struct DevBuf {
     }
     template <class T>
     T* get(size_t count) {
-        const size_t need = std::max<size_t>(count * sizeof(T), 256);
+        const size_t need = std::max<size_t>(count * sizeof(T), size_t(1) << 20);
         if (need > bytes) {
             release();
             hcheck(hipMalloc(&p, need), "hipMalloc");
@@ -240,8 +242,8 @@ struct dfjk_handle {
     double bw_alpha = 1.0, bw_beta = 0.0;
     std::vector<double> fit_M;      // host metric factor, kept for rebuilding Bw after an omega change
     // workspace
-    DevBuf ws_craw, ws_cl, ws_cr, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_Pd, ws_J, ws_K, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
-    DevBuf ws_ct, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
+    DevBuf ws_craw, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_J, ws_K, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
+    DevBuf ws_CB, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
     // column map of the half-transform: the device copy is re-uploaded (from pinned memory,
     // asynchronously) only when it changes
     std::vector<int> cmap_dev;          // what ws_cmap holds
@@ -331,7 +333,7 @@ void build_tiles(dfjk_handle* h) {
 }
 
 int g_kgemm_wgs = 2048;  // workgroups the Q split of the contraction aims at (tuning: PSI4AMD_KGEMM_WGS)
-size_t g_x_budget = size_t(16) << 30;       // FP64 X workspace bytes without a memory setting
+size_t g_x_budget = size_t(8) << 30;        // FP64 X workspace bytes without a memory setting
 size_t g_x_budget_mixed = size_t(4) << 30;  // the same for FP32 / BF16x3 (both: PSI4AMD_X_BUDGET_GB)
 
 // Workspace bytes under the memory setting: what it leaves beyond the resident bytes, capped
@@ -467,69 +469,69 @@ struct Lap {
                            " (metric not positive definite: set DFJK_FIT_EIGEN, psi4's truncating J^-1/2)");
 }
 
-// M = L^-1 with J = L L^T, on the device.  Right-looking blocked Cholesky: each NB x NB
-// diagonal block is factorised and inverted on the host (cholesky_lower, lower_inverse), the
-// panel below it becomes L_ik = A_ik L_kk^-T and the trailing block A_22 -= L_i L_i^T (FP64
-// MFMA GEMMs); then X = L^-1 by block forward substitution, X_i = -L_ii^-1 (L_i,<i X_<i), with
-// the host inverses of the diagonal blocks.  M stays in ws_G for the fit (dM_ready); it is
-// returned on the host (row-major, lower) only when want_host.
+// M = L^-1 with J = L L^T, on the device, without a host round trip per block.  Right-looking blocked
+// Cholesky: one workgroup inverts each 128-row diagonal factor (launch_chol_inverse), the panel below
+// becomes L_ik = A_ik L_kk^-T and the lower blocks of the trailing matrix A_22 -= L_i L_i^T (FP64
+// MFMA GEMMs).  Then L^-1 from its diagonal blocks by doubling: of two neighbouring inverses X_1, X_2
+// of size S the block below the first is -X_2 L_21 X_1, all pairs of a size in one batched
+// product.  M stays in ws_G for the fit (dM_ready); it is returned on the host (row-major, lower)
+// only when want_host.
 std::vector<double> device_metric_factor(dfjk_handle* h, const std::vector<double>& Jm, bool want_host,
                                          const double* dJm = nullptr) {
     const int n = h->naux;
-    constexpr int NB = 256;
+    constexpr int NB = kCholBlock;
     const hipStream_t s = h->stream;
     const size_t nn = static_cast<size_t>(n) * n;
-    DevBuf dA, dP, dPT, dT, dL;
+    DevBuf dA, dP, dPT, dT, dL, dinfo;
     h->dM_ready = false;
     double* A = dA.get<double>(nn);
     double* X = h->ws_G.get<double>(nn);
     double* P = dP.get<double>(static_cast<size_t>(n) * NB);
     double* PT = dPT.get<double>(static_cast<size_t>(n) * NB);
-    double* T = dT.get<double>(static_cast<size_t>(n) * NB);
+    double* T = dT.get<double>(nn / 4 + static_cast<size_t>(n) * NB);
     double* Li = dL.get<double>(static_cast<size_t>(NB) * NB);
+    int* info = dinfo.get<int>(1);
     const size_t ld = static_cast<size_t>(n) * sizeof(double);
     if (dJm)
         hcheck(hipMemcpyAsync(A, dJm, nn * sizeof(double), hipMemcpyDeviceToDevice, s), "copy metric");
     else
         copy_settled(A, Jm.data(), nn * sizeof(double), hipMemcpyHostToDevice, s, "upload metric");
     hcheck(hipMemsetAsync(X, 0, nn * sizeof(double), s), "memset");
-    std::vector<double> blk(NB * NB), invT(NB * NB);
-    std::vector<std::vector<double>> dinv;  // host inverses of the diagonal blocks
+    int bad = n;
+    copy_settled(info, &bad, sizeof(int), hipMemcpyHostToDevice, s, "pivot status");
     for (int k0 = 0; k0 < n; k0 += NB) {
         const int nb = std::min(NB, n - k0), k1 = k0 + nb, m = n - k1;
         const size_t bw = static_cast<size_t>(nb) * sizeof(double);
-        double* Akk = A + static_cast<size_t>(k0) * n + k0;
-        copy2d_settled(blk.data(), bw, Akk, ld, bw, nb, hipMemcpyDeviceToHost, s, "diagonal block");
-        const int bad = cholesky_lower(blk.data(), nb, h->nthreads);
-        if (bad >= 0) cholesky_failed(k0 + bad);
-        dinv.emplace_back(static_cast<size_t>(nb) * nb);
-        std::vector<double>& inv = dinv.back();
-        lower_inverse(blk.data(), nb, inv.data(), h->nthreads);
-        for (int r = 0; r < nb; ++r)
-            for (int c = 0; c < nb; ++c) invT[static_cast<size_t>(c) * nb + r] = inv[static_cast<size_t>(r) * nb + c];
-        copy2d_settled(Akk, ld, blk.data(), bw, bw, nb, hipMemcpyHostToDevice, s, "L_kk");
-        copy2d_settled(X + static_cast<size_t>(k0) * n + k0, ld, inv.data(), bw, bw, nb, hipMemcpyHostToDevice, s,
-                       "X_kk");
+        launch_chol_inverse(A + static_cast<size_t>(k0) * n + k0, n, nb, k0, X + static_cast<size_t>(k0) * n + k0, n, Li,
+                            info, s);
         if (m > 0) {
-            copy_settled(Li, invT.data(), bw * nb, hipMemcpyHostToDevice, s, "L_kk^-T");
             double* Aik = A + static_cast<size_t>(k1) * n + k0;
             launch_gemm_nn_f64(Aik, n, Li, nb, P, nb, m, nb, nb, 1.0, 0.0, s);
             hcheck(hipMemcpy2DAsync(Aik, ld, P, bw, bw, m, hipMemcpyDeviceToDevice, s), "panel");
             launch_transpose(P, m, nb, nb, PT, m, s);
-            launch_gemm_nn_f64(P, nb, PT, m, A + static_cast<size_t>(k1) * n + k1, n, m, m, nb, -1.0, 1.0, s);
+            launch_gemm_nn_f64(P, nb, PT, m, A + static_cast<size_t>(k1) * n + k1, n, m, m, nb, -1.0, 1.0, s, 1, 0, 0, 0, 0,
+                               1);
         }
-        // the host blocks are rewritten in the next pass: the copies above must have run
-        hcheck(hipStreamSynchronize(s), "panel");
     }
-    for (int i0 = NB, bi = 1; i0 < n; i0 += NB, ++bi) {
-        const int nb = std::min(NB, n - i0);
-        launch_gemm_nn_f64(A + static_cast<size_t>(i0) * n, n, X, n, T, i0, nb, i0, i0, 1.0, 0.0, s);
-        copy_settled(Li, dinv[bi].data(), static_cast<size_t>(nb) * nb * sizeof(double), hipMemcpyHostToDevice, s,
-                     "L_ii^-1");
-        launch_gemm_nn_f64(Li, nb, T, i0, X + static_cast<size_t>(i0) * n, n, nb, i0, nb, -1.0, 0.0, s, 1, 0, 0, 0,
-                           1);
-        hcheck(hipStreamSynchronize(s), "block row");
+    for (int S = NB; S < n; S *= 2) {
+        // pairs (r0, r0 + S), r0 = 2 S z: the whole ones in one batch, a last one with a short second block
+        const size_t step = static_cast<size_t>(2 * S) * (n + 1);
+        const int whole = n / (2 * S);
+        auto pairs = [&](int z0, int nz, int S2) {
+            const size_t o = z0 * step;
+            const double* L21 = A + o + static_cast<size_t>(S) * n;
+            const double* X1 = X + o;
+            const double* X2 = X + o + static_cast<size_t>(S) * (n + 1);
+            double* X21 = X + o + static_cast<size_t>(S) * n;
+            launch_gemm_nn_f64(L21, n, X1, n, T, S, S2, S, S, 1.0, 0.0, s, nz, step, step, static_cast<size_t>(S2) * S);
+            launch_gemm_nn_f64(X2, n, T, S, X21, n, S2, S, S2, -1.0, 0.0, s, nz, step, static_cast<size_t>(S2) * S, step, 1);
+        };
+        if (whole) pairs(0, whole, S);
+        const int r1 = whole * 2 * S + S;
+        if (r1 < n) pairs(whole, 1, n - r1);
     }
+    copy_settled(&bad, info, sizeof(int), hipMemcpyDeviceToHost, s, "pivot status");
+    if (bad < n) cholesky_failed(bad);
     h->dM_ready = true;
     std::vector<double> M;
     if (want_host) {
@@ -660,6 +662,9 @@ void fit_on_device(dfjk_handle* h, const std::vector<double>& M, const std::vect
     double* dM = h->ws_G.get<double>(static_cast<size_t>(na) * na);
     if (!h->dM_ready)
         copy_settled(dM, M.data(), M.size() * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload metric factor");
+    DevBuf dMF;
+    double* MF = dMF.get<double>(fit_packed_size(na));
+    launch_fit_pack(dM, na, MF, h->stream);
     // chunk of columns so that the staging buffer stays <= ~1 GiB
     size_t cw = std::max<size_t>(TILE2, (size_t(1) << 27) / std::max(1, na));
     cw = std::min(ncolB, cw / TILE2 * TILE2);
@@ -671,14 +676,12 @@ void fit_on_device(dfjk_handle* h, const std::vector<double>& M, const std::vect
                                 hipMemcpyHostToDevice, h->stream),
                "upload (P|mn)");
         if (host_dst) {
-            launch_gemm_nn_f64(dM, na, dA, static_cast<int>(w), dBp, static_cast<int>(w), na, static_cast<int>(w), na,
-                               1.0, 0.0, h->stream, 1, 0, 0, 0, h->fit_lower ? 1 : 0);
+            launch_fit(MF, na, dA, w, w, dBp, w, h->fit_lower, h->stream);
             hcheck(hipMemcpy2DAsync(host_dst + c0, ncolB * sizeof(double), dBp, w * sizeof(double),
                                     w * sizeof(double), na, hipMemcpyDeviceToHost, h->stream),
                    "download fitted B");
         } else {
-            launch_gemm_nn_f64(dM, na, dA, static_cast<int>(w), dBp + c0, static_cast<int>(ncolB), na,
-                               static_cast<int>(w), na, 1.0, 0.0, h->stream, 1, 0, 0, 0, h->fit_lower ? 1 : 0);
+            launch_fit(MF, na, dA, w, w, dBp + c0, ncolB, h->fit_lower, h->stream);
         }
         hcheck(hipStreamSynchronize(h->stream), "fit");
     }
@@ -934,23 +937,18 @@ void fit_device_A(dfjk_handle* h, const std::vector<double>& M, const double* A,
     double* dM = h->ws_G.get<double>(static_cast<size_t>(na) * na);
     if (!h->dM_ready)
         copy_settled(dM, M.data(), M.size() * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload metric factor");
+    DevBuf dMF;
+    double* MF = dMF.get<double>(fit_packed_size(na));
+    launch_fit_pack(dM, na, MF, h->stream);
     if (!host_dst) {
-        double* dBp = dst.get<double>(b_doubles(h));
-        size_t cw = std::max<size_t>(TILE2, (size_t(1) << 30) / (sizeof(double) * std::max(1, na)));
-        cw = std::min(ncolB, cw / TILE2 * TILE2);
-        for (size_t c0 = 0; c0 < ncolB; c0 += cw) {
-            const size_t w = std::min(cw, ncolB - c0);
-            launch_gemm_nn_f64(dM, na, A + c0, static_cast<int>(ncolB), dBp + c0, static_cast<int>(ncolB), na,
-                               static_cast<int>(w), na, 1.0, 0.0, h->stream, 1, 0, 0, 0, h->fit_lower ? 1 : 0);
-        }
+        launch_fit(MF, na, A, ncolB, ncolB, dst.get<double>(b_doubles(h)), ncolB, h->fit_lower, h->stream);
     } else {
         size_t cw = std::max<size_t>(TILE2, (size_t(1) << 27) / std::max(1, na));
         cw = std::min(ncolB, cw / TILE2 * TILE2);
         double* tmp = h->ws_XR.get<double>(static_cast<size_t>(na) * cw);
         for (size_t c0 = 0; c0 < ncolB; c0 += cw) {
             const size_t w = std::min(cw, ncolB - c0);
-            launch_gemm_nn_f64(dM, na, A + c0, static_cast<int>(ncolB), tmp, static_cast<int>(w), na,
-                               static_cast<int>(w), na, 1.0, 0.0, h->stream, 1, 0, 0, 0, h->fit_lower ? 1 : 0);
+            launch_fit(MF, na, A + c0, ncolB, w, tmp, w, h->fit_lower, h->stream);
             hcheck(hipMemcpy2DAsync(host_dst + c0, ncolB * sizeof(double), tmp, w * sizeof(double),
                                     w * sizeof(double), na, hipMemcpyDeviceToHost, h->stream),
                    "download fitted B");
@@ -1348,23 +1346,24 @@ ColGroups one_group(const double* src, int ncol, const double* partner) {
     return cg;
 }
 
-// D = Cl Cr^T (jk.cc:314-354), FP64: the contraction kernel over the columns of the packed C
+// D = Cl Cr^T (jk.cc:314-354), FP64: the contraction kernel over the columns of the packed C.  Its
+// workspace is that of the build that follows on the stream.
 void compute_D(dfjk_handle* h, const double* dCl, const double* dCr, int ncol, double* D, Work& wk) {
     const hipStream_t s = h->stream;
     const bool sym = dCr == nullptr || dCr == dCl;
     const int ncb = (ncol + 15) / 16, nk = (ncol + 7) / 8;
     const size_t csz = static_cast<size_t>(h->nbfp) * 16 * ncb;
-    double* DL = wk.get<double>(h->ws_cl, csz);
+    double* DL = wk.get<double>(h->ws_CA, csz);
     launch_pack_frag(one_group(dCl, ncol, dCl), h->nbf, h->nbfp, nullptr, DL, s);
     double* DR = DL;
     if (!sym) {
-        DR = wk.get<double>(h->ws_cr, csz);
+        DR = wk.get<double>(h->ws_CD, csz);
         launch_pack_frag(one_group(dCr, ncol, dCr), h->nbf, h->nbfp, nullptr, DR, s);
     }
     const int nblk = kc_blocks(h->nT, sym);
     int nsp = kc_choose_splits(h->nT, sym, nk, 1, 64);
     if (wk.fixed()) nsp = 1;
-    double* P = wk.get<double>(h->ws_Pd, static_cast<size_t>(nsp) * nblk * 4096);
+    double* P = wk.get<double>(h->ws_P, static_cast<size_t>(nsp) * nblk * 4096);
     KcSegs sg;
     sg.n = 1;
     sg.nsplit = nsp;
@@ -1756,7 +1755,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     int qblk = nq_total, nsplit = 1;
     double* P = nullptr;
     if (!wk.fixed()) {
-        // bytes of X workspace (16 GiB FP64, 4 GiB in the mixed modes, whose contraction runs
+        // bytes of X workspace (4 GiB in the mixed modes, whose contraction runs
         // best on smaller Q-blocks), or what the memory setting leaves beyond the resident tensor
         size_t budget = prec == DFJK_PREC_FP64 ? g_x_budget : g_x_budget_mixed;
         budget = memory_limited(h, budget,
@@ -2283,7 +2282,7 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
     const size_t csz = static_cast<size_t>(nbfp) * 16 * ncb, xq = csz, zq = static_cast<size_t>(256) * ncb * ncb;
     double* CA = h->ws_CA.get<double>(csz);
     double* CD = h->ws_CD.get<double>(csz);
-    double* CB = h->ws_cl.get<double>(csz);
+    double* CB = h->ws_CB.get<double>(csz);
     launch_pack_frag(one_group(dC, nocc, dC), nbf, nbfp, CA, CD, s);
     launch_pack_rows(dC, nocc, nocc, nbf, nbfp, ncb, CB, s);
 
@@ -2861,9 +2860,9 @@ int dfjk_finalize(dfjk_handle* h) {
     return guarded([&] {
         require_state(h, false);
         if (h->initialized && h->stream) hcheck(hipStreamSynchronize(h->stream), "finalize");
-        DevBuf* ws[] = {&h->ws_craw, &h->ws_cl,  &h->ws_cr,  &h->ws_D,    &h->ws_W,  &h->ws_dpart, &h->ws_d,
-                        &h->ws_Jpart, &h->ws_XL, &h->ws_XR,  &h->ws_P,    &h->ws_Pd, &h->ws_J,     &h->ws_K,
-                        &h->ws_G,    &h->ws_sign, &h->ws_c32, &h->ws_cbf, &h->ws_cmap, &h->ws_ct,   &h->ws_red,
+        DevBuf* ws[] = {&h->ws_craw, &h->ws_CB, &h->ws_D,    &h->ws_W,  &h->ws_dpart, &h->ws_d,
+                        &h->ws_Jpart, &h->ws_XL, &h->ws_XR,  &h->ws_P, &h->ws_J,     &h->ws_K,
+                        &h->ws_G,    &h->ws_sign, &h->ws_c32, &h->ws_cbf, &h->ws_cmap,   &h->ws_red,
                         &h->ws_Y,    &h->ws_PC,  &h->ws_gam, &h->ws_dc, &h->ws_stage[0], &h->ws_stage[1],
                         &h->ws_stage32, &h->ws_stage32t, &h->ws_CA, &h->ws_CD, &h->ws_M};
         for (DevBuf* b : ws) b->release();

@@ -280,13 +280,15 @@ __global__ __launch_bounds__(256 * kTrGroups) void k_tile_reduce(const double* _
 // Row-major C = alpha*A*B + beta*C, 128x128 output tiles, FP64 MFMA, 4 waves of 64x64.
 // grid = (ceil(N/128), ceil(M/128), batch); operand z is offset by z * stride (0 = shared).
 // lower_a: A is lower triangular (A[m][k] = 0 for k > m), so row block m0 stops at k = m0 + 128.
+// lower_c: only the 128 x 128 blocks on and below the diagonal of C are formed.
 // K-step 16, double-buffered LDS: the next step's operands are loaded into registers before
 // the current step's MFMAs and stored to the other buffer after them, one barrier per step.
 // Out-of-range elements load as zero.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_nn_f64(
     const double* __restrict__ A, int lda, const double* __restrict__ Bm, int ldb, double* __restrict__ Cm, int ldc,
-    int M, int N, int K, double alpha, double beta, size_t sA, size_t sB, size_t sC, int lower_a) {
+    int M, int N, int K, double alpha, double beta, size_t sA, size_t sB, size_t sC, int lower_a, int lower_c) {
     constexpr int KS = 16;
+    if (lower_c && blockIdx.x > blockIdx.y) return;
     __shared__ double As[2][128][17];
     __shared__ double Bs[2][16][132];
     A += blockIdx.z * sA;
@@ -478,12 +480,12 @@ void launch_tile_reduce(const double* P, int nsplit, int ntile, const int* d_til
 
 void launch_gemm_nn_f64(const double* A, int lda, const double* B, int ldb, double* C, int ldc, int M, int N, int K,
                         double alpha, double beta, hipStream_t s, int batch, size_t sA, size_t sB, size_t sC,
-                        int lower_a) {
+                        int lower_a, int lower_c) {
     require(lda >= K && ldb >= N && ldc >= N && batch >= 1 && batch <= 65535, "gemm_nn_f64");
     if (M <= 0 || N <= 0) return;
     dim3 grid((N + 127) / 128, (M + 127) / 128, batch);
     hipLaunchKernelGGL(k_gemm_nn_f64, grid, dim3(256), 0, s, A, lda, B, ldb, C, ldc, M, N, K, alpha, beta, sA, sB, sC,
-                       lower_a);
+                       lower_a, lower_c);
 }
 
 // ---- adjoint helpers ----
