@@ -19,6 +19,7 @@ PREC_FP32 = _core.PREC_FP32
 PREC_BF16X3 = _core.PREC_BF16X3
 FIT_CHOLESKY = _core.FIT_CHOLESKY
 FIT_EIGEN = _core.FIT_EIGEN
+trim_memory = _core.trim_memory
 
 _SUPPORTED = ("DF", "MEM_DF")
 

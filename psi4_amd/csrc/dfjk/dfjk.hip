@@ -93,17 +93,96 @@ void copy2d_settled(void* dst, size_t dpitch, const void* src, size_t spitch, si
     hcheck(hipDeviceSynchronize(), what);
 }
 
+// Device memory that handles gave back, kept for the next allocation of about the same size: at most
+// kPoolBytes in all.  hipMalloc costs 0.1-0.4 ms, and 30 ms per GB once the process has cycled through
+// the card's memory (freed pages are cleared before they are handed out again): a set-up of
+// (H2O)16 allocates 3.4 GB, which took 105 of its 121 ms in such a process.  A block enters the pool
+// when the device is idle, as hipFree would leave it, so any stream and thread may take it.  Blocks
+// are given back oldest first when the bound is reached, all of them when an allocation fails, and by
+// dfjk_trim_memory; free-memory decisions count them as free.
+constexpr size_t kPoolBytes = size_t(4) << 30;
+class DevPool {
+   public:
+    // a block of at least need bytes on device dev (its size in *got), or nullptr
+    void* take(size_t need, int dev, size_t* got) {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t best = blocks_.size();
+        for (size_t i = 0; i < blocks_.size(); ++i) {
+            const Block& b = blocks_[i];
+            if (b.dev != dev || b.bytes < need || b.bytes > need + need / 4) continue;
+            if (best == blocks_.size() || b.bytes < blocks_[best].bytes) best = i;
+        }
+        if (best == blocks_.size()) return nullptr;
+        void* p = blocks_[best].p;
+        *got = blocks_[best].bytes;
+        total_ -= *got;
+        blocks_.erase(blocks_.begin() + best);
+        return p;
+    }
+    void give(void* p, size_t bytes, int dev) {
+        int cur = -1;
+        if (bytes <= kPoolBytes && hipGetDevice(&cur) == hipSuccess && cur == dev &&
+            hipDeviceSynchronize() == hipSuccess) {
+            std::lock_guard<std::mutex> lock(mu_);
+            while (total_ + bytes > kPoolBytes) drop_oldest();
+            blocks_.push_back({p, bytes, dev});
+            total_ += bytes;
+            return;
+        }
+        (void)hipFree(p);
+    }
+    void trim() {
+        std::lock_guard<std::mutex> lock(mu_);
+        while (!blocks_.empty()) drop_oldest();
+    }
+    size_t held(int dev) {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t n = 0;
+        for (const Block& b : blocks_) n += b.dev == dev ? b.bytes : 0;
+        return n;
+    }
+
+   private:
+    struct Block {
+        void* p;
+        size_t bytes;
+        int dev;
+    };
+    void drop_oldest() {
+        (void)hipFree(blocks_.front().p);
+        total_ -= blocks_.front().bytes;
+        blocks_.erase(blocks_.begin());
+    }
+    std::mutex mu_;
+    std::vector<Block> blocks_;
+    size_t total_ = 0;
+};
+// never destroyed: the runtime may be gone when static objects are
+DevPool& dev_pool() {
+    static DevPool* p = new DevPool;
+    return *p;
+}
+// Free bytes of the current device, the pool's blocks among them
+size_t device_free_bytes() {
+    size_t free_b = 0, total_b = 0;
+    hcheck(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    int dev = 0;
+    hcheck(hipGetDevice(&dev), "hipGetDevice");
+    return free_b + dev_pool().held(dev);
+}
+
 // Growable device buffer.  At least 1 MiB: the builds of a small system then fit what the first one
 // allocated, whatever their precision and form (an allocation costs as much as such a build).
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    int dev = 0;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) dev_pool().give(p, bytes, dev);
         p = nullptr;
         bytes = 0;
     }
@@ -112,8 +191,20 @@ struct DevBuf {
         const size_t need = std::max<size_t>(count * sizeof(T), size_t(1) << 20);
         if (need > bytes) {
             release();
-            hcheck(hipMalloc(&p, need), "hipMalloc");
-            bytes = need;
+            hcheck(hipGetDevice(&dev), "hipGetDevice");
+            size_t got = need;
+            p = dev_pool().take(need, dev, &got);
+            if (!p) {
+                hipError_t e = hipMalloc(&p, need);
+                if (e == hipErrorOutOfMemory) {
+                    (void)hipGetLastError();
+                    dev_pool().trim();
+                    e = hipMalloc(&p, need);
+                }
+                if (e != hipSuccess) p = nullptr;
+                hcheck(e, "hipMalloc");
+            }
+            bytes = got;
         }
         return static_cast<T*>(p);
     }
@@ -242,7 +333,7 @@ struct dfjk_handle {
     double bw_alpha = 1.0, bw_beta = 0.0;
     std::vector<double> fit_M;      // host metric factor, kept for rebuilding Bw after an omega change
     // workspace
-    DevBuf ws_craw, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_J, ws_K, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
+    DevBuf ws_craw, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_out, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
     DevBuf ws_CB, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
     // column map of the half-transform: the device copy is re-uploaded (from pinned memory,
     // asynchronously) only when it changes
@@ -250,6 +341,8 @@ struct dfjk_handle {
     int* cmap_pin = nullptr;            // pinned staging of the last upload
     size_t cmap_pin_cap = 0;
     hipEvent_t ev_cmap = nullptr;       // that upload has been read
+    char* io_pin = nullptr;             // pinned staging of the host-array entry points
+    size_t io_pin_cap = 0;
     int8_t* sign_pin = nullptr;         // pinned copy of the column-structure test
     size_t sign_pin_cap = 0;
     // timing
@@ -877,8 +970,7 @@ bool gpu_three_index(dfjk_handle* h, double omega, DevBuf& Abuf) {
         if (sh.l > 4) return false;
     const size_t ncolB = static_cast<size_t>(h->ntp) * TILE2;
     const size_t abytes = static_cast<size_t>(h->naux) * ncolB * sizeof(double);
-    size_t free_b = 0, total_b = 0;
-    hcheck(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    const size_t free_b = device_free_bytes();
     // the fit writes B (omega = 0) or the attenuated tensor: count it unless already allocated
     const DevBuf& fit_dst = omega > 0.0 ? h->dBw : h->dB;
     const size_t dst_bytes = fit_dst.bytes >= abytes ? 0 : abytes;
@@ -983,8 +1075,7 @@ void choose_subalgorithm(dfjk_handle* h) {
     } else if (h->subalgo == DFJK_SUBALGO_INCORE) {
         h->ooc = false;
     } else {
-        size_t free_b = 0, total_b = 0;
-        hcheck(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        const size_t free_b = device_free_bytes();
         h->ooc = resident_doubles(h) * sizeof(double) + (size_t(4) << 30) > free_b;
     }
     if (h->ooc && h->do_wK)  // dfhelper.cc:201-205
@@ -1128,8 +1219,7 @@ int choose_nsplit(int ntile, int nbatch) {
 // hi/lo as it stages each block.
 // A copy that does not fit the free device memory is refused with a message that says so.
 void require_copy_room(size_t bytes) {
-    size_t free_b = 0, total_b = 0;
-    hcheck(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    const size_t free_b = device_free_bytes();
     if (bytes > free_b)
         fail(DFJK_ERR_MEMORY, "DFJK: the FP32 copies of B for the mixed precisions need " +
                                   std::to_string(bytes >> 20) + " MiB more device memory, " +
@@ -2054,41 +2144,120 @@ void reset_timers(dfjk_handle* h) {
     ensure_stream(h);
 }
 
+// Copies between host arrays and the device through the handle's pinned staging: queued on its stream
+// with no host wait of their own (pageable copies cost a drained stream, a synchronous copy and
+// an idle device each, copy_settled: an (H2O)4 build took 147 us with them, 109 with these).  Up to kPinBytes per direction and
+// call; larger transfers, or no pinned memory, take copy_settled.
+constexpr size_t kPinBytes = size_t(64) << 20;
+struct HostCopy {
+    double* dev;
+    double* host;
+    size_t n;  // doubles
+};
+bool pin_room(dfjk_handle* h, const std::vector<HostCopy>& x) {
+    size_t need = 0;
+    for (const HostCopy& c : x) need += c.n * sizeof(double);
+    if (need > kPinBytes) return false;
+    if (need > h->io_pin_cap) {
+        if (h->io_pin) hcheck(hipHostFree(h->io_pin), "hipHostFree");
+        h->io_pin = nullptr;
+        h->io_pin_cap = 0;
+        const size_t cap = std::max<size_t>(need, size_t(1) << 20);
+        if (hipHostMalloc(reinterpret_cast<void**>(&h->io_pin), cap, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            h->io_pin = nullptr;
+            return false;
+        }
+        h->io_pin_cap = cap;
+    }
+    return true;
+}
+// one copy per run of adjacent device arrays
+template <class F>
+void for_runs(const std::vector<HostCopy>& x, F&& f) {
+    size_t off = 0;
+    for (size_t i = 0; i < x.size();) {
+        size_t j = i + 1, n = x[i].n;
+        while (j < x.size() && x[j].dev == x[j - 1].dev + x[j - 1].n) n += x[j++].n;
+        f(x[i].dev, off, n * sizeof(double));
+        off += n * sizeof(double);
+        i = j;
+    }
+}
+// (the staging is free: every call that fills it ends by waiting for the stream)
+void upload_arrays(dfjk_handle* h, const std::vector<HostCopy>& x, const char* what) {
+    if (!pin_room(h, x)) {
+        for (const HostCopy& c : x) copy_settled(c.dev, c.host, c.n * sizeof(double), hipMemcpyHostToDevice, h->stream, what);
+        return;
+    }
+    size_t off = 0;
+    for (const HostCopy& c : x) {
+        std::memcpy(h->io_pin + off, c.host, c.n * sizeof(double));
+        off += c.n * sizeof(double);
+    }
+    for_runs(x, [&](double* dev, size_t o, size_t bytes) {
+        hcheck(hipMemcpyAsync(dev, h->io_pin + o, bytes, hipMemcpyHostToDevice, h->stream), what);
+    });
+}
+// The results, after the work queued on the stream; waits for them.
+void download_arrays(dfjk_handle* h, const std::vector<HostCopy>& x, const char* what) {
+    if (!x.empty() && pin_room(h, x)) {
+        for_runs(x, [&](double* dev, size_t o, size_t bytes) {
+            hcheck(hipMemcpyAsync(h->io_pin + o, dev, bytes, hipMemcpyDeviceToHost, h->stream), what);
+        });
+        hcheck(hipStreamSynchronize(h->stream), what);
+        size_t off = 0;
+        for (const HostCopy& c : x) {
+            std::memcpy(c.host, h->io_pin + off, c.n * sizeof(double));
+            off += c.n * sizeof(double);
+        }
+        return;
+    }
+    for (const HostCopy& c : x) copy_settled(c.host, c.dev, c.n * sizeof(double), hipMemcpyDeviceToHost, h->stream, what);
+    hcheck(hipStreamSynchronize(h->stream), what);
+}
+
 // J, K (and D) of a batch of pairs whose pointers are the caller's (device or host).
 void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool device, char* arena,
                size_t arena_bytes) {
     const size_t nn = static_cast<size_t>(h->nbf) * h->nbf;
     const int np = static_cast<int>(batch.size());
     std::vector<PairIn> pr(batch);
+    std::vector<HostCopy> down;
     if (!device) {
         // operands to the device, an array that several pairs share once
         size_t csum = 0;
         for (const PairIn& p : batch) csum += (p.cr ? 2 : 1) * static_cast<size_t>(h->nbf) * p.ncol;
         double* raw = h->ws_craw.get<double>(csum);
-        std::vector<std::pair<std::pair<const double*, int>, double*>> seen;
-        auto up = [&](const double* c, int ncol, const char* what) -> const double* {
-            for (const auto& e : seen)
-                if (e.first.first == c && e.first.second == ncol) return e.second;
+        std::vector<HostCopy> upl;
+        auto up = [&](const double* c, int ncol) -> const double* {
             const size_t csz = static_cast<size_t>(h->nbf) * ncol;
-            copy_settled(raw, c, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, what);
-            seen.push_back({{c, ncol}, raw});
+            for (const HostCopy& e : upl)
+                if (e.host == c && e.n == csz) return e.dev;
+            upl.push_back({raw, const_cast<double*>(c), csz});
             raw += csz;
-            return seen.back().second;
+            return upl.back().dev;
         };
-        double* gD = h->ws_D.get<double>(nn * np);
-        double* gJ = h->ws_J.get<double>(nn * np);
-        double* gK = h->ws_K.get<double>(nn * np);
         for (int i = 0; i < np; ++i) {
-            pr[i].cl = up(batch[i].cl, batch[i].ncol, "upload C_left");
-            if (batch[i].cr) pr[i].cr = up(batch[i].cr, batch[i].ncol, "upload C_right");
-            if (batch[i].D) pr[i].D = gD + nn * i;
-            if (batch[i].J) pr[i].J = gJ + nn * i;
-            if (batch[i].K) pr[i].K = gK + nn * i;
-            if (accumulate) {
-                if (batch[i].J) copy_settled(pr[i].J, batch[i].J, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
-                if (batch[i].K) copy_settled(pr[i].K, batch[i].K, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
-            }
+            pr[i].cl = up(batch[i].cl, batch[i].ncol);
+            if (batch[i].cr) pr[i].cr = up(batch[i].cr, batch[i].ncol);
         }
+        size_t nout = 0;
+        for (const PairIn& p : batch) nout += (p.D ? 1 : 0) + (p.J ? 1 : 0) + (p.K ? 1 : 0);
+        double* g = h->ws_out.get<double>(nn * nout);
+        for (int i = 0; i < np; ++i) {
+            auto place = [&](double* host, double*& dev, bool wanted, bool add) {
+                if (!host) return;
+                dev = g;
+                g += nn;
+                if (wanted) down.push_back({dev, host, nn});
+                if (add) upl.push_back({dev, host, nn});
+            };
+            place(batch[i].D, pr[i].D, true, false);
+            place(batch[i].J, pr[i].J, h->do_J, accumulate);
+            place(batch[i].K, pr[i].K, h->do_K, accumulate);
+        }
+        upload_arrays(h, upl, "upload");
     }
     Work wk;  // per batch: the batches run in stream order, so a fixed arena is reused
     wk.base = arena;
@@ -2110,16 +2279,7 @@ void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool 
     } else {
         for (int i = 0; i < np; ++i) compute_pair(h, pr[i], form[i], accumulate, wk);
     }
-    if (!device) {
-        for (int i = 0; i < np; ++i) {
-            if (batch[i].D) copy_settled(batch[i].D, pr[i].D, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download D");
-            if (batch[i].J && h->do_J)
-                copy_settled(batch[i].J, pr[i].J, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download J");
-            if (batch[i].K && h->do_K)
-                copy_settled(batch[i].K, pr[i].K, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download K");
-        }
-        hcheck(hipStreamSynchronize(h->stream), "compute");
-    }
+    if (!device) download_arrays(h, down, "download");
 }
 
 // arena: null for the allocating entry points, else the device address of this device's
@@ -2235,22 +2395,20 @@ void compute_wk_impl(dfjk_handle* h, int n, const double* const* Cl, const doubl
         double* gW = dW;
         if (!device) {
             double* raw = h->ws_craw.get<double>(2 * csz);
-            copy_settled(raw, cl, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload C_left");
+            gW = h->ws_out.get<double>(nn);
+            std::vector<HostCopy> upl{{raw, const_cast<double*>(cl), csz}};
             cl = raw;
             if (cr) {
-                copy_settled(raw + csz, cr, csz * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload C_right");
+                upl.push_back({raw + csz, const_cast<double*>(cr), csz});
                 cr = raw + csz;
             }
-            gW = h->ws_K.get<double>(nn);
-            if (accumulate) copy_settled(gW, dW, nn * sizeof(double), hipMemcpyHostToDevice, h->stream, "up");
+            if (accumulate) upl.push_back({gW, dW, nn});
+            upload_arrays(h, upl, "upload");
         }
         compute_wk_pair(h, cl, cr, ncol[i], gW, accumulate);
         // lr_symmetric: MemDFJK::compute_JK hermitivitizes wK (MemDFJK.cc:101-107)
         if (!cr) launch_hermitivitize(gW, h->nbf, h->nbf, h->stream);
-        if (!device) {
-            copy_settled(dW, gW, nn * sizeof(double), hipMemcpyDeviceToHost, h->stream, "download wK");
-            hcheck(hipStreamSynchronize(h->stream), "compute wK");
-        }
+        if (!device) download_arrays(h, {{gW, dW, nn}}, "download wK");
     }
     finish_timers(h);
 }
@@ -2427,6 +2585,7 @@ int dfjk_destroy(dfjk_handle* h) {
         if (h->hB) (void)hipHostFree(h->hB);
         if (h->cmap_pin) (void)hipHostFree(h->cmap_pin);
         if (h->sign_pin) (void)hipHostFree(h->sign_pin);
+        if (h->io_pin) (void)hipHostFree(h->io_pin);
         if (h->ev_cmap) (void)hipEventDestroy(h->ev_cmap);
         delete h;
         if (cs) (void)hipStreamDestroy(cs);
@@ -2856,12 +3015,16 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc) {
     });
 }
 
+int dfjk_trim_memory(void) {
+    return guarded([&] { dev_pool().trim(); });
+}
+
 int dfjk_finalize(dfjk_handle* h) {
     return guarded([&] {
         require_state(h, false);
         if (h->initialized && h->stream) hcheck(hipStreamSynchronize(h->stream), "finalize");
         DevBuf* ws[] = {&h->ws_craw, &h->ws_CB, &h->ws_D,    &h->ws_W,  &h->ws_dpart, &h->ws_d,
-                        &h->ws_Jpart, &h->ws_XL, &h->ws_XR,  &h->ws_P, &h->ws_J,     &h->ws_K,
+                        &h->ws_Jpart, &h->ws_XL, &h->ws_XR,  &h->ws_P, &h->ws_out,
                         &h->ws_G,    &h->ws_sign, &h->ws_c32, &h->ws_cbf, &h->ws_cmap,   &h->ws_red,
                         &h->ws_Y,    &h->ws_PC,  &h->ws_gam, &h->ws_dc, &h->ws_stage[0], &h->ws_stage[1],
                         &h->ws_stage32, &h->ws_stage32t, &h->ws_CA, &h->ws_CD, &h->ws_M};

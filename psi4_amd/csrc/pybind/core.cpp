@@ -205,11 +205,13 @@ class JK {
                 D_.push_back(Arr({nbf_, nbf_}));
                 J_.push_back(Arr({nbf_, nbf_}));
                 K_.push_back(Arr({nbf_, nbf_}));
-                std::fill(J_.back().mutable_data(), J_.back().mutable_data() + nbf_ * nbf_, 0.0);
-                std::fill(K_.back().mutable_data(), K_.back().mutable_data() + nbf_ * nbf_, 0.0);
+                // what compute does not overwrite starts from zero
+                auto zero = [&](Arr& a) { std::fill(a.mutable_data(), a.mutable_data() + a.size(), 0.0); };
+                if (accumulate_ || !do_J_) zero(J_.back());
+                if (accumulate_ || !do_K_) zero(K_.back());
                 if (do_wK_) {
                     wK_.push_back(Arr({nbf_, nbf_}));
-                    std::fill(wK_.back().mutable_data(), wK_.back().mutable_data() + nbf_ * nbf_, 0.0);
+                    if (accumulate_) zero(wK_.back());
                 }
             }
         }
@@ -428,6 +430,8 @@ PYBIND11_MODULE(_core, m) {
     m.attr("PREC_BF16X3") = static_cast<int>(DFJK_PREC_BF16X3);
     m.attr("FIT_CHOLESKY") = static_cast<int>(DFJK_FIT_CHOLESKY);
     m.attr("FIT_EIGEN") = static_cast<int>(DFJK_FIT_EIGEN);
+    m.def("trim_memory", [] { check(dfjk_trim_memory()); },
+          "give back the device memory kept from finished JK objects (4 GiB at most)");
     py::class_<JK, std::shared_ptr<JK>>(m, "JK", py::dynamic_attr())
         .def_static("build_JK", &JK::build, py::arg("basis"), py::arg("aux"), py::arg("do_wK") = false,
                     py::arg("doubles") = static_cast<size_t>(256000000))

@@ -157,3 +157,39 @@ def test_adjoint_sizes(gpu_available, nbf, naux, nocc):
         jk.set_aux_range(2, 5)
         E2, dC2, dB2 = jk.energy_adjoint(C, True)
         assert E2 == E and np.array_equal(dC2, dC) and np.array_equal(dB2, dB[2:5])
+
+
+def test_memory_of_finished_handles_is_reused_and_given_back(gpu_available):
+    """Buffers that earlier handles left behind (their contents too) serve later ones of other shapes,
+    also from two threads at once; trim_memory gives the memory back to the device."""
+    import gc
+    import threading
+
+    import torch
+
+    from psi4_amd.core import trim_memory
+
+    announce("handles after handles on reused memory")
+
+    def one(nbf, naux, ncol, bad):
+        jk, B = _tensor(nbf, naux, nbf)
+        C = np.random.default_rng(naux).standard_normal((nbf, ncol))
+        D, J, K = _compute(jk, [C])
+        try:
+            _check(B, C, C, D[0], J[0], K[0])
+        except AssertionError as e:
+            bad.append((nbf, naux, ncol, e))
+
+    bad = []
+    for shape in ((150, 200, 40), (40, 300, 9), (129, 150, 70)):
+        one(*shape, bad)
+    threads = [threading.Thread(target=one, args=(n, 90, 20, bad)) for n in (100, 61)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    gc.collect()
+    before = torch.cuda.mem_get_info()[0]
+    trim_memory()
+    assert torch.cuda.mem_get_info()[0] > before
