@@ -50,7 +50,7 @@ def build_ints(verbose=False):
     return out
 
 
-DFJK_SOURCES = ("kernels.hip", "kernels_f64.hip", "kernels_fit.hip", "kernels_k.hip", "kernels_ints.hip",
+DFJK_SOURCES = ("kernels.hip", "kernels_f64.hip", "kernels_f32.hip", "kernels_fit.hip", "kernels_k.hip", "kernels_ints.hip",
                 "kernels_ints_l0.hip", "kernels_ints_l1.hip", "kernels_ints_l2.hip", "kernels_ints_l3.hip",
                 "kernels_ints_l4.hip", "kernels_schwarz.hip", "kernels_schwarz_f.hip", "dfjk.hip")
 

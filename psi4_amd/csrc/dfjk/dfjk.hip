@@ -25,6 +25,7 @@
 #include "../ints/ints.hpp"
 #include "../ints/hostlinalg.hpp"
 #include "kernels.hpp"
+#include "kernels_f32.hpp"
 #include "kernels_f64.hpp"
 #include "kernels_fit.hpp"
 #include "kernels_ints.hpp"
@@ -1750,7 +1751,9 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     if (need_D) {
         hipEvent_t e0 = tm.begin();
         if (!Dm) Dm = wk.get<double>(h->ws_D, static_cast<size_t>(nbf) * nbf);
+        const size_t mark = wk.used;
         compute_D(h, dCl, dCr, ncol, Dm, wk);
+        wk.used = mark;  // D's operands are dead before the next kernel of this stream
         tm.end(T_OTHER, e0);
     }
 
@@ -1766,20 +1769,26 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     const int prec = h->precision;
     if (doK && prec == DFJK_PREC_FP64) fail(DFJK_ERR_INTERNAL, "FP64 K outside compute_f64");
 
-    // column map of the half-transform
+    // column map of the half-transform: column groups are padded to the contraction's depth, 16 in
+    // FP32 and 32 in BF16
+    const bool f32 = prec == DFJK_PREC_FP32;
+    const int kpad = f32 ? 16 : 32;
     int ncol_eff = ncol, kplus = 0, half = 0, wcross = 0;
     if (signed_sym) {
-        kplus = round_up(static_cast<int>(plus.size()), 32);
-        ncol_eff = kplus + round_up(static_cast<int>(minus.size()), 32);
+        kplus = round_up(static_cast<int>(plus.size()), kpad);
+        ncol_eff = kplus + round_up(static_cast<int>(minus.size()), kpad);
     } else if (cross) {
         half = ncol / 2;
-        wcross = round_up(half, 32);
+        wcross = round_up(half, kpad);
         ncol_eff = 2 * wcross;
     }
     int nbw, npanel, ldc;
     ht_panel_shape(ncol_eff, &nbw, &npanel, &ldc);
+    const int ncb1 = round_up(ncol_eff, 16) / 16;  // FP32: 16-column blocks of the left matrix
+    const int ncb = general ? 2 * ncb1 : ncb1;     // and of X, the right matrix's beside them
+    if (f32) ldc = 16 * ncb;
     int* dmap = nullptr;
-    if (doK) {
+    if (doK && (!f32 || signed_sym || cross)) {
         std::vector<int> cmap(ldc, -1);
         if (signed_sym) {
             for (size_t i = 0; i < plus.size(); ++i) cmap[i] = plus[i];
@@ -1795,7 +1804,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
         dmap = upload_cmap(h, cmap, wk);
     }
     const size_t qs = static_cast<size_t>(h->ntp) * TILE2;  // elements per Q
-    const size_t xq = static_cast<size_t>(xrows) * ldc;      // X elements per Q
+    const size_t xq = static_cast<size_t>(f32 ? nbfp : xrows) * ldc;  // X elements per Q
     const size_t esz = prec == DFJK_PREC_FP64 ? 8 : 4;       // FP64, FP32, or BF16 hi+lo
 
     // resident lower-precision copies (in core); the fixed-workspace entry point allocates
@@ -1840,10 +1849,37 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     const bool upper = sym;
     const int ntile = upper ? h->ntile_sym : h->ntile_all;
     const int2* otiles = upper ? h->d_otiles_sym.as<int2>() : h->d_otiles_all.as<int2>();
-    const size_t per_q = xq * esz * (general ? 2 : 1);  // X bytes per Q
+    const size_t per_q = xq * esz * (general && !f32 ? 2 : 1);  // X bytes per Q
     const size_t csz = static_cast<size_t>(nbfp) * ldc;
     int qblk = nq_total, nsplit = 1;
     double* P = nullptr;
+    // FP32: the passes of one launch and their splits
+    KcSegs segs;
+    double* M = nullptr;
+    auto split_f32 = [&](int nq, size_t budget) {
+        const int k0 = kplus / 16, kc = wcross / 16;
+        if (signed_sym) {
+            if (!plus.empty()) segs.s[segs.n++] = KcSeg{0, 0, 0, 0, k0, 1.0};
+            segs.s[segs.n++] = KcSeg{0, 0, k0, k0, ncb - k0, -1.0};
+        } else if (cross) {
+            segs.s[segs.n++] = KcSeg{0, 0, 0, kc, kc, 1.0};
+        } else {
+            segs.s[segs.n++] = KcSeg{0, 0, 0, general ? ncb1 : 0, ncb1, 1.0};
+        }
+        const size_t bytes = kc32_blocks(h->nT, upper) * kc32_partial * sizeof(double);
+        const size_t most = std::min<size_t>(
+            1 << 20, wk.fixed() ? wk.left() / 4 / (bytes * segs.n)
+                                : std::max<size_t>(budget / 4, size_t(256) << 20) / (bytes * segs.n));
+        for (int i = 0; i < segs.n; ++i) {
+            KcSeg& sg = segs.s[i];
+            sg.sp0 = segs.nsplit;
+            sg.nsp = kc32_choose_splits(h->nT, upper, kc_steps(nq, sg.nk), segs.n,
+                                        static_cast<int>(std::max<size_t>(1, most)));
+            segs.nsplit += sg.nsp;
+        }
+        P = wk.get<double>(h->ws_P, segs.nsplit * kc32_blocks(h->nT, upper) * kc32_partial);
+        if (cross) M = wk.get<double>(h->ws_M, static_cast<size_t>(nbf) * nbf);
+    };
     if (!wk.fixed()) {
         // bytes of X workspace (4 GiB in the mixed modes, whose contraction runs
         // best on smaller Q-blocks), or what the memory setting leaves beyond the resident tensor
@@ -1864,10 +1900,14 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
         }
         const int nblocks0 = (nq_total + qblk - 1) / qblk;
         qblk = (nq_total + nblocks0 - 1) / nblocks0;
-        if (doK) {
+        if (doK && f32) {
+            split_f32(qblk, budget);
+        } else if (doK) {
             nsplit = choose_nsplit(ntile, qblk);
             P = wk.get<double>(h->ws_P, static_cast<size_t>(nsplit) * ntile * 16384);
         }
+    } else if (doK && f32) {
+        split_f32(std::min(nq_total, 65535), 0);
     } else if (doK) {
         // fixed workspace: the K partials take at most a quarter of what is left, the packed C
         // copies their share, and X the rest
@@ -1884,7 +1924,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     };
     // padding columns of X are zero: each pass stops at the contraction's k-step after
     // the last real column of its group
-    const int kstep = prec == DFJK_PREC_BF16X3 ? 32 : 16;
+    const int kstep = 32;
     std::vector<Pass> passes;
     if (signed_sym) {
         if (!plus.empty()) passes.push_back({0, round_up(static_cast<int>(plus.size()), kstep), 1.0, 0, 0});
@@ -1894,18 +1934,23 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     } else {
         passes.push_back({0, std::min(ldc, round_up(ncol, kstep)), 1.0, 0, 0});
     }
-    const float *c32l = nullptr, *c32r = nullptr;
+    float* c32 = nullptr;
     uint16_t *cth_l = nullptr, *ctl_l = nullptr, *cth_r = nullptr, *ctl_r = nullptr;
     char *XL = nullptr, *XR = nullptr;
     if (doK) {
-        if (prec == DFJK_PREC_FP32) {
-            float* a = wk.get<float>(h->ws_c32, 2 * csz);
-            launch_pack_cmap_f32(dCl, ncol, nbf, dmap, a, nbfp, ldc, s);
-            c32l = c32r = a;
+        if (f32) {
+            c32 = wk.get<float>(h->ws_c32, csz);
+            ColGroups cg;
+            cg.ncb = ncb;
             if (general) {
-                launch_pack_cmap_f32(dCr, ncol, nbf, dmap, a + csz, nbfp, ldc, s);
-                c32r = a + csz;
+                cg.n = 2;
+                cg.g[0] = ColGroup{dCl, nullptr, nullptr, ncol, ncol, 0, ncb1};
+                cg.g[1] = ColGroup{dCr, nullptr, nullptr, ncol, ncol, ncb1, ncb1};
+            } else {
+                cg.n = 1;
+                cg.g[0] = ColGroup{dCl, nullptr, dmap, ncol, ncol, 0, ncb1};
             }
+            launch_pack_frag32(cg, nbf, nbfp, c32, s);
         } else if (prec == DFJK_PREC_BF16X3) {
             uint16_t* a = wk.get<uint16_t>(h->ws_cbf, 4 * csz);
             cth_l = a;
@@ -1929,7 +1974,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
             qblk = (nq_total + nb0 - 1) / nb0;
         }
         XL = wk.get<char>(h->ws_XL, xq * esz * qblk);
-        XR = general ? wk.get<char>(h->ws_XR, xq * esz * qblk) : XL;
+        XR = general && !f32 ? wk.get<char>(h->ws_XR, xq * esz * qblk) : XL;
     }
     const int nblocks = (nq_total + qblk - 1) / qblk;
     if (doJ && h->ooc) {
@@ -2021,12 +2066,9 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
         if (doK) {
             const int nsp = std::min(nsplit, nq);
             hipEvent_t e0 = tm.begin();
-            if (prec == DFJK_PREC_FP32) {
-                launch_ht2_f32(g, b32, 0, nq, c32l, ldc, nbw, npanel, reinterpret_cast<float*>(XL), xrows, h->dZero.p,
-                               s);
-                if (general)
-                    launch_ht2_f32(g, b32, 0, nq, c32r, ldc, nbw, npanel, reinterpret_cast<float*>(XR), xrows,
-                                   h->dZero.p, s);
+            if (f32) {
+                launch_ht_f32(g, b32, nq, c32, ncb, ht_row_tiles(h->nT, qblk, ncb), reinterpret_cast<float*>(XL),
+                              h->dZero.p, s);
             } else {
                 uint16_t* xl = reinterpret_cast<uint16_t*>(XL);
                 uint16_t* xr = reinterpret_cast<uint16_t*>(XR);
@@ -2036,25 +2078,22 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
                                   h->dZero.p, s);
             }
             tm.end(T_HT, e0);
-            h->n_ht += general ? 2 : 1;
+            h->n_ht += general && !f32 ? 2 : 1;
             hipEvent_t e1 = tm.begin();
-            for (size_t ip = 0; ip < passes.size(); ++ip) {
-                const Pass& pp = passes[ip];
-                const int acc = (blk > 0 || ip > 0) ? 1 : 0;
-                if (prec == DFJK_PREC_FP32) {
-                    float* xl = reinterpret_cast<float*>(XL) + pp.offl;
-                    float* xr = reinterpret_cast<float*>(XR) + pp.offr;
-                    launch_kgemm2_f32(xl, xr, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp, otiles, ntile, P, pp.alpha,
-                                      acc, upper ? 1 : 0, s);
-                } else {
-                    uint16_t* xl = reinterpret_cast<uint16_t*>(XL) + pp.offl;
-                    uint16_t* xr = reinterpret_cast<uint16_t*>(XR) + pp.offr;
-                    launch_kgemm_bf3(xl, xl + xq * qblk, xr, xr + xq * qblk, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp,
-                                     otiles, ntile, P, pp.alpha, acc, upper ? 1 : 0, s);
-                }
+            if (f32) {
+                launch_kc_f32(reinterpret_cast<const float*>(XL), xq, ncb, h->nT, nq, segs, upper, P, blk > 0 ? 1 : 0, s);
                 h->n_kgemm += 1;
             }
-            if (nsp < nsplit && blk == 0)
+            for (size_t ip = 0; !f32 && ip < passes.size(); ++ip) {
+                const Pass& pp = passes[ip];
+                const int acc = (blk > 0 || ip > 0) ? 1 : 0;
+                uint16_t* xl = reinterpret_cast<uint16_t*>(XL) + pp.offl;
+                uint16_t* xr = reinterpret_cast<uint16_t*>(XR) + pp.offr;
+                launch_kgemm_bf3(xl, xl + xq * qblk, xr, xr + xq * qblk, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp,
+                                 otiles, ntile, P, pp.alpha, acc, upper ? 1 : 0, s);
+                h->n_kgemm += 1;
+            }
+            if (!f32 && nsp < nsplit && blk == 0)
                 launch_zero(P + static_cast<size_t>(nsp) * ntile * 16384,
                             static_cast<size_t>(nsplit - nsp) * ntile * 16384, s);
             tm.end(T_KGEMM, e1);
@@ -2063,8 +2102,16 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     }
     if (doK) {
         hipEvent_t e2 = tm.begin();
-        launch_tile_reduce(P, nsplit, ntile, upper ? h->d_otile_of_sym.as<int>() : h->d_otile_of_all.as<int>(), h->nB,
-                           upper ? 1 : (cross ? 2 : 0), nbf, nbf, dK, nbf, 1.0, accumulate, s);
+        if (f32) {
+            KcOuts o;
+            o.n = 1;
+            o.o[0] = KcOut{0, segs.nsplit, cross ? M : dK};
+            launch_kc32_reduce(P, h->nT, nbf, upper, o, cross ? 0 : accumulate, s);
+            if (cross) launch_add_transpose(M, nbf, dK, accumulate, s);
+        } else {
+            launch_tile_reduce(P, nsplit, ntile, upper ? h->d_otile_of_sym.as<int>() : h->d_otile_of_all.as<int>(),
+                               h->nB, upper ? 1 : (cross ? 2 : 0), nbf, nbf, dK, nbf, 1.0, accumulate, s);
+        }
         tm.end(T_OTHER, e2);
     }
 }

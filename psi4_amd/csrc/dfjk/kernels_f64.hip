@@ -22,39 +22,11 @@
 #include <type_traits>
 
 #include "kernels_f64.hpp"
+#include "wave_kernels.hpp"
 
 namespace p4a {
 
 namespace {
-
-typedef double d2_t __attribute__((ext_vector_type(2)));
-
-constexpr int kXCD = 8;
-constexpr int kSlots = 256;  // waves one XCD holds: 32 CUs x 4 SIMDs x 2 waves
-
-// 16 bytes at a wave-uniform base plus a per-lane byte offset
-__device__ inline d2_t ld2(const double* base, unsigned off) {
-    return *reinterpret_cast<const d2_t*>(reinterpret_cast<const char*>(base) + off);
-}
-__device__ inline double ld1(const double* base, unsigned off) {
-    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
-}
-__device__ inline int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
-
-// Workgroups go round-robin to the XCDs (each with its own L2): wave w of the launch belongs to XCD
-// (workgroup % 8); consecutive waves of an XCD take the items of one group (the row and column blocks
-// of one Q, the output blocks of one split), so a group's operands meet in one L2.
-struct WaveItem {
-    int group, item;
-};
-__device__ inline WaveItem wave_item(int items) {
-    const int wg = blockIdx.x, lw = (wg / kXCD) * (blockDim.x >> 6) + uni(threadIdx.x >> 6);
-    return {(lw / items) * kXCD + wg % kXCD, lw % items};
-}
-inline unsigned wave_grid(int ngroups, int items, int wpw) {  // wpw: waves per workgroup
-    const long long per = static_cast<long long>((ngroups + kXCD - 1) / kXCD) * items;  // waves per XCD
-    return static_cast<unsigned>(kXCD * ((per + wpw - 1) / wpw));
-}
 
 // ------------------------------------------------------------------ packing
 __global__ __launch_bounds__(256) void k_pack_frag(ColGroups cg, int nbf, int nbfp, double* __restrict__ CA,
@@ -101,18 +73,13 @@ __device__ __forceinline__ void ht_body(const double* __restrict__ BQ, const int
     // row 2 lg, column lm of one used transposed
     const unsigned off_n = (lm * TILE + 2 * lg) * 8, off_t = (2 * lg * TILE + lm) * 8, off_c = lane * 16;
     const double* tp[RT];
-    // the first column tile >= j that meets one of the wave's row tiles (nT: none), with the tiles
-    // (an absent one reads zeros)
-    auto seek = [&](int j, const double** t) {
-        for (; j < nT; ++j) {
-            int any = 0;
+    TileRow<RT> row(tidx, nT, I0);
+    auto seek = [&](const double** t) {  // the next tile's rows (an absent one reads zeros)
+        int o[RT];
+        const int j = row.next(o);
+        if (j < nT) {
 #pragma unroll
-            for (int s = 0; s < RT; ++s) {
-                const int I = I0 + s, o = tidx[min(I, j) * nT + max(I, j)];
-                t[s] = o >= 0 ? BQ + static_cast<size_t>(o) * TILE2 : zt;
-                any |= o >= 0;
-            }
-            if (any) break;
+            for (int s = 0; s < RT; ++s) t[s] = o[s] >= 0 ? BQ + static_cast<size_t>(o[s]) * TILE2 : zt;
         }
         return j;
     };
@@ -133,7 +100,6 @@ __device__ __forceinline__ void ht_body(const double* __restrict__ BQ, const int
         const double* cp = CA + (static_cast<size_t>(4 * J + s) * ncb + cb0) * 128;
 #pragma unroll
         for (int i = 0; i < NC; ++i) c[i] = ld2(cp + 128 * i, off_c);
-        __builtin_amdgcn_sched_barrier(0);
     };
     auto mul = [&](const d2_t* a, const d2_t* c) {
 #pragma unroll
@@ -143,26 +109,27 @@ __device__ __forceinline__ void ht_body(const double* __restrict__ BQ, const int
 #pragma unroll
                 for (int f = 0; f < NF; ++f)
                     acc[f][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(c[i][e], a[f][e], acc[f][i], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    // load the next step's operands while this one's are multiplied
+    auto step = [&](auto tr, int J, const double* const* t, int s, d2_t* an, d2_t* cn, const d2_t* a, const d2_t* c) {
+        load(tr, J, t, s, an, cn);
+        mul(a, c);
+        interleave<(decltype(tr)::value ? 2 : 1) * NF + NC, 2 * NF * NC>();
     };
     // Tile J, its step 0 already loaded, and step 0 of tile Jn (past the last tile: of J again, never
     // used), so that every path through the loops issues the same loads and a wait for one step's
     // operands leaves the next step's in flight.
     const double* tn[RT];
-    int J = seek(0, tp), Jn;
+    int J = seek(tp), Jn;
     auto tile = [&](auto tr, auto trn) {
-        load(tr, J, tp, 1, a1, c1);
-        mul(a0, c0);
-        load(tr, J, tp, 2, a0, c0);
-        mul(a1, c1);
-        load(tr, J, tp, 3, a1, c1);
-        mul(a0, c0);
+        step(tr, J, tp, 1, a1, c1, a0, c0);
+        step(tr, J, tp, 2, a0, c0, a1, c1);
+        step(tr, J, tp, 3, a1, c1, a0, c0);
         const bool last = Jn >= nT;
         const double* tl[RT];
 #pragma unroll
         for (int s = 0; s < RT; ++s) tl[s] = last ? tp[s] : tn[s];
-        load(trn, last ? J : Jn, tl, 0, a0, c0);
-        mul(a1, c1);
+        step(trn, last ? J : Jn, tl, 0, a0, c0, a1, c1);
         J = Jn;
 #pragma unroll
         for (int s = 0; s < RT; ++s) tp[s] = tl[s];
@@ -171,17 +138,19 @@ __device__ __forceinline__ void ht_body(const double* __restrict__ BQ, const int
     using As = std::false_type;
     if (J <= I0) {
         load(Tr{}, J, tp, 0, a0, c0);
-        Jn = seek(J + 1, tn);
+        __builtin_amdgcn_sched_barrier(0);
+        Jn = seek(tn);
         while (Jn <= I0) {
             tile(Tr{}, Tr{});
-            Jn = seek(J + 1, tn);
+            Jn = seek(tn);
         }
         tile(Tr{}, As{});
     } else if (J < nT) {
         load(As{}, J, tp, 0, a0, c0);
+        __builtin_amdgcn_sched_barrier(0);
     }
     while (J < nT) {
-        Jn = seek(J + 1, tn);
+        Jn = seek(tn);
         tile(As{}, As{});
     }
     // X in fragment order, and the wave's share of d_q per column block
@@ -879,17 +848,6 @@ void launch_dpart_reduce(const double* dpart, int nq, int nrg, int ncb, const DR
 
 int kc_block_rows(int nT) { return (nT + 1) / 2; }
 
-// Splits of `steps` steps when a split is nw waves.  A wave's partial sums (32 KB written and read
-// again) cost about as much as 10 steps, and the waves of a launch end unevenly, which costs about half a
-// round of the chip's 2048 wave slots: 10 ns / steps + 1024 / (ns nw) is least at ns = sqrt(102 steps / nw)
-// (nbf 576 / 120 columns / 2784 Q: 307; measured 2.43, 2.23, 2.17, 2.19 ms with 96, 144, 288, 384).
-// Where the launch streams more X than the L2s hold, about 320 steps a split keep a split's waves
-// within 8 Q of one another (see k_kc_f64).  At least 4 steps; multiples of 8, one split per XCD.
-static int balanced_splits(long long nw, int steps, int max_splits) {
-    long long ns = std::max<long long>(steps / 320, std::llround(std::sqrt(102.0 * steps / nw)));
-    ns = std::max<long long>(1, std::min<long long>({ns, steps / 4, max_splits}));
-    return static_cast<int>(ns >= 8 ? ns / 8 * 8 : ns);
-}
 int kc_choose_splits(int nT, bool upper, int steps, int nseg, int max_splits) {
     return balanced_splits(static_cast<long long>(kc_blocks(nT, upper)) * nseg, steps, max_splits);
 }

@@ -1,15 +1,10 @@
-// K-path kernels for gfx950: half-transform X_Q = B_Q C and the contraction
-// K = sum_Q X_Q S X_Q^T (S = diag of column signs, or a second operand X'),
-// in FP64, FP32 and 3-term BF16 split precision.
+// BF16x3 K-path kernels for gfx950: half-transform X_Q = B_Q C and the contraction
+// K = sum_Q X_Q S X_Q^T (S = diag of column signs, or a second operand X') in 3-term BF16 split
+// precision, staged through LDS, and the conversions and column tests of the mixed modes.
 //
-// All kernels are software pipelined: the next K-step's global loads are
-// issued into registers before the current step's MFMAs, then written to the
-// other half of a double-buffered LDS stage, with one barrier per step.
-//
-// MFMA lane layouts (checked on the device):
-//   f64 16x16x4 : A[i][k] lane i+16k; B[k][j] lane j+16k; D[i][j] lane j+16(i%4), reg i/4
-//   f32 16x16x4 : A, B as above;                          D[i][j] lane j+16(i/4), reg i%4
-//   bf16 16x16x32: A[i][8g+e] lane i+16g elem e; B[8g+e][j] lane j+16g elem e; D as f32
+// MFMA lane layout (checked on the device):
+//   bf16 16x16x32: A[i][8g+e] lane i+16g elem e; B[8g+e][j] lane j+16g elem e;
+//   D[i][j] lane j+16(i/4), reg i%4
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -28,26 +23,6 @@ __device__ inline uint16_t f2bf(float x) {
     return static_cast<uint16_t>(u >> 16);
 }
 __device__ inline float bf2f(uint16_t h) { return __uint_as_float(static_cast<uint32_t>(h) << 16); }
-
-// Element e of a 128 x KS chunk of A: row tile e / (32*KS), then (r, c) in the stored
-// tile's own orientation so that global reads are contiguous for both orientations.
-struct ACoord {
-    int sub, r, c;
-};
-template <int KS>
-__device__ inline ACoord a_coord(int e, int I0, int J) {
-    ACoord a;
-    a.sub = e / (32 * KS);
-    const int f = e % (32 * KS);
-    if (I0 + a.sub <= J) {
-        a.r = f / KS;
-        a.c = f % KS;
-    } else {
-        a.c = f / 32;
-        a.r = f % 32;
-    }
-    return a;
-}
 
 // Workgroups are dispatched round-robin over the XCDs (flat id w runs on XCD w % 8,
 // each XCD with its own L2).  xcd_map turns the flat id into (group, item) so that
@@ -122,190 +97,6 @@ __device__ inline void build_steps(StepList<RT>& sl, const int* __restrict__ tid
         if (tid == kMaxColTiles - 1) sl.n = sl.cnt[tid];
     }
     __syncthreads();
-}
-
-// =====================================================================================
-// Half-transform, FP64 / FP32 (16x16x4 MFMA).  WM*256 threads = WM*4 waves (WM rows x
-// 4 cols), workgroup tile 64*WM rows x 64*NBW columns, wave tile 64 x 16*NBW.
-// K-step 8 (FP64) or 16 (FP32).  Absent tiles read a device zero tile (no branches).
-// T = double or float; B is the FP64 tensor (T=double) or its FP32 copy (T=float).
-// grid = (xrows / (64*WM), nq, npanel)
-// =====================================================================================
-template <typename T, int NBW, int WM>
-__global__ __launch_bounds__(WM * 256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ht_mfma(const T* __restrict__ B, const int* __restrict__ tidx, int nT,
-                                                      int ntp, int q0, int nq, int npanel, const T* __restrict__ C,
-                                                      int ldc, T* __restrict__ X, int xrows,
-                                                      const T* __restrict__ ztile) {
-    constexpr bool F64 = sizeof(T) == 8;
-    constexpr int NTHR = WM * 256;
-    constexpr int RT = 2 * WM;            // row tiles per workgroup
-    constexpr int ROWS = 64 * WM;
-    constexpr int PAN = 64 * NBW;
-    constexpr int KS = F64 ? (WM == 1 ? 4 : 8) : 16;
-    constexpr int AP = KS + 1;
-    constexpr int CP = PAN + 4;
-    constexpr int NA = ROWS * KS / NTHR;  // A elements per thread per step
-    constexpr int NC = KS * PAN / NTHR;   // C elements per thread per step
-    static_assert((ROWS * KS) % NTHR == 0 && (KS * PAN) % NTHR == 0, "staging shape");
-    __shared__ T As[2][ROWS * AP];
-    __shared__ T Cs[2][KS * CP];
-    __shared__ StepList<RT> sl;
-    typedef typename std::conditional<F64, d4_t, f4_t>::type acc_t;
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 2, wn = wave & 3;
-    const int nrb = xrows / ROWS;
-    const XcdItem xi = xcd_map(blockIdx.x, nrb * npanel, nq);
-    if (!xi.valid) return;
-    const int rb = xi.item / npanel;
-    const int I0 = RT * rb;
-    const int q = xi.group;
-    const int col0 = (xi.item % npanel) * PAN;
-    const T* BQ = B + static_cast<size_t>(q0 + q) * ntp * TILE2;
-
-    build_steps<RT>(sl, tidx, nT, I0, tid, NTHR);
-    const int nsteps = sl.n * (TILE / KS);
-
-    acc_t acc[4][NBW];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-
-    T ra[NA], rc[NC];
-    // Column tile of the next step to load, read from the LDS step list one step
-    // ahead, so a step's loads wait on one LDS lookup (the block offsets) instead of two.
-    // The FP64 5-column-block shape looks the tile up in place (measured faster there).
-    constexpr bool PF = !(F64 && NBW == 5);
-    int nJ = 0;
-    auto fetch = [&](int st) {
-        if constexpr (PF) nJ = sl.J[st / (TILE / KS)];
-    };
-    int lJ = 0;  // column tile of the step held in ra/rc
-    auto gload = [&](int st) {
-        int J;
-        if constexpr (PF)
-            J = nJ;
-        else
-            J = sl.J[st / (TILE / KS)];
-        lJ = J;
-        const int kh = (st % (TILE / KS)) * KS;
-#pragma unroll
-        for (int it = 0; it < NA; ++it) {
-            const ACoord ac = a_coord<KS>(tid + NTHR * it, I0, J);
-            const int off = sl.off[J * RT + ac.sub];
-            const T* tp = off >= 0 ? BQ + off : ztile;
-            // B is streamed (non-temporal) so that the C panel every workgroup re-reads stays in L2
-            ra[it] = __builtin_nontemporal_load((I0 + ac.sub <= J) ? tp + ac.r * TILE + kh + ac.c
-                                                                   : tp + (kh + ac.c) * TILE + ac.r);
-        }
-        const T* Cj = C + static_cast<size_t>(J * TILE + kh) * ldc + col0;
-#pragma unroll
-        for (int it = 0; it < NC; ++it) {
-            const int e = tid + NTHR * it;
-            const int kk = e / PAN, cc = e - kk * PAN;
-            rc[it] = Cj[static_cast<size_t>(kk) * ldc + cc];
-        }
-        if (st + 1 < nsteps) fetch(st + 1);
-    };
-    auto lstore = [&](int buf, int st) {
-        int J;
-        if constexpr (PF)
-            J = lJ;
-        else
-            J = sl.J[st / (TILE / KS)];
-#pragma unroll
-        for (int it = 0; it < NA; ++it) {
-            const ACoord ac = a_coord<KS>(tid + NTHR * it, I0, J);
-            As[buf][(ac.sub * 32 + ac.r) * AP + ac.c] = ra[it];
-        }
-#pragma unroll
-        for (int it = 0; it < NC; ++it) {
-            const int e = tid + NTHR * it;
-            const int kk = e / PAN, cc = e - kk * PAN;
-            Cs[buf][kk * CP + cc] = rc[it];
-        }
-    };
-    // One step's products: per 4-k sub-step the A fragments of the next sub-step and the C
-    // fragment of the next column block are read while the current block's MFMAs run, so
-    // the LDS reads overlap the MFMAs (consecutive updates of one accumulator are 4*NBW
-    // MFMAs apart).
-    // The last row block can reach past the last row tile: a wave's 16-row fragments there
-    // keep zero accumulators, and their A reads and MFMAs are skipped (NI = fragments kept).
-    constexpr int NSUB = KS / 4;
-    const int nfr = __builtin_amdgcn_readfirstlane(min(4, max(0, 2 * (nT - I0 - 2 * wm))));
-    auto compute = [&](int buf, auto ni) {
-        constexpr int NI = decltype(ni)::value;
-        T a[2][4], b[2];
-        auto aread = [&](int u, int slot) {
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-                a[slot][i] = As[buf][(wm * 64 + i * 16 + (lane & 15)) * AP + 4 * u + (lane >> 4)];
-        };
-        auto bread = [&](int u, int j, int slot) {
-            b[slot] = Cs[buf][(4 * u + (lane >> 4)) * CP + wn * NBW * 16 + j * 16 + (lane & 15)];
-        };
-        aread(0, 0);
-        bread(0, 0, 0);
-#pragma unroll
-        for (int u = 0; u < NSUB; ++u) {
-#pragma unroll
-            for (int j = 0; j < NBW; ++j) {
-                const int t = u * NBW + j;  // running block index: C fragment slot t & 1
-                if (j + 1 < NBW)
-                    bread(u, j + 1, (t + 1) & 1);
-                else if (u + 1 < NSUB)
-                    bread(u + 1, 0, (t + 1) & 1);
-                if (j == 0 && u + 1 < NSUB) aread(u + 1, (u + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < NI; ++i) {
-                    if constexpr (F64)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u & 1][i], b[t & 1], acc[i][j], 0, 0, 0);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u & 1][i], b[t & 1], acc[i][j], 0, 0, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    };
-
-    auto mainloop = [&](auto ni) {
-        fetch(0);
-        gload(0);
-        lstore(0, 0);
-        __syncthreads();
-        int buf = 0;
-        for (int st = 0; st < nsteps; ++st) {
-            const bool more = st + 1 < nsteps;
-            if (more) gload(st + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (decltype(ni)::value > 0) compute(buf, ni);
-            if (more) lstore(buf ^ 1, st + 1);
-            __syncthreads();
-            buf ^= 1;
-        }
-    };
-    if (nsteps > 0) {
-        if (nfr == 4)
-            mainloop(std::integral_constant<int, 4>{});
-        else if (nfr == 2)
-            mainloop(std::integral_constant<int, 2>{});
-        else
-            mainloop(std::integral_constant<int, 0>{});
-    }
-    // every row of the workgroup's block is written (absent row tiles give zeros)
-    T* Xq = X + static_cast<size_t>(q) * xrows * ldc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NBW; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = F64 ? (4 * r + (lane >> 4)) : (4 * (lane >> 4) + r);
-                const int m = ROWS * rb + wm * 64 + i * 16 + rr;
-                Xq[static_cast<size_t>(m) * ldc + col0 + wn * NBW * 16 + j * 16 + (lane & 15)] = acc[i][j][r];
-            }
 }
 
 // BF16 LDS tiles of 32 k per row (64 bytes): the four 16-byte chunks of row r are stored at
@@ -806,188 +597,6 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // =====================================================================================
-// K contraction, FP64 / FP32 (16x16x4 MFMA): P[split][tile] (+)= sum_b A_b S B_b^T over
-// 128x128 output tiles, 4 waves (2x2) of 64x64, K-step 16, double-buffered LDS.
-// S = diag(sign) if sign != nullptr.  Accumulators are stored to FP64 partials.
-// FP32: the MFMA accumulators hold at most kFold32 k-terms before they are added into FP64
-// totals, so the rounding error of a sum does not grow with the number of auxiliary
-// functions a split covers.
-// =====================================================================================
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_kgemm_mfma(const T* __restrict__ A, size_t strideA, const T* __restrict__ Bm,
-                                                    size_t strideB, int ld, int kbeg, int kend, int nbatch,
-                                                    int nsplit, const int2* __restrict__ tiles, int ntile,
-                                                    double* __restrict__ P, double alpha, int accumulate,
-                                                    int upper, int nvalid) {
-    constexpr int KS = 16, AP = KS + 1;
-    constexpr bool F64 = sizeof(T) == 8;
-    typedef typename std::conditional<F64, d4_t, f4_t>::type acc_t;
-    __shared__ T As[2][128 * AP];
-    __shared__ T Bs[2][128 * AP];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
-    const XcdItem xi = xcd_map(blockIdx.x, ntile, nsplit);
-    if (!xi.valid) return;
-    const int tile = xi.item, split = xi.group;
-    const int2 tb = tiles[tile];
-    // a wave does the staging but no MFMAs when its 64x64 block lies below the diagonal of a
-    // diagonal tile of a symmetric result (only the upper triangle is read) or entirely in the
-    // zero padding rows / columns of X past nvalid
-    const bool idle = (upper && tb.x == tb.y && wr > wc) || tb.x * 128 + wr * 64 >= nvalid ||
-                      tb.y * 128 + wc * 64 >= nvalid;
-    const int b0 = static_cast<int>((static_cast<long long>(nbatch) * split) / nsplit);
-    const int b1 = static_cast<int>((static_cast<long long>(nbatch) * (split + 1)) / nsplit);
-    const int nks = (kend - kbeg) / KS;
-    const int nsteps = (b1 - b0) * nks;
-    // thread's fixed (row, k) slots within a 128 x 16 chunk: rows r0 + 16*it, k = tid & 15
-    const int r0 = tid >> 4, kk = tid & 15;
-    const T* Ab = A + static_cast<size_t>(tb.x * 128 + r0) * ld + kbeg + kk;
-    const T* Bb = Bm + static_cast<size_t>(tb.y * 128 + r0) * ld + kbeg + kk;
-
-    acc_t acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = acc_t{0, 0, 0, 0};
-    // FP64 totals of the folded FP32 accumulators (unused for FP64)
-    constexpr int FOLD = F64 ? 0 : kFold32 / KS;
-    d4_t tot[F64 ? 1 : 16];
-#pragma unroll
-    for (int i = 0; i < (F64 ? 1 : 16); ++i) tot[i] = d4_t{0, 0, 0, 0};
-    auto fold = [&]() {
-        if constexpr (!F64) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) tot[i][r] += static_cast<double>(acc[i][r]);
-                acc[i] = acc_t{0, 0, 0, 0};
-            }
-        }
-    };
-
-    T ra[8], rb[8];
-    int b = b0, ks0 = 0;
-    auto gload = [&]() {
-        const size_t oa = static_cast<size_t>(b) * strideA + ks0;
-        const size_t ob = static_cast<size_t>(b) * strideB + ks0;
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            ra[it] = Ab[oa + static_cast<size_t>(16 * it) * ld];
-            rb[it] = Bb[ob + static_cast<size_t>(16 * it) * ld];
-        }
-        ks0 += KS;
-        if (ks0 == nks * KS) {
-            ks0 = 0;
-            ++b;
-        }
-    };
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            As[buf][(r0 + 16 * it) * AP + kk] = ra[it];
-            Bs[buf][(r0 + 16 * it) * AP + kk] = rb[it];
-        }
-    };
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ks += 4) {
-            T a[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[buf][(wr * 64 + i * 16 + (lane & 15)) * AP + ks + (lane >> 4)];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = Bs[buf][(wc * 64 + j * 16 + (lane & 15)) * AP + ks + (lane >> 4)];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if constexpr (F64)
-                        acc[i * 4 + j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i * 4 + j], 0, 0, 0);
-                    else
-                        acc[i * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], bv[j], acc[i * 4 + j], 0, 0, 0);
-                }
-        }
-    };
-
-    if constexpr (F64) {
-        // FP64: a step's operands are loaded two steps before their LDS store (two register
-        // sets named statically in a loop over step pairs; loads past the last step re-read it)
-        T sa0[8], sb0[8], sa1[8], sb1[8];
-        auto gload_at = [&](int st, T* xa, T* xb) {
-            st = min(st, nsteps - 1);
-            const size_t oa = static_cast<size_t>(b0 + st / nks) * strideA + (st % nks) * KS;
-            const size_t ob = static_cast<size_t>(b0 + st / nks) * strideB + (st % nks) * KS;
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                xa[it] = Ab[oa + static_cast<size_t>(16 * it) * ld];
-                xb[it] = Bb[ob + static_cast<size_t>(16 * it) * ld];
-            }
-        };
-        auto lstore_from = [&](int buf, const T* xa, const T* xb) {
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                As[buf][(r0 + 16 * it) * AP + kk] = xa[it];
-                Bs[buf][(r0 + 16 * it) * AP + kk] = xb[it];
-            }
-        };
-        if (nsteps > 0) {
-            gload_at(0, sa0, sb0);
-            gload_at(1, sa1, sb1);
-            lstore_from(0, sa0, sb0);
-            __syncthreads();
-            int st = 0;
-            for (; st + 1 < nsteps; st += 2) {
-                gload_at(st + 2, sa0, sb0);
-                __builtin_amdgcn_sched_barrier(0);
-                if (!idle) compute(0);
-                lstore_from(1, sa1, sb1);
-                __syncthreads();
-                gload_at(st + 3, sa1, sb1);
-                __builtin_amdgcn_sched_barrier(0);
-                if (!idle) compute(1);
-                lstore_from(0, sa0, sb0);
-                __syncthreads();
-            }
-            if (st < nsteps && !idle) compute(0);  // odd step count: the last step is in buffer 0
-        }
-    } else if (nsteps > 0) {
-        gload();
-        lstore(0);
-        __syncthreads();
-        int buf = 0, nf = 0;
-        for (int s = 0; s < nsteps; ++s) {
-            const bool more = s + 1 < nsteps;
-            if (more) gload();
-            if (!idle) {
-                compute(buf);
-                if (++nf == FOLD) {
-                    fold();
-                    nf = 0;
-                }
-            }
-            if (more) lstore(buf ^ 1);
-            __syncthreads();
-            buf ^= 1;
-        }
-    }
-    if (idle) return;
-    fold();
-    double* Pt = P + (static_cast<size_t>(split) * ntile + tile) * 16384;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = F64 ? (4 * r + (lane >> 4)) : (4 * (lane >> 4) + r);
-                const int row = wr * 64 + i * 16 + rr;
-                const int col = wc * 64 + j * 16 + (lane & 15);
-                double* o = Pt + row * 128 + col;
-                double v;
-                if constexpr (F64) v = acc[i * 4 + j][r];
-                else v = tot[i * 4 + j][r];
-                *o = alpha * v + (accumulate ? *o : 0.0);
-            }
-}
-
-// =====================================================================================
 // K contraction, 3-term BF16 split on hi/lo X: A S B^T ~ Ah Bh + Ah Bl + Al Bh.
 // 128x128 tiles, 4 waves of 64x64, K-step 32, double-buffered LDS.  LDS rows are
 // 64 bytes (32 k) with the four 16-byte chunks of row r stored at chunk c ^ ((r>>1)&3):
@@ -1194,17 +803,6 @@ __global__ void k_to_f32_t(const double* __restrict__ src, float* __restrict__ d
     }
 }
 
-// C [nbf][ld] FP64 -> padded [nbfp][ldc] in T, column c taken from source column cmap[c] (< 0: zero)
-template <typename T>
-__global__ void k_pack_cmap(const double* __restrict__ src, int ldsrc, int nbf, const int* __restrict__ cmap,
-                            T* __restrict__ dst, int nbfp, int ldc) {
-    const size_t idx = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= static_cast<size_t>(nbfp) * ldc) return;
-    const int m = static_cast<int>(idx / ldc), c = static_cast<int>(idx % ldc);
-    const int i = cmap[c];
-    dst[idx] = (m < nbf && i >= 0) ? static_cast<T>(src[static_cast<size_t>(m) * ldsrc + i]) : T(0);
-}
-
 // C [nbf][ld] FP64 -> transposed padded [ldc][nbfp] BF16 hi/lo, with the column map
 __global__ void k_pack_cT_bf(const double* __restrict__ src, int ldsrc, int nbf, const int* __restrict__ cmap,
                              uint16_t* __restrict__ hi, uint16_t* __restrict__ lo, int nbfp, int ldc) {
@@ -1260,45 +858,7 @@ void ht_panel_shape(int ncol, int* nbw, int* npanel, int* ldc) {
     *ldc = np * 64 * w;
 }
 
-template <typename T, int NBW, int WM>
-static void ht_mfma_nbw(const TileGeom& g, const T* B, int q0, int nq, const T* C, int ldc, int npanel, T* X,
-                        int xrows, const void* ztile, hipStream_t s) {
-    dim3 grid(xcd_grid(nq, xrows / (64 * WM) * npanel));
-    hipLaunchKernelGGL((k_ht_mfma<T, NBW, WM>), grid, dim3(WM * 256), 0, s, B, g.d_tidx, g.nT, g.ntp, q0, nq, npanel, C,
-                       ldc, X, xrows, static_cast<const T*>(ztile));
-}
-
-template <typename T, int WM>
-static void ht_mfma_wm(const TileGeom& g, const T* B, int q0, int nq, const T* C, int ldc, int nbw, int npanel, T* X,
-                       int xrows, const void* zt, hipStream_t s) {
-    switch (nbw) {
-        case 1: ht_mfma_nbw<T, 1, WM>(g, B, q0, nq, C, ldc, npanel, X, xrows, zt, s); break;
-        case 2: ht_mfma_nbw<T, 2, WM>(g, B, q0, nq, C, ldc, npanel, X, xrows, zt, s); break;
-        case 3: ht_mfma_nbw<T, 3, WM>(g, B, q0, nq, C, ldc, npanel, X, xrows, zt, s); break;
-        case 4: ht_mfma_nbw<T, 4, WM>(g, B, q0, nq, C, ldc, npanel, X, xrows, zt, s); break;
-        default: ht_mfma_nbw<T, 5, WM>(g, B, q0, nq, C, ldc, npanel, X, xrows, zt, s); break;
-    }
-}
-
-int g_ht_wm = 0;       // 0: default shape; 1, 2 (and 4 for BF16x3) select others (tuning sweeps)
-
-template <typename T>
-static void ht_mfma(const TileGeom& g, const T* B, int q0, int nq, const T* C, int ldc, int nbw, int npanel, T* X,
-                    int xrows, const void* zt, hipStream_t s) {
-    require(nbw >= 1 && nbw <= 5 && ldc == npanel * 64 * nbw && nq > 0 && nq <= 65535 &&
-                xrows == (g.nT + 3) / 4 * 128 && g.nT <= kMaxColTiles && zt != nullptr,
-            "ht_mfma shape");
-    const int wm = g_ht_wm ? g_ht_wm : 2;
-    if (wm == 1)
-        ht_mfma_wm<T, 1>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
-    else
-        ht_mfma_wm<T, 2>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
-}
-
-void launch_ht2_f32(const TileGeom& g, const float* B, int q0, int nq, const float* C, int ldc, int nbw, int npanel,
-                    float* X, int xrows, const void* zt, hipStream_t s) {
-    ht_mfma<float>(g, B, q0, nq, C, ldc, nbw, npanel, X, xrows, zt, s);
-}
+int g_ht_wm = 0;       // 0: default shape; 1, 3, 4 select others (tuning sweeps)
 void set_ht_rowwaves(int wm) { g_ht_wm = (wm >= 1 && wm <= 4) ? wm : 0; }
 int g_kgemm_dc = 1;    // BF16x3 contraction: operands loaded straight into LDS (1) or staged (0)
 void set_kgemm_direct(int on) { g_kgemm_dc = on ? 1 : 0; }
@@ -1348,14 +908,6 @@ static void kgemm_check(int xrows, int ld, int kbeg, int kend, int nbatch, int n
             "kgemm shape");
 }
 
-void launch_kgemm2_f32(const float* A, const float* B, size_t stride, int xrows, int nvalid, int ld, int kbeg, int kend,
-                       int nbatch, int nsplit, const int2* tiles, int ntile, double* P, double alpha, int accumulate,
-                       int upper, hipStream_t s) {
-    kgemm_check(xrows, ld, kbeg, kend, nbatch, nsplit, ntile, 16);
-    require(nvalid > 0 && nvalid <= xrows, "kgemm valid rows");
-    hipLaunchKernelGGL((k_kgemm_mfma<float>), dim3(xcd_grid(nsplit, ntile)), dim3(256), 0, s, A, stride, B, stride, ld,
-                       kbeg, kend, nbatch, nsplit, tiles, ntile, P, alpha, accumulate, upper, nvalid);
-}
 void launch_kgemm_bf3(const uint16_t* Ah, const uint16_t* Al, const uint16_t* Bh, const uint16_t* Bl, size_t stride,
                       int xrows, int nvalid, int ld, int kbeg, int kend, int nbatch, int nsplit, const int2* tiles,
                       int ntile, double* P, double alpha, int accumulate, int upper, hipStream_t s) {
@@ -1371,12 +923,6 @@ void launch_to_f32(const double* src, float* dst, size_t n, hipStream_t s) {
 void launch_to_f32_t(const double* src, float* dst, size_t n, hipStream_t s) {
     require(n % TILE2 == 0, "to_f32_t");
     hipLaunchKernelGGL(k_to_f32_t, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
-}
-void launch_pack_cmap_f32(const double* src, int ldsrc, int nbf, const int* cmap, float* dst, int nbfp, int ldc,
-                          hipStream_t s) {
-    const size_t n = static_cast<size_t>(nbfp) * ldc;
-    hipLaunchKernelGGL((k_pack_cmap<float>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, src, ldsrc,
-                       nbf, cmap, dst, nbfp, ldc);
 }
 void launch_pack_cT_bf(const double* src, int ldsrc, int nbf, const int* cmap, uint16_t* hi, uint16_t* lo, int nbfp,
                        int ldc, hipStream_t s) {
