@@ -226,7 +226,7 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc);
 int dfjk_finalize(dfjk_handle* h);
 
 /* Device memory that handles freed (dfjk_finalize, dfjk_destroy, a buffer that grew) is kept for the next
- * allocations of this library, 4 GiB at most over all handles and devices; it is given back when an
+ * allocations of this library, 12 GiB at most over all handles and devices; it is given back when an
  * allocation fails and by this call. */
 int dfjk_trim_memory(void);
 

@@ -100,8 +100,10 @@ void copy2d_settled(void* dst, size_t dpitch, const void* src, size_t spitch, si
 // (H2O)16 allocates 3.4 GB, which took 105 of its 121 ms in such a process.  A block enters the pool
 // when the device is idle, as hipFree would leave it, so any stream and thread may take it.  Blocks
 // are given back oldest first when the bound is reached, all of them when an allocation fails, and by
-// dfjk_trim_memory; free-memory decisions count them as free.
-constexpr size_t kPoolBytes = size_t(4) << 30;
+// dfjk_trim_memory; free-memory decisions count them as free.  The bound takes the whole workspace of a
+// build (8 GiB of X and its partial sums), so that a new handle's first build waits for no cleared
+// pages: with 4 GiB, nbf 1500 / naux 6000 after other handles took 1.55 s instead of 0.2.
+constexpr size_t kPoolBytes = size_t(12) << 30;
 class DevPool {
    public:
     // a block of at least need bytes on device dev (its size in *got), or nullptr
