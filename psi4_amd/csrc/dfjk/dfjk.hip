@@ -2089,8 +2089,8 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
             for (size_t ip = 0; !f32 && ip < passes.size(); ++ip) {
                 const Pass& pp = passes[ip];
                 const int acc = (blk > 0 || ip > 0) ? 1 : 0;
-                uint16_t* xl = reinterpret_cast<uint16_t*>(XL) + pp.offl;
-                uint16_t* xr = reinterpret_cast<uint16_t*>(XR) + pp.offr;
+                uint16_t* xl = reinterpret_cast<uint16_t*>(XL) + pp.offl * 16;
+                uint16_t* xr = reinterpret_cast<uint16_t*>(XR) + pp.offr * 16;
                 launch_kgemm_bf3(xl, xl + xq * qblk, xr, xr + xq * qblk, xq, xrows, nbf, ldc, pp.kbeg, pp.kend, nq, nsp,
                                  otiles, ntile, P, pp.alpha, acc, upper ? 1 : 0, s);
                 h->n_kgemm += 1;

@@ -109,6 +109,7 @@ __device__ inline int kg_swz(int row, int chunk) { return row * 32 + ((chunk ^ (
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 typedef float f2v_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2v_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf4v_t __attribute__((ext_vector_type(4)));
 typedef unsigned int v4u_t __attribute__((ext_vector_type(4)));
 __device__ inline void split_bf16x8(const v4f_t& x, const v4f_t& y, v4u_t& h, v4u_t& l) {
     auto hi = [](float a, float b) { return __builtin_convertvector(f2v_t{a, b}, bf2v_t); };
@@ -367,11 +368,11 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
                 if (j + 1 < NBW) cread(j + 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j & 1], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j & 1], ah[i], acc[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j & 1], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[j & 1], ah[i], acc[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j & 1], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j & 1], al[i], acc[i][j], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             if (j == 0) {
                 pre();
@@ -485,15 +486,15 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
             for (int j = 0; j < NBW; ++j)
 #pragma unroll
-                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j], ah[i], acc[i][j], 0, 0, 0);
 #pragma unroll
             for (int j = 0; j < NBW; ++j)
 #pragma unroll
-                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[j], ah[i], acc[i][j], 0, 0, 0);
 #pragma unroll
             for (int j = 0; j < NBW; ++j)
 #pragma unroll
-                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < NI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[j], al[i], acc[i][j], 0, 0, 0);
             set_priority<0>();
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -580,28 +581,32 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
         else
             go(std::integral_constant<int, 0>{});
     }
+    // X in fragment order (ht_bf3 above): the MFMAs formed C^T B_Q, so a lane holds row lane % 16 and four
+    // consecutive columns of X, 8 bytes of a 1 KB block
     const size_t xq = static_cast<size_t>(q) * xrows * ldc;
+    const int nk32 = ldc / 32, xlane = ((lane >> 5) * 16 + (lane & 15)) * 8 + 4 * ((lane >> 4) & 1);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < NBW; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = ROWS * rb + wm * 64 + i * 16 + 4 * (lane >> 4) + r;
-                const size_t o = xq + static_cast<size_t>(m) * ldc + col0 + wn * NBW * 16 + j * 16 + (lane & 15);
-                const float x = acc[i][j][r];
-                const uint16_t hi = f2bf(x);
-                Xh[o] = hi;
-                Xl[o] = f2bf(x - bf2f(hi));
-            }
+        for (int j = 0; j < NBW; ++j) {
+            const int r16 = ROWS / 16 * rb + wm * 4 + i, c16 = col0 / 16 + wn * NBW + j;
+            const size_t o = xq + (static_cast<size_t>(r16) * nk32 + (c16 >> 1)) * 512 + (c16 & 1) * 256 + xlane;
+            const v4f_t x = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            const bf4v_t hi = __builtin_convertvector(x, bf4v_t);
+            *reinterpret_cast<bf4v_t*>(Xh + o) = hi;
+            *reinterpret_cast<bf4v_t*>(Xl + o) = __builtin_convertvector(x - __builtin_convertvector(hi, v4f_t), bf4v_t);
+        }
 }
 
 // =====================================================================================
 // K contraction, 3-term BF16 split on hi/lo X: A S B^T ~ Ah Bh + Ah Bl + Al Bh.
-// 128x128 tiles, 4 waves of 64x64, K-step 32, double-buffered LDS.  LDS rows are
-// 64 bytes (32 k) with the four 16-byte chunks of row r stored at chunk c ^ ((r>>1)&3):
-// the fragment reads (16 rows x one chunk per 16 lanes) and the staging writes are
-// bank-conflict free, and the 64 KB footprint leaves room for two workgroups per CU.
+// 128x128 tiles, 4 waves of 64x64, K-step 32, double-buffered LDS.  X comes in fragment order, 16 rows x 32
+// columns in 1 KB, so a staging load is one contiguous KB (whole cache lines; rows of X of 64 bytes
+// a step took twice the L2 requests), and a fragment is read from LDS as it lies there, free of bank
+// conflicts.  64 KB of LDS leave room for two workgroups per CU.  Naux 1000 / nbf 1500, every block over 304
+// columns: 3.92 ms, 1.16 PFLOP/s, 57 % of the cycles busy at 1.95 GHz (rows of X: 4.58 ms): like the
+// half-transform against the power limit.  Loads two steps ahead (a barrier between the fragment reads and
+// the MFMAs) were no faster: 3.9-4.1 ms.
 // The MFMA accumulators are folded into a second set of FP32 totals every kFold32 k-terms
 // (FP64 totals would not fit beside the fragments in 256 registers): a sum of N terms then
 // rounds like two chains of about sqrt(N) additions instead of one chain of N.
@@ -650,28 +655,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
 
-    // per step: 4 arrays x 128 rows x 32 k = 4 x 512 vectors of 8; 256 threads -> 2 vectors per array
-    // thread's two 8-element vectors per array: rows (tid>>2) and (tid>>2)+64, chunk tid&3
-    const int vrow = tid >> 2, vc = tid & 3, vk8 = 8 * vc;
+    // per step: 4 arrays x 8 blocks of 16 rows x 32 k; a thread's two 16-byte vectors per array lie in
+    // blocks tid / 64 and tid / 64 + 4
+    const int nk32 = ld / 32;
+    auto block = [&](const uint16_t* X, int s, int r16) {
+        return X + static_cast<size_t>(b0 + s / nks) * stride +
+               (static_cast<size_t>(r16) * nk32 + kbeg / 32 + s % nks) * 512 + lane * 8;
+    };
+    const int w = __builtin_amdgcn_readfirstlane(wave);
     uint4 a0h, a0l, b0h, b0l, a1h, a1l, b1h, b1l;
     auto gload = [&](int s) {
-        const int b = b0 + s / nks;
-        const int k0 = kbeg + (s % nks) * KS;
-        const size_t base = static_cast<size_t>(b) * stride + k0 + vk8;
-        const size_t oa0 = base + static_cast<size_t>(m0 + vrow) * ld;
-        const size_t oa1 = oa0 + static_cast<size_t>(64) * ld;
-        const size_t ob0 = base + static_cast<size_t>(n0 + vrow) * ld;
-        const size_t ob1 = ob0 + static_cast<size_t>(64) * ld;
-        a0h = *reinterpret_cast<const uint4*>(Ah_ + oa0);
-        a0l = *reinterpret_cast<const uint4*>(Al_ + oa0);
-        a1h = *reinterpret_cast<const uint4*>(Ah_ + oa1);
-        a1l = *reinterpret_cast<const uint4*>(Al_ + oa1);
-        b0h = *reinterpret_cast<const uint4*>(Bh_ + ob0);
-        b0l = *reinterpret_cast<const uint4*>(Bl_ + ob0);
-        b1h = *reinterpret_cast<const uint4*>(Bh_ + ob1);
-        b1l = *reinterpret_cast<const uint4*>(Bl_ + ob1);
+        auto ld16 = [&](const uint16_t* X, int r16) { return *reinterpret_cast<const uint4*>(block(X, s, r16)); };
+        a0h = ld16(Ah_, m0 / 16 + w);
+        a0l = ld16(Al_, m0 / 16 + w);
+        a1h = ld16(Ah_, m0 / 16 + w + 4);
+        a1l = ld16(Al_, m0 / 16 + w + 4);
+        b0h = ld16(Bh_, n0 / 16 + w);
+        b0l = ld16(Bl_, n0 / 16 + w);
+        b1h = ld16(Bh_, n0 / 16 + w + 4);
+        b1l = ld16(Bl_, n0 / 16 + w + 4);
     };
-    const int o0 = kg_swz(vrow, vc), o1 = kg_swz(vrow + 64, vc);
+    const int o0 = tid * 8, o1 = o0 + 2048;
     auto lstore = [&](int buf) {
         uint16_t* L = lbuf(buf);
         *reinterpret_cast<uint4*>(L + o0) = a0h;
@@ -683,57 +687,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         *reinterpret_cast<uint4*>(L + 2 * SZ + o1) = b1h;
         *reinterpret_cast<uint4*>(L + 3 * SZ + o1) = b1l;
     };
-    // direct loads of step s into buf: the 32 groups of 16 LDS rows (Ah, Al, Bh, Bl x 8) are
-    // dealt to the waves; lane L lands in 16-byte slot L and fetches the logical chunk that
-    // the swizzle of kg_swz places there
+    // direct loads of step s into buf: the 32 blocks (Ah, Al, Bh, Bl x 8) are dealt to the waves
     auto issue = [&](int s, int buf) {
-        const int b = b0 + s / nks;
-        const int k0 = kbeg + (s % nks) * KS;
-        const int w = __builtin_amdgcn_readfirstlane(wave);
-        const int r0 = lane >> 2, pc = lane & 3;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int arr = i >> 1, rg = w + 4 * (i & 1);  // group w + 4 i of the 32
-            const int r = rg * 16 + r0;
-            const uint16_t* base = arr == 0 ? Ah_ : arr == 1 ? Al_ : arr == 2 ? Bh_ : Bl_;
-            const size_t row = static_cast<size_t>((arr < 2 ? m0 : n0) + r);
-            load_lds16(base + static_cast<size_t>(b) * stride + row * ld + k0 + 8 * (pc ^ ((r >> 1) & 3)),
-                       lbuf(buf) + arr * SZ + rg * 512);
+            const int arr = i >> 1, rg = w + 4 * (i & 1);
+            const uint16_t* X = arr == 0 ? Ah_ : arr == 1 ? Al_ : arr == 2 ? Bh_ : Bl_;
+            load_lds16(block(X, s, (arr < 2 ? m0 : n0) / 16 + rg), lbuf(buf) + arr * SZ + rg * 512);
         }
     };
-    const int fc = lane >> 4;
-    auto compute = [&](int buf, auto&& pre) {
-        const uint16_t* L = lbuf(buf);
-        bf8_t ah[4], al[4], bh[4], bl[4];
+    bf8_t ah[4], al[4], bh[4], bl[4];
+    auto read = [&](const uint16_t* L) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int ra = kg_swz(wr * 64 + i * 16 + (lane & 15), fc);
-            const int rb = kg_swz(wc * 64 + i * 16 + (lane & 15), fc);
+            const int ra = (wr * 4 + i) * 512 + lane * 8, rb = (wc * 4 + i) * 512 + lane * 8;
             ah[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + ra));
             al[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + SZ + ra));
             bh[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + 2 * SZ + rb));
             bl[i] = __builtin_bit_cast(bf8_t, *reinterpret_cast<const uint4*>(L + 3 * SZ + rb));
         }
-        if constexpr (DC) {
-            __builtin_amdgcn_sched_barrier(0);
-            pre();
-            __builtin_amdgcn_sched_barrier(0);
+    };
+    int nf = 0;
+    auto mul = [&] {
+        auto term = [&](const bf8_t* a, const bf8_t* b) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[i * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i * 4 + j], 0, 0, 0);
+        };
+        term(ah, bh);
+        term(ah, bl);
+        term(al, bh);
+        if (++nf == kFold32 / KS) {
+            fold();
+            nf = 0;
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[i * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i * 4 + j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[i * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i * 4 + j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[i * 4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i * 4 + j], 0, 0, 0);
     };
 
     if (nsteps > 0) {
@@ -745,24 +734,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             lstore(0);
         }
         __syncthreads();
-        int buf = 0, nf = 0;
-        for (int s = 0; s < nsteps; ++s) {
-            const bool more = s + 1 < nsteps;
-            auto next = [&] {
-                if constexpr (DC)
-                    if (more) issue(s + 1, buf ^ 1);
-            };
+        int buf = 0;
+        for (int st = 0; st < nsteps; ++st) {
+            const bool more = st + 1 < nsteps;
             if constexpr (!DC)
-                if (more) gload(s + 1);
-            if (!idle) {
-                compute(buf, next);
-                if (++nf == kFold32 / KS) {
-                    fold();
-                    nf = 0;
-                }
-            } else {
-                next();
+                if (more) gload(st + 1);
+            if (!idle) read(lbuf(buf));
+            if constexpr (DC) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (more) issue(st + 1, buf ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (!idle) mul();
             if constexpr (DC)
                 wait_vmem<0>();
             else if (more)

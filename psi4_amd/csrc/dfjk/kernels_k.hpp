@@ -19,14 +19,15 @@ void set_ht_rowwaves(int wm);
 void set_kgemm_direct(int on);
 // X[q][m][i] = sum_n B_{q0+q}[m][n] C[n][i] from the FP32 copy of B [naux][ntp][32][32] and its
 // tile-transposed copy BT (split into hi/lo as they are staged) and C^T hi/lo [ldc][nbfp]; X hi/lo
-// [nq][xrows][ldc] with xrows = 128*ceil(nT/4); every row of X is written (rows past nbf are zero).
+// in the contraction's fragment order [nq][xrows/16][ldc/32][lane][8] (row lane % 16, columns
+// 8 (lane / 16)..) with xrows = 128*ceil(nT/4); every row of X is written (rows past nbf are zero).
 // zt: device zero tile of at least TILE*TILE*8 bytes (read for absent blocks).
 void launch_ht_bf3(const TileGeom& g, const float* B, const float* BT, int q0, int nq, const uint16_t* CTh, const uint16_t* CTl,
                    int ldc, int nbw, int npanel, uint16_t* Xh, uint16_t* Xl, int xrows, const void* zt,
                    hipStream_t s);
 
 // P[split][tile] (+)= alpha * sum_b A_b[:, kbeg:kend] B_b[:, kbeg:kend]^T over 128x128 tiles;
-// A_b = A + b*stride, rows of length ld, xrows rows (a multiple of 128).
+// A_b = A + b*stride in fragment order, ld columns (a multiple of 32), xrows rows (of 128).
 // nvalid: rows of X that are not zero padding (nbf); fragments past it are skipped
 void launch_kgemm_bf3(const uint16_t* Ah, const uint16_t* Al, const uint16_t* Bh, const uint16_t* Bl, size_t stride,
                       int xrows, int nvalid, int ld, int kbeg, int kend, int nbatch, int nsplit, const int2* tiles,
