@@ -48,53 +48,51 @@ inline unsigned xcd_grid(int ngroups, int items) {
 
 // Per-workgroup list of the column tiles J that meet at least one of the
 // workgroup's RT row tiles, with the element offset of each (row tile, J) block
-// in B_Q (or -1), built once in LDS at kernel start (parallel presence test and
-// an inclusive scan), so the K loop does no dependent tile-table lookups.
+// in B_Q (or -1), built once in LDS at kernel start (one thread per column tile, positions
+// from ballots: two barriers), so the K loop does no dependent tile-table lookups.
 constexpr int kMaxColTiles = 256;  // nbf <= 8192
 // k-terms an FP32 MFMA accumulator of the K contraction holds before it is folded into FP64
 constexpr int kFold32 = 512;
 
 template <int RT>
 struct StepList {
-    int off[kMaxColTiles * RT];    // by column tile
     int soff[kMaxColTiles * RT];   // by step
     int J[kMaxColTiles];
-    int cnt[kMaxColTiles];
+    int cnt[kMaxColTiles / 64];
     int n;
 };
 
 template <int RT>
-__device__ inline void build_steps(StepList<RT>& sl, const int* __restrict__ tidx, int nT, int I0, int tid, int nthr) {
-    for (int j = tid; j < kMaxColTiles; j += nthr) {
-        int present = 0;
+__device__ inline void build_steps(StepList<RT>& sl, const int* __restrict__ tidx, int nT, int I0, int tid) {
+    const int lane = tid & 63, wv = tid >> 6;
+    int off[RT];
+    bool present = false;
+    unsigned long long mask = 0;
+    if (tid < kMaxColTiles) {  // whole waves
+        const int j = tid;
 #pragma unroll
         for (int s = 0; s < RT; ++s) {
             const int I = I0 + s;
             int t = -1;
             if (j < nT && I < nT) t = tidx[min(I, j) * nT + max(I, j)];
-            sl.off[j * RT + s] = t >= 0 ? t * TILE2 : -1;
-            present |= (t >= 0);
+            off[s] = t >= 0 ? t * TILE2 : -1;
+            present |= t >= 0;
         }
-        sl.cnt[j] = present;
+        mask = __ballot(present);
+        if (lane == 0) sl.cnt[wv] = __popcll(mask);
     }
     __syncthreads();
-    // inclusive scan of the presence flags (Hillis-Steele over kMaxColTiles entries)
-    for (int d = 1; d < kMaxColTiles; d <<= 1) {
-        int v = 0;
-        if (tid < kMaxColTiles && tid >= d) v = sl.cnt[tid - d];
-        __syncthreads();
-        if (tid < kMaxColTiles) sl.cnt[tid] += v;
-        __syncthreads();
-    }
-    // compact: step k -> J and its block offsets
-    if (tid < kMaxColTiles) {
-        const int prev = tid ? sl.cnt[tid - 1] : 0;
-        if (sl.cnt[tid] != prev) {
-            sl.J[prev] = tid;
+    if (present) {
+        int k = __popcll(mask & ((1ull << lane) - 1));
+        for (int i = 0; i < wv; ++i) k += sl.cnt[i];
+        sl.J[k] = tid;
 #pragma unroll
-            for (int s = 0; s < RT; ++s) sl.soff[prev * RT + s] = sl.off[tid * RT + s];
-        }
-        if (tid == kMaxColTiles - 1) sl.n = sl.cnt[tid];
+        for (int s = 0; s < RT; ++s) sl.soff[k * RT + s] = off[s];
+    }
+    if (tid == 0) {
+        int n = 0;
+        for (int i = 0; i < kMaxColTiles / 64; ++i) n += sl.cnt[i];
+        sl.n = n;
     }
     __syncthreads();
 }
@@ -194,7 +192,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
     static_assert((NAV == 1 || NAV == 2) && NAV * NTHR == ROWS * 4, "one or two A vectors per thread");
     static_assert(NCV + (NCV_R ? 1 : 0) <= 5, "C staging slots");
     static_assert(NCV_R % 4 == 0, "whole C rows per partial round");
-    static_assert(NTHR >= kMaxColTiles, "build_steps scans with one thread per column tile");
+    static_assert(NTHR >= kMaxColTiles, "build_steps takes one thread per column tile");
     constexpr int NSLOT = NCV + (NCV_R ? 1 : 0);  // C vector rounds per thread
     // the two stage buffers are separate arrays, so the compiler can tell a direct load into
     // one from the fragment reads of the other and need not wait for it before them
@@ -214,7 +212,7 @@ __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2,
     const int col0 = (xi.item % npanel) * PAN;
     const size_t qoff = static_cast<size_t>(q0 + q) * ntp * TILE2;
 
-    build_steps<RT>(sl, tidx, nT, I0, tid, NTHR);
+    build_steps<RT>(sl, tidx, nT, I0, tid);
     const int nsteps = sl.n;
 
     f4_t acc[4][NBW];
