@@ -448,10 +448,11 @@ __device__ inline int group_start(int g, int ncb, int ng, int NC) {
     return g * NC - max(0, g - (ncb - ng * (NC - 1)));
 }
 
-// Y and Z of one q: blocks [i0, i0 + NI) x [j0, j0 + NJ).  X is gathered 8 bytes per lane in the
-// transposed sense (rows along the sum); each 16 x 16 piece feeds NI MFMA steps, so the gather (32
-// cache cycles) hides under them.
-template <int NI, int NJ>
+// Y and Z of one q: blocks [i0, i0 + NI) x [j0, j0 + NJ) of the symmetric Y, the ones below the diagonal
+// (DIAG: i0 = j0) stored as mirror images.  X is gathered 8 bytes per lane in the transposed sense (rows
+// along the sum); each 16 x 16 piece feeds NI MFMA steps, so the gather (32 cache cycles) hides under
+// them.  1856 Q / nbf 384 / 80 columns: 0.152 ms, 15 of 25 sub-tiles (every sub-tile in four waves: 0.265).
+template <int NI, int NJ, bool DIAG>
 __device__ __forceinline__ void adj_z_body(const double* __restrict__ CB, const double* __restrict__ Xq, int nkb, int ncb,
                                            int i0, int j0, double dq, double* __restrict__ Zq,
                                            double* __restrict__ ep) {
@@ -485,7 +486,7 @@ __device__ __forceinline__ void adj_z_body(const double* __restrict__ CB, const 
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+                    if (!DIAG || i <= j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     load(0, a0, b0);
@@ -495,52 +496,72 @@ __device__ __forceinline__ void adj_z_body(const double* __restrict__ CB, const 
         load(kb + 2, a0, b0);
         mul(a1, b1);
     }
+    // mirror image: element 4 r + lg of a row in lane lj is row lj, element 4 r + lg
+    const unsigned off_m = ((lj >> 3) * ncb * 128 + ((lj & 3) * 16 + lg) * 2 + ((lj >> 2) & 1)) * 8;
     double es = 0.0;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+        for (int j = 0; j < NJ; ++j) {
+            if (DIAG && i > j) continue;
+            double ts = 0.0;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 d2_t z;
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     const double y = acc[i][j][2 * h + e];
-                    const bool diag = 16 * (i0 + i) + 8 * h + 4 * e + lg == 16 * (j0 + j) + lj;
+                    const bool diag = DIAG && i == j && 8 * h + 4 * e + lg == lj;
                     z[e] = (diag ? 2.0 * dq : 0.0) - y;
-                    es = fma(y, z[e], es);
+                    ts = fma(y, z[e], ts);
                 }
                 *reinterpret_cast<d2_t*>(reinterpret_cast<char*>(
                                              Zq + (static_cast<size_t>(2 * (i0 + i) + h) * ncb + j0 + j) * 128) + off_c) = z;
             }
+            if (!DIAG || i < j) {
+                ts *= 2.0;
+                double* zm = Zq + (static_cast<size_t>(2 * (j0 + j)) * ncb + i0 + i) * 128;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    *reinterpret_cast<double*>(reinterpret_cast<char*>(zm + 8 * r) + off_m) = -acc[i][j][r];
+            }
+            es += ts;
+        }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) es += __shfl_xor(es, o);
     if (lane == 0) *ep = es;
 }
 
-constexpr int kZ = 4;  // column blocks per side of a wave's part of Y
 __global__ __launch_bounds__(256, 2) void k_adj_z(const double* __restrict__ CB, const double* __restrict__ X, int nT,
                                                   int ncb, int ng, int nc, int nq, const double* __restrict__ d,
                                                   double* __restrict__ Z, double* __restrict__ epart) {
-    const WaveItem w = wave_item(ng * ng);
+    const int items = ng * (ng + 1) / 2;
+    const WaveItem w = wave_item(items);
     if (w.group >= nq) return;
-    const int q = w.group, gi = w.item / ng, gj = w.item % ng;
+    int gi = 0, gj = w.item;
+    while (gj >= ng - gi) {
+        gj -= ng - gi;
+        ++gi;
+    }
+    gj += gi;
+    const int q = w.group;
     const int i0 = group_start(gi, ncb, ng, nc), j0 = group_start(gj, ncb, ng, nc);
     const int ni = group_start(gi + 1, ncb, ng, nc) - i0, nj = group_start(gj + 1, ncb, ng, nc) - j0;
     const double* Xq = X + static_cast<size_t>(q) * nT * 4 * ncb * 128;
     double* Zq = Z + static_cast<size_t>(q) * 2 * ncb * ncb * 128;
-    double* ep = epart + static_cast<size_t>(q) * ng * ng + w.item;
+    double* ep = epart + static_cast<size_t>(q) * items + w.item;
     const double dq = d[q];
-#define P4A_Z(NI, NJ) \
-    if (ni == NI && nj == NJ) return adj_z_body<NI, NJ>(CB, Xq, 4 * nT, ncb, i0, j0, dq, Zq, ep)
-    P4A_Z(4, 4);
-    P4A_Z(4, 3);
-    P4A_Z(3, 4);
-    P4A_Z(3, 3);
-    P4A_Z(3, 2);
-    P4A_Z(2, 3);
-    P4A_Z(2, 2);
-    P4A_Z(1, 1);
+#define P4A_Z(NI, NJ, DIAG)                        \
+    if (ni == NI && nj == NJ && (gi == gj) == DIAG) \
+    return adj_z_body<NI, NJ, DIAG>(CB, Xq, 4 * nT, ncb, i0, j0, dq, Zq, ep)
+    P4A_Z(5, 5, true);
+    P4A_Z(4, 4, true);
+    P4A_Z(3, 3, true);
+    P4A_Z(2, 2, true);
+    P4A_Z(1, 1, true);
+    P4A_Z(4, 4, false);
+    P4A_Z(4, 3, false);
+    P4A_Z(3, 3, false);
 #undef P4A_Z
 }
 
@@ -632,7 +653,10 @@ __global__ __launch_bounds__(256, 2) void k_adj_p(const double* __restrict__ Z, 
 }
 
 // G_q = 2 P_q C^T, a 64 x 64 block on or above the diagonal, written with its mirror image.  Bound
-// by writing G (8 n^2 bytes per q).
+// by writing G (8 n^2 bytes per q).  The mirror image is turned in registers, so that a lane stores 32
+// consecutive bytes; stores pass the caches by.  Nbf 384 / 1856 Q (2.19 GB) / 80 columns: 0.71 ms, 3.1 TB/s
+// (8-byte mirror stores: 0.84; cached ones 0.74; without the product 0.44; 32 x 64 blocks at twice the
+// occupancy 0.82).
 template <int NI, int NJ, bool DIAG>
 __device__ __forceinline__ void adj_g_body(const double* __restrict__ Pq, const double* __restrict__ CD, int nkx, int nk,
                                            int rb0, int cb0, int n, double* __restrict__ G) {
@@ -655,13 +679,27 @@ __device__ __forceinline__ void adj_g_body(const double* __restrict__ Pq, const 
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             if (DIAG && i > j) continue;
+            const bool diag = DIAG && i == j;
+            const int m0 = 16 * (rb0 + i), c = 16 * (cb0 + j) + lj;
+            double v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int m = 16 * (rb0 + i) + 4 * r + lg, c = 16 * (cb0 + j) + lj;
-                if (m >= n || c >= n || (DIAG && m > c)) continue;
-                const double v = 2.0 * acc[j][i][r];
-                G[static_cast<size_t>(m) * n + c] = v;
-                G[static_cast<size_t>(c) * n + m] = v;
+                const int m = m0 + 4 * r + lg;
+                v[r] = 2.0 * acc[j][i][r];
+                if (m < n && c < n && (!diag || m <= c)) __builtin_nontemporal_store(v[r], G + static_cast<size_t>(m) * n + c);
+            }
+            transpose4(v);
+            const int m = m0 + 4 * lg;
+            double* g = G + static_cast<size_t>(c) * n + m;
+            if (!diag && m + 4 <= n) {
+                if (c < n) {
+                    __builtin_nontemporal_store(d2u_t{v[0], v[1]}, reinterpret_cast<d2u_t*>(g));
+                    __builtin_nontemporal_store(d2u_t{v[2], v[3]}, reinterpret_cast<d2u_t*>(g + 2));
+                }
+            } else if (c < n) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (m + r < n && (!diag || m + r <= c)) g[r] = v[r];
             }
         }
 }
@@ -894,14 +932,15 @@ void launch_pack_rows(const double* C, int ld, int ncol, int nbf, int nbfp, int 
     hipLaunchKernelGGL(k_pack_rows, dim3(std::min(4096, (n + 255) / 256)), dim3(256), 0, s, C, ld, ncol, nbf, n, ncb, CB);
 }
 
-static int z_groups(int ncb) { return (ncb + kZ - 1) / kZ; }
-int adj_z_waves(int ncb) { return z_groups(ncb) * z_groups(ncb); }
+// Up to 5 blocks in one group (the upper 15 of 25 sub-tiles fit the registers), more in groups of 3 or 4
+static int z_groups(int ncb) { return ncb <= 5 ? 1 : (ncb + 3) / 4; }
+int adj_z_waves(int ncb) { return z_groups(ncb) * (z_groups(ncb) + 1) / 2; }
 void launch_adj_z(const double* CB, const double* X, int nT, int ncb, int nq, const double* d, double* Z, double* epart,
                   hipStream_t s) {
     require(nT > 0 && ncb > 0 && nq > 0, "adj_z");
     const int ng = z_groups(ncb), nc = (ncb + ng - 1) / ng;
-    // groups are nc or nc - 1 wide: 1 (one block), 2, 3 or 4, and 2 beside 1 never occurs
-    hipLaunchKernelGGL(k_adj_z, dim3(wave_grid(nq, ng * ng, 4)), dim3(256), 0, s, CB, X, nT, ncb, ng, nc, nq, d, Z, epart);
+    hipLaunchKernelGGL(k_adj_z, dim3(wave_grid(nq, adj_z_waves(ncb), 4)), dim3(256), 0, s, CB, X, nT, ncb, ng, nc, nq, d,
+                       Z, epart);
 }
 
 template <class F>

@@ -24,6 +24,34 @@ __device__ inline double ld1(const double* base, unsigned off) {
 }
 __device__ inline int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
+// v[r] in lane group g (lanes 16 g ..) becomes v[g] in lane group r: after an FP64 MFMA, four consecutive rows
+// of a column in a lane instead of four rows 4 apart.
+__device__ __forceinline__ void transpose4(double* v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef unsigned u2_t __attribute__((ext_vector_type(2)));
+    auto swap = [](double& a, double& b, auto&& f) {
+        u2_t x = __builtin_bit_cast(u2_t, a), y = __builtin_bit_cast(u2_t, b);
+        const u2_t l = f(x[0], y[0]), h = f(x[1], y[1]);
+        a = __builtin_bit_cast(double, u2_t{l[0], h[0]});
+        b = __builtin_bit_cast(double, u2_t{l[1], h[1]});
+    };
+    // lanes 32..63 of the first with lanes 0..31 of the second; odd 16-lane rows with even ones
+    auto s32 = [](unsigned x, unsigned y) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        return u2_t{r[0], r[1]};
+    };
+    auto s16 = [](unsigned x, unsigned y) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        return u2_t{r[0], r[1]};
+    };
+    swap(v[0], v[2], s32);
+    swap(v[1], v[3], s32);
+    swap(v[0], v[1], s16);
+    swap(v[2], v[3], s16);
+#endif
+}
+
 // Workgroups go round-robin to the XCDs (each with its own L2): wave w of the launch belongs to XCD
 // (workgroup % 8); consecutive waves of an XCD take the items of one group (the row and column blocks
 // of one Q, the output blocks of one split), so a group's operands meet in one L2.
@@ -93,9 +121,14 @@ struct TileRow {
 // round of the chip's 2048 wave slots: 10 ns / steps + 1024 / (ns nw) is least at ns = sqrt(102 steps / nw)
 // (nbf 576 / 120 columns / 2784 Q in FP64: 307; measured 2.43, 2.23, 2.17, 2.19 ms with 96, 144, 288, 384).
 // Where the launch streams more X than the L2s hold, about 320 steps a split keep a split's waves
-// within 8 Q of one another (see k_kc_f64).  At least 4 steps; multiples of 8, one split per XCD.
+// within 8 Q of one another (see k_kc_f64).  A launch of between one and three rounds is cut to whole ones (2000
+// k8 steps of 3 x 3 x 3 blocks: 0.19 -> 0.165 ms; the adjoint's dE/dC at nbf 384: 0.206 -> 0.170).  At least 4
+// steps; multiples of 8, one split per XCD.
 inline int balanced_splits(long long nw, int steps, int max_splits) {
+    constexpr double slots = kXCD * kSlots;
     long long ns = std::max<long long>(steps / 320, std::llround(std::sqrt(102.0 * steps / nw)));
+    const double rounds = ns * static_cast<double>(nw) / slots;
+    if (rounds > 1 && rounds < 3) ns = static_cast<long long>(std::floor(rounds) * slots / nw);
     ns = std::max<long long>(1, std::min<long long>({ns, steps / 4, max_splits}));
     return static_cast<int>(ns >= 8 ? ns / 8 * 8 : ns);
 }
