@@ -1439,33 +1439,48 @@ ColGroups one_group(const double* src, int ncol, const double* partner) {
     return cg;
 }
 
-// D = Cl Cr^T (jk.cc:314-354), FP64: the contraction kernel over the columns of the packed C.  Its
-// workspace is that of the build that follows on the stream.
-void compute_D(dfjk_handle* h, const double* dCl, const double* dCr, int ncol, double* D, Work& wk) {
+// D = Cl Cr^T (jk.cc:314-354) of the pairs that want it (at most kMaxPairs), FP64: the contraction
+// kernel over the columns of the packed C, all pairs in one launch (two when symmetric and other pairs
+// meet).  Its workspace is that of the build that follows on the stream.
+void compute_D(dfjk_handle* h, const PairIn* pr, int np, Work& wk) {
     const hipStream_t s = h->stream;
-    const bool sym = dCr == nullptr || dCr == dCl;
-    const int ncb = (ncol + 15) / 16, nk = (ncol + 7) / 8;
-    const size_t csz = static_cast<size_t>(h->nbfp) * 16 * ncb;
-    double* DL = wk.get<double>(h->ws_CA, csz);
-    launch_pack_frag(one_group(dCl, ncol, dCl), h->nbf, h->nbfp, nullptr, DL, s);
-    double* DR = DL;
-    if (!sym) {
-        DR = wk.get<double>(h->ws_CD, csz);
-        launch_pack_frag(one_group(dCr, ncol, dCr), h->nbf, h->nbfp, nullptr, DR, s);
+    ColGroups cg;
+    auto add = [&](const double* src, int ncol) {
+        cg.g[cg.n] = ColGroup{src, src, nullptr, ncol, ncol, cg.ncb, (ncol + 15) / 16};
+        cg.ncb += cg.g[cg.n].ncb;
+        return 2 * cg.g[cg.n++].cb0;
+    };
+    KcSegs segs[2];  // [0]: symmetric, [1]: the others
+    KcOuts outs[2];
+    for (int p = 0; p < np; ++p) {
+        if (!pr[p].D) continue;
+        const int k = pr[p].cr && pr[p].cr != pr[p].cl ? 1 : 0, nk = (pr[p].ncol + 7) / 8;
+        const int ka = add(pr[p].cl, pr[p].ncol), kb = k ? add(pr[p].cr, pr[p].ncol) : ka;
+        outs[k].o[segs[k].n].out = pr[p].D;
+        segs[k].s[segs[k].n++] = KcSeg{0, 0, ka, kb, nk, 1.0};
     }
-    const int nblk = kc_blocks(h->nT, sym);
-    int nsp = kc_choose_splits(h->nT, sym, nk, 1, 64);
-    if (wk.fixed()) nsp = 1;
-    double* P = wk.get<double>(h->ws_P, static_cast<size_t>(nsp) * nblk * 4096);
-    KcSegs sg;
-    sg.n = 1;
-    sg.nsplit = nsp;
-    sg.s[0] = KcSeg{0, nsp, 0, 0, nk, 1.0};
-    launch_kc_f64(DL, DR, 0, 2 * ncb, h->nT, 1, sg, sym, P, 0, s);
-    KcOuts o;
-    o.n = 1;
-    o.o[0] = KcOut{0, nsp, D};
-    launch_kc_reduce(P, h->nT, h->nbf, sym, o, 0, s);
+    if (!cg.n) return;
+    double* C = wk.get<double>(h->ws_CA, static_cast<size_t>(h->nbfp) * 16 * cg.ncb);
+    launch_pack_frag(cg, h->nbf, h->nbfp, nullptr, C, s);
+    size_t psize = 0;
+    for (int k = 0; k < 2; ++k) {
+        for (int i = 0; i < segs[k].n; ++i) {
+            KcSeg& g = segs[k].s[i];
+            g.sp0 = segs[k].nsplit;
+            g.nsp = wk.fixed() ? 1 : kc_choose_splits(h->nT, k == 0, g.nk, segs[k].n, 64);
+            segs[k].nsplit += g.nsp;
+            outs[k].o[outs[k].n].sp0 = g.sp0;
+            outs[k].o[outs[k].n++].nsp = g.nsp;
+        }
+        psize += static_cast<size_t>(segs[k].nsplit) * kc_blocks(h->nT, k == 0) * 4096;
+    }
+    double* P = wk.get<double>(h->ws_P, psize);
+    for (int k = 0; k < 2; ++k) {
+        if (!segs[k].n) continue;
+        launch_kc_f64(C, C, 0, 2 * cg.ncb, h->nT, 1, segs[k], k == 0, P, 0, s);
+        launch_kc_reduce(P, h->nT, h->nbf, k == 0, outs[k], 0, s);
+        P += static_cast<size_t>(segs[k].nsplit) * kc_blocks(h->nT, k == 0) * 4096;
+    }
 }
 
 // Chunks of the second J pass over nq auxiliary functions: about 4096 workgroups, at least four Q each
@@ -1508,14 +1523,13 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     const int q0 = h->aux_q0, q1 = h->aux_q1, nq_total = q1 - q0;
     const int nT = h->nT, nbf = h->nbf, nbfp = h->nbfp;
     EventTimer& tm = h->timer;
-    for (int p = 0; p < np; ++p)
-        if (pr[p].D) {
-            hipEvent_t e0 = tm.begin();
-            const size_t mark = wk.used;
-            compute_D(h, pr[p].cl, pr[p].cr, pr[p].ncol, pr[p].D, wk);
-            wk.used = mark;  // D's operands are dead before the next kernel of this stream
-            tm.end(T_OTHER, e0);
-        }
+    {
+        hipEvent_t e0 = tm.begin();
+        const size_t mark = wk.used;
+        compute_D(h, pr, np, wk);
+        wk.used = mark;  // D's operands are dead before the next kernel of this stream
+        tm.end(T_OTHER, e0);
+    }
     // column groups, contraction passes and output blocks
     ColGroups cg;
     auto add = [&](const double* src, int ld, int ncol, const int* cmap, int ncolp, const double* partner) {
@@ -1754,7 +1768,9 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
         hipEvent_t e0 = tm.begin();
         if (!Dm) Dm = wk.get<double>(h->ws_D, static_cast<size_t>(nbf) * nbf);
         const size_t mark = wk.used;
-        compute_D(h, dCl, dCr, ncol, Dm, wk);
+        PairIn d = in;
+        d.D = Dm;
+        compute_D(h, &d, 1, wk);
         wk.used = mark;  // D's operands are dead before the next kernel of this stream
         tm.end(T_OTHER, e0);
     }
