@@ -14,6 +14,7 @@
 
 #include <algorithm>
 
+#include "j_unpack.hpp"
 #include "kernels.hpp"
 
 namespace p4a {
@@ -174,39 +175,9 @@ __global__ __launch_bounds__(256) void k_j2(BS B, const double* __restrict__ d, 
     }
 }
 
-// J from the partials of every Q chunk.  A workgroup sums 128 elements (4 rows) of one tile, the
-// chunks dealt to 8 groups of threads and added in LDS in a fixed order, and writes each element
-// with its mirror image, so J is exactly symmetric.  Bound by latency at small sizes: one thread
-// per element of J walking every chunk took 145 us at nbf 96 (464 chunks) and 36 us at nbf 576
-// (24 chunks); this takes 9 us and 11 us.  Tiles that are not stored stay at the caller's zeros
-// (or are zeroed by k_j_clear when not accumulating).
-constexpr int kJuGroups = 8;
-__global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(const double* __restrict__ Jpart, size_t pstride,
-                                                             int nchunk, int ntp, const int2* __restrict__ tiles,
-                                                             int nbf, JOut out, int ldJ, double alpha, int accumulate) {
-    __shared__ double red[kJuGroups][128];
-    Jpart += blockIdx.z * pstride;
-    double* __restrict__ J = out.J[blockIdx.z];
-    const int t = blockIdx.x, el = threadIdx.x & 127, grp = threadIdx.x >> 7;
-    const int e = blockIdx.y * 128 + el;
-    double s = 0.0;
-#pragma unroll 4
-    for (int c = grp; c < nchunk; c += kJuGroups) s += Jpart[(static_cast<size_t>(c) * ntp + t) * TILE2 + e];
-    red[grp][el] = s;
-    __syncthreads();
-    if (grp != 0) return;
-    double v = red[0][el];
-#pragma unroll
-    for (int g = 1; g < kJuGroups; ++g) v += red[g][el];
-    const int2 IJ = tiles[t];
-    const int m = IJ.x * TILE + e / TILE, n = IJ.y * TILE + e % TILE;
-    if (m >= nbf || n >= nbf || m > n) return;  // the lower triangle of a diagonal tile is its mirror image
-    double* o = J + static_cast<size_t>(m) * ldJ + n;
-    *o = alpha * v + (accumulate ? *o : 0.0);
-    if (m != n) {
-        double* ot = J + static_cast<size_t>(n) * ldJ + m;
-        *ot = alpha * v + (accumulate ? *ot : 0.0);
-    }
+__global__ __launch_bounds__(128 * kJuGroups) void k_j_unpack(JUnpack u) {
+    __shared__ double red[128 * kJuGroups];
+    j_unpack_block(u, blockIdx.x, blockIdx.y, blockIdx.z, red);
 }
 // J = 0 on the 32 x 32 blocks that have no stored tile
 __global__ void k_j_clear(const int* __restrict__ tidx, int nT, int nbf, JOut out, int ldJ) {
@@ -461,13 +432,17 @@ void launch_j2(const TileGeom& g, const JSource& B, const double* d, int ldd, in
     });
 }
 
-void launch_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np, int ldJ,
-                     double alpha, int accumulate, hipStream_t s) {
+JUnpack prepare_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np,
+                         int ldJ, double alpha, int accumulate, hipStream_t s) {
     require(ldJ >= g.nbf && g.ntp > 0 && nchunk > 0 && np >= 1 && np <= 4, "j_unpack");
     if (!accumulate && g.ntp < g.nT * (g.nT + 1) / 2)
         hipLaunchKernelGGL(k_j_clear, dim3(g.nT, g.nT, np), dim3(256), 0, s, g.d_tidx, g.nT, g.nbf, out, ldJ);
-    hipLaunchKernelGGL(k_j_unpack, dim3(g.ntp, TILE2 / 128, np), dim3(128 * kJuGroups), 0, s, Jpart, pstride, nchunk,
-                       g.ntp, g.d_tiles, g.nbf, out, ldJ, alpha, accumulate);
+    return JUnpack{Jpart, pstride, nchunk, g.ntp, np, g.d_tiles, g.nbf, out, ldJ, alpha, accumulate};
+}
+void launch_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np, int ldJ,
+                     double alpha, int accumulate, hipStream_t s) {
+    const JUnpack u = prepare_j_unpack(g, Jpart, pstride, nchunk, out, np, ldJ, alpha, accumulate, s);
+    hipLaunchKernelGGL(k_j_unpack, dim3(g.ntp, TILE2 / 128, np), dim3(128 * kJuGroups), 0, s, u);
 }
 
 void launch_tile_reduce(const double* P, int nsplit, int ntile, const int* d_tile_of, int nB, int sym, int M, int N,

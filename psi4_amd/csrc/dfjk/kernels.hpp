@@ -40,7 +40,21 @@ void launch_j2(const TileGeom& g, const JSource& B, const double* d, int ldd, in
 struct JOut {
     double* J[4];
 };
-// J_p[m][n] = alpha * sum_c Jpart[p][c][tile(m,n)] (+ J_p if accumulate)
+// J_p[m][n] = alpha * sum_c Jpart[p][c][tile(m,n)] (+ J_p if accumulate): at once, or prepared (the
+// blocks without a stored tile cleared) for a launch that takes it along
+struct JUnpack {
+    const double* Jpart;
+    size_t pstride;
+    int nchunk, ntp, np;
+    const int2* tiles;
+    int nbf;
+    JOut out;
+    int ldJ;
+    double alpha;
+    int accumulate;
+};
+JUnpack prepare_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np,
+                         int ldJ, double alpha, int accumulate, hipStream_t s);
 void launch_j_unpack(const TileGeom& g, const double* Jpart, size_t pstride, int nchunk, const JOut& out, int np, int ldJ,
                      double alpha, int accumulate, hipStream_t s);
 

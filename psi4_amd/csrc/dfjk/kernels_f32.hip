@@ -424,7 +424,7 @@ void launch_kc_f32(const float* X, size_t qstride, int nkx, int nT, int nq, cons
 }
 
 void launch_kc32_reduce(const double* P, int nT, int n, bool upper, const KcOuts& outs, int accumulate, hipStream_t s) {
-    require(outs.n >= 1 && outs.n <= kMaxPairs && n > 0 && n <= nT * TILE, "kc32_reduce");
+    require(outs.n >= 1 && outs.n <= 2 * kMaxPairs && n > 0 && n <= nT * TILE, "kc32_reduce");
     const int nblk = kc32_blocks(nT, upper);
     hipLaunchKernelGGL(k_kc32_reduce, dim3(nblk, 8, outs.n), dim3(256 * kRed32), 0, s, P, nblk, nT, n, upper ? 1 : 0, outs,
                        accumulate);

@@ -21,6 +21,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "j_unpack.hpp"
 #include "kernels_f64.hpp"
 #include "wave_kernels.hpp"
 
@@ -368,12 +369,18 @@ __global__ __launch_bounds__(64, 2) void k_kc_f64(
 }
 
 // Sum over a pair's splits of one 16 x 16 sub-tile, the splits dealt to 4 groups of 256 threads and
-// added in LDS in a fixed order.
+// added in LDS in a fixed order.  J's reduction rides in the same launch (z past the outputs): bound by
+// latency both, the two in a row cost 8 us at nbf 24.
 constexpr int kRedGroups = 4;
 __global__ __launch_bounds__(256 * kRedGroups) void k_kc_reduce(const double* __restrict__ P, int nblk, int nbr, int n,
-                                                               int upper, KcOuts outs, int accumulate) {
+                                                               int upper, KcOuts outs, int accumulate, JUnpack ju) {
     __shared__ double red[kRedGroups][256];
     const int blk = blockIdx.x, st = blockIdx.y;
+    if (static_cast<int>(blockIdx.z) >= outs.n) {
+        const int i = ((blockIdx.z - outs.n) * 16 + st) * nblk + blk, per = ju.ntp * (TILE2 / 128);
+        if (i < per * ju.np) j_unpack_block(ju, i % per % ju.ntp, i % per / ju.ntp, i / per, &red[0][0]);
+        return;
+    }
     const KcOut O = outs.o[blockIdx.z];
     int I = 0, J = 0;
     if (upper) {
@@ -912,10 +919,14 @@ void launch_kc_f64(const double* XA, const double* XB, size_t qstride, int nkx, 
                            accumulate);
 }
 
-void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& outs, int accumulate, hipStream_t s) {
-    require(outs.n >= 1 && outs.n <= kMaxPairs && n > 0 && n <= nT * TILE, "kc_reduce");
-    hipLaunchKernelGGL(k_kc_reduce, dim3(kc_blocks(nT, upper), 16, outs.n), dim3(256 * kRedGroups), 0, s, P,
-                       kc_blocks(nT, upper), kc_block_rows(nT), n, upper ? 1 : 0, outs, accumulate);
+void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& outs, int accumulate, hipStream_t s,
+                      const JUnpack* ju) {
+    static_assert(256 * kRedGroups == 128 * kJuGroups, "one workgroup size");
+    require(outs.n >= 1 && outs.n <= 2 * kMaxPairs && n > 0 && n <= nT * TILE, "kc_reduce");
+    const int nblk = kc_blocks(nT, upper);
+    const int nj = ju ? ju->ntp * (TILE2 / 128) * ju->np : 0;
+    hipLaunchKernelGGL(k_kc_reduce, dim3(nblk, 16, outs.n + (nj + 16 * nblk - 1) / (16 * nblk)), dim3(256 * kRedGroups), 0,
+                       s, P, nblk, kc_block_rows(nT), n, upper ? 1 : 0, outs, accumulate, ju ? *ju : JUnpack{});
 }
 
 void launch_add_transpose(const double* M, int n, double* K, int accumulate, hipStream_t s) {

@@ -78,13 +78,14 @@ struct KcOut {
 };
 struct KcOuts {
     int n = 0;
-    KcOut o[kMaxPairs];
+    KcOut o[2 * kMaxPairs];  // K and D of each pair
 };
 // out (+)= sum over the pair's splits; upper: written with its mirror image (exactly symmetric)
-void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& outs, int accumulate, hipStream_t s);
+// ju (or null): J's reduction, taken along in the same launch
+void launch_kc_reduce(const double* P, int nT, int n, bool upper, const KcOuts& outs, int accumulate, hipStream_t s,
+                      const JUnpack* ju = nullptr);
 // K (+)= M + M^T (n x n)
 void launch_add_transpose(const double* M, int n, double* K, int accumulate, hipStream_t s);
-
 
 // ---- adjoint of E = tr(D (2J - K)), D = C C^T, with ncb 16-column blocks of C ----
 // CB [nbfp/8][ncb][64][2]: C in the row order of X's fragments (rows 8 kb + 4 e + lane / 16)
