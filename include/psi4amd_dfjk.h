@@ -16,14 +16,15 @@
  *   - Host-pointer entry points copy through device buffers owned by the
  *     handle; *_device entry points take device pointers and never copy to the host.
  *   - Calls on one handle are not reentrant; separate handles are independent.
- *   - All device work of a handle runs on one HIP stream (dfjk_set_stream).  The
- *     handle's own stream is a blocking stream, so it is ordered with work on the
- *     legacy default (null) stream; a caller on a non-blocking stream passes that
- *     stream.  *_device calls return with their work queued (host-pointer calls
- *     return after it finished).  Two cases wait for the stream: the structure test
- *     of a non-symmetric pair when the pair form is DFJK_FORM_DETECT (the launch
- *     shapes depend on its outcome; declare the form with dfjk_set_pair_form to
- *     skip it), and the adjoint, which returns E on the host.
+ *   - All device work of a handle is ordered on one HIP stream (dfjk_set_stream; large
+ *     FP64 calls run a memory-bound pass on a second stream, forked from and joined to
+ *     it by events, but not while the stream is captured).  The handle's own stream is a
+ *     blocking stream, so it is ordered with work on the legacy default (null) stream;
+ *     a caller on a non-blocking stream passes that stream.  *_device calls return with
+ *     their work queued (host-pointer calls return after it finished).  Two cases wait
+ *     for the stream: the structure test of a non-symmetric pair when the pair form is
+ *     DFJK_FORM_DETECT (the launch shapes depend on its outcome; declare the form with
+ *     dfjk_set_pair_form to skip it), and the adjoint, which returns E on the host.
  */
 #ifndef PSI4AMD_DFJK_H
 #define PSI4AMD_DFJK_H

@@ -314,6 +314,8 @@ struct dfjk_handle {
     double* hB = nullptr;               // pinned host B, b_doubles
     hipStream_t cstream = nullptr;      // copy stream (default priority, ordered by events)
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
+    hipStream_t jstream = nullptr;      // streaming passes beside MFMA-bound kernels (see SideStream)
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     DevBuf ws_stage[2], ws_stage32, ws_stage32t;
     // range-separated exchange: Bw = M (P|erf(omega r)/r|mn), same layout and fit as B
     DevBuf dBw;
@@ -380,6 +382,49 @@ void ensure_stream(dfjk_handle* h) {
     if (!h->own_stream) hcheck(hipStreamCreateWithFlags(&h->own_stream, hipStreamDefault), "hipStreamCreate");
     if (!h->stream) h->stream = h->own_stream;
     h->timer.s = h->stream;
+}
+
+// Work beside the handle's stream: fork() orders the side stream after what is queued on the handle's, join()
+// the handle's after the side stream, so to a caller everything still runs on the handle's.  A fork that is not
+// joined (an exception) is waited for on the host.
+struct SideStream {
+    dfjk_handle* h;
+    bool open = false;
+    explicit SideStream(dfjk_handle* hh) : h(hh) {}
+    hipStream_t fork() {
+        if (!h->jstream) {
+            hcheck(hipStreamCreateWithFlags(&h->jstream, hipStreamNonBlocking), "side stream");
+            hcheck(hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming), "event");
+            hcheck(hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming), "event");
+        }
+        hcheck(hipEventRecord(h->ev_fork, h->stream), "fork");
+        hcheck(hipStreamWaitEvent(h->jstream, h->ev_fork, 0), "fork");
+        open = true;
+        return h->jstream;
+    }
+    void join() {
+        if (!open) return;
+        open = false;
+        hcheck(hipEventRecord(h->ev_join, h->jstream), "join");
+        hcheck(hipStreamWaitEvent(h->stream, h->ev_join, 0), "join");
+    }
+    ~SideStream() {
+        if (open) (void)hipStreamSynchronize(h->jstream);
+    }
+};
+// Is a pass over `bytes` of memory worth its own stream beside kernels that the MFMA pipes bound?  The fork and
+// join cost a few us: J's second FP64 pass gains from 160 MB on (678 -> 645 us, a third of the pass) and
+// nothing at 22 MB ((H2O)4); at 3.9 GB the build takes 5.72 ms instead of 6.24.  In the mixed precisions, whose K
+// kernels fill the registers and the LDS, J beside K gained nothing (BF16x3) or lost 4 % (FP32).
+// Not while the stream is captured, nor where phases are timed.
+bool worth_side_stream(const dfjk_handle* h, double bytes) {
+    if (h->timer.on || bytes < 64e6) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusNone;
 }
 
 // Tile geometry from the function-pair mask (tile-granular screening).
@@ -1697,6 +1742,13 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         for (int i = 0; i < 2; ++i) hcheck(hipEventRecord(h->ev_free[i], s), "record");
         stage_block(h, 0, qblk);
     }
+    const bool beside = doJ && !h->ooc && !wk.fixed() &&
+                        worth_side_stream(h, static_cast<double>(nq_total) * qs * sizeof(double));
+    SideStream side(h);
+    auto j_pass = [&](hipStream_t js) {
+        launch_j2(g, JSource{JSource::F64, h->dB.as<double>() + static_cast<size_t>(q0) * qs}, dvec + q0, ldd, np,
+                  nq_total, jchunk, Jpart, jstride, js);
+    };
     for (int blk = 0; blk < nblocks; ++blk) {
         const int qa = q0 + blk * qblk, nq = std::min(qblk, q1 - qa);
         const double* b64;
@@ -1721,6 +1773,7 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
             }
             tm.end(T_J, ej);
         }
+        if (beside && blk + 1 == nblocks) j_pass(side.fork());
         hipEvent_t e1 = tm.begin();
         for (int k = 0; k < 2; ++k)
             if (segs[k].n) {
@@ -1734,8 +1787,10 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     const JUnpack* pju = nullptr;
     if (doJ && !h->ooc) {
         hipEvent_t ej = tm.begin();
-        launch_j2(g, JSource{JSource::F64, h->dB.as<double>() + static_cast<size_t>(q0) * qs}, dvec + q0, ldd, np,
-                  nq_total, jchunk, Jpart, jstride, s);
+        if (beside)
+            side.join();
+        else
+            j_pass(s);
         ju = prepare_j_unpack(g, Jpart, jstride, jn, jout, np, nbf, 1.0, accumulate, s);
         pju = &ju;  // its sums are taken along by the first reduction below
         tm.end(T_J, ej);
@@ -2595,7 +2650,11 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
         if (h->ooc) hcheck(hipEventRecord(h->ev_free[blk & 1], s), "record");
         launch_dpart_reduce(dpart, nq, nrg, ncb, dr, dvec + qa, h->naux, s);
         launch_adj_z(CB, X, nT, ncb, nq, dvec + qa, Z, epart + static_cast<size_t>(qa - q0) * nzw, s);
-        if (dEdC) launch_adj_dc(X, Z, nT, ncb, nk, nq, nsp, part, blk > 0 ? 1 : 0, s);
+        // dE/dC beside dE/dB, which is bound by its writes
+        SideStream side(h);
+        if (dEdC)
+            launch_adj_dc(X, Z, nT, ncb, nk, nq, nsp, part, blk > 0 ? 1 : 0,
+                          gam && worth_side_stream(h, static_cast<double>(nn) * nq * sizeof(double)) ? side.fork() : s);
         const int ga = std::max(qa, uq0), gb = std::min(qa + nq, uq1);
         if (gam && ga < gb) {
             double* out = gam_host ? Gb : gam_dev + static_cast<size_t>(ga - uq0) * nn;
@@ -2605,6 +2664,7 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
                 copy_settled(gam_host + static_cast<size_t>(ga - uq0) * nn, Gb, nn * (gb - ga) * sizeof(double),
                              hipMemcpyDeviceToHost, s, "download dE/dB");
         }
+        side.join();
     }
     if (dEdC) launch_adj_dc_reduce(part, nsp, nT, ncb, nbf, nocc, 4.0, dEdC, s);
     if (E) {
@@ -2674,7 +2734,10 @@ int dfjk_destroy(dfjk_handle* h) {
         if (!h) return;
         if (h->own_stream) (void)hipStreamSynchronize(h->own_stream);
         if (h->cstream) (void)hipStreamSynchronize(h->cstream);
-        hipStream_t s = h->own_stream, cs = h->cstream;
+        if (h->jstream) (void)hipStreamSynchronize(h->jstream);
+        hipStream_t s = h->own_stream, cs = h->cstream, js = h->jstream;
+        if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
+        if (h->ev_join) (void)hipEventDestroy(h->ev_join);
         for (int i = 0; i < 2; ++i) {
             if (h->ev_copied[i]) (void)hipEventDestroy(h->ev_copied[i]);
             if (h->ev_free[i]) (void)hipEventDestroy(h->ev_free[i]);
@@ -2686,6 +2749,7 @@ int dfjk_destroy(dfjk_handle* h) {
         if (h->ev_cmap) (void)hipEventDestroy(h->ev_cmap);
         delete h;
         if (cs) (void)hipStreamDestroy(cs);
+        if (js) (void)hipStreamDestroy(js);
         if (s) (void)hipStreamDestroy(s);
     });
 }

@@ -193,3 +193,28 @@ def test_memory_of_finished_handles_is_reused_and_given_back(gpu_available):
     before = torch.cuda.mem_get_info()[0]
     trim_memory()
     assert torch.cuda.mem_get_info()[0] > before
+
+
+def test_j_beside_k_on_a_caller_stream(gpu_available):
+    """A build large enough (B 72 MB) for J's second pass to run on its own stream: results, and repeated
+    builds queued back to back on a caller's stream with the outputs read on that stream."""
+    import torch
+
+    announce("nbf 256 naux 245 on a side stream")
+    nbf, naux = 256, 245
+    jk, B = _tensor(nbf, naux, 12)
+    rng = np.random.default_rng(6)
+    Cs = [rng.standard_normal((nbf, 24)) for _ in range(3)]
+    s = torch.cuda.Stream()
+    jk.set_stream(s.cuda_stream)
+    with torch.cuda.stream(s):
+        dC = [torch.tensor(C, device="cuda") for C in Cs]
+        outs = []
+        for C in dC:
+            D, J, K = (torch.empty(nbf, nbf, dtype=torch.float64, device="cuda") for _ in range(3))
+            jk.compute_device([C.data_ptr()], [], [24], [D.data_ptr()], [J.data_ptr()], [K.data_ptr()])
+            outs.append([x.clone() for x in (D, J, K)])
+    s.synchronize()
+    for C, o in zip(Cs, outs):
+        _check(B, C, C, *(x.cpu().numpy() for x in o))
+    jk.set_stream(0)
