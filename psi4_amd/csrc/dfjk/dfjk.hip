@@ -174,6 +174,57 @@ size_t device_free_bytes() {
     return free_b + dev_pool().held(dev);
 }
 
+// A second stream of a handle, with the events that order it.
+struct SideQueue {
+    int dev = -1;
+    hipStream_t s = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
+};
+// Side queues of finished handles, for the next ones: a new stream costs up to 1 ms.  At most 8, idle.
+class SideQueues {
+   public:
+    SideQueue take() {
+        int dev = 0;
+        hcheck(hipGetDevice(&dev), "hipGetDevice");
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            for (size_t i = 0; i < free_.size(); ++i)
+                if (free_[i].dev == dev) {
+                    const SideQueue q = free_[i];
+                    free_.erase(free_.begin() + i);
+                    return q;
+                }
+        }
+        SideQueue q;
+        q.dev = dev;
+        hcheck(hipEventCreateWithFlags(&q.fork, hipEventDisableTiming), "event");
+        hcheck(hipEventCreateWithFlags(&q.join, hipEventDisableTiming), "event");
+        hcheck(hipStreamCreateWithFlags(&q.s, hipStreamNonBlocking), "side stream");
+        return q;
+    }
+    void give(const SideQueue& q) {
+        if (hipStreamSynchronize(q.s) == hipSuccess) {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (free_.size() < 8) {
+                free_.push_back(q);
+                return;
+            }
+        }
+        (void)hipEventDestroy(q.fork);
+        (void)hipEventDestroy(q.join);
+        (void)hipStreamDestroy(q.s);
+    }
+
+   private:
+    std::mutex mu_;
+    std::vector<SideQueue> free_;
+};
+// never destroyed: the runtime may be gone when static objects are
+SideQueues& side_queues() {
+    static SideQueues* p = new SideQueues;
+    return *p;
+}
+
 // Growable device buffer.  At least 1 MiB: the builds of a small system then fit what the first one
 // allocated, whatever their precision and form (an allocation costs as much as such a build).
 struct DevBuf {
@@ -314,8 +365,7 @@ struct dfjk_handle {
     double* hB = nullptr;               // pinned host B, b_doubles
     hipStream_t cstream = nullptr;      // copy stream (default priority, ordered by events)
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
-    hipStream_t jstream = nullptr;      // streaming passes beside MFMA-bound kernels (see SideStream)
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    SideQueue side;                     // streaming passes beside MFMA-bound kernels (see SideStream)
     DevBuf ws_stage[2], ws_stage32, ws_stage32t;
     // range-separated exchange: Bw = M (P|erf(omega r)/r|mn), same layout and fit as B
     DevBuf dBw;
@@ -392,24 +442,20 @@ struct SideStream {
     bool open = false;
     explicit SideStream(dfjk_handle* hh) : h(hh) {}
     hipStream_t fork() {
-        if (!h->jstream) {
-            hcheck(hipStreamCreateWithFlags(&h->jstream, hipStreamNonBlocking), "side stream");
-            hcheck(hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming), "event");
-            hcheck(hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming), "event");
-        }
-        hcheck(hipEventRecord(h->ev_fork, h->stream), "fork");
-        hcheck(hipStreamWaitEvent(h->jstream, h->ev_fork, 0), "fork");
+        if (!h->side.s) h->side = side_queues().take();
+        hcheck(hipEventRecord(h->side.fork, h->stream), "fork");
+        hcheck(hipStreamWaitEvent(h->side.s, h->side.fork, 0), "fork");
         open = true;
-        return h->jstream;
+        return h->side.s;
     }
     void join() {
         if (!open) return;
         open = false;
-        hcheck(hipEventRecord(h->ev_join, h->jstream), "join");
-        hcheck(hipStreamWaitEvent(h->stream, h->ev_join, 0), "join");
+        hcheck(hipEventRecord(h->side.join, h->side.s), "join");
+        hcheck(hipStreamWaitEvent(h->stream, h->side.join, 0), "join");
     }
     ~SideStream() {
-        if (open) (void)hipStreamSynchronize(h->jstream);
+        if (open) (void)hipStreamSynchronize(h->side.s);
     }
 };
 // Is a pass over `bytes` of memory worth its own stream beside kernels that the MFMA pipes bound?  The fork and
@@ -2734,10 +2780,8 @@ int dfjk_destroy(dfjk_handle* h) {
         if (!h) return;
         if (h->own_stream) (void)hipStreamSynchronize(h->own_stream);
         if (h->cstream) (void)hipStreamSynchronize(h->cstream);
-        if (h->jstream) (void)hipStreamSynchronize(h->jstream);
-        hipStream_t s = h->own_stream, cs = h->cstream, js = h->jstream;
-        if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
-        if (h->ev_join) (void)hipEventDestroy(h->ev_join);
+        if (h->side.s) side_queues().give(h->side);
+        hipStream_t s = h->own_stream, cs = h->cstream;
         for (int i = 0; i < 2; ++i) {
             if (h->ev_copied[i]) (void)hipEventDestroy(h->ev_copied[i]);
             if (h->ev_free[i]) (void)hipEventDestroy(h->ev_free[i]);
@@ -2749,7 +2793,6 @@ int dfjk_destroy(dfjk_handle* h) {
         if (h->ev_cmap) (void)hipEventDestroy(h->ev_cmap);
         delete h;
         if (cs) (void)hipStreamDestroy(cs);
-        if (js) (void)hipStreamDestroy(js);
         if (s) (void)hipStreamDestroy(s);
     });
 }

@@ -24,13 +24,23 @@ __device__ inline double ld1(const double* base, unsigned off) {
     return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
 }
 
+// 1 / sqrt(x): the hardware's estimate (better than 2^-22) and one step of third order, e = 1 - x y^2,
+// y + y e (1/2 + 3/8 e), which leaves (5/16) e^3 < 2^-66; a sixth of the latency of a root and a division.
+__device__ inline double rsqrt_refined(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+
 // ------------------------------------------------------------------ L_kk^-1
 // One workgroup, the block in registers: thread (ty, tx) holds rows ty + 32 a, columns tx + 32 b.  At
 // step k, with r = 1 / sqrt(T_kk), row i > k takes T_ij -= l_i w_j, l_i = T_ik r, where column j > k
 // still holds A (w_j = l_j) and column j < k already holds L^-1 (w_j = T_kj r); row k becomes row k of
 // L^-1.  Row and column k go through LDS, double buffered: one barrier a step.  Bound by that chain
-// (sqrt, division, barrier, LDS): 128 steps take 88 us (114 us when every wave computes the root);
-// factor and inverse on the host, with the copies to and from it, took 7 ms per 256 rows.
+// (root, barrier, LDS): 128 steps take 74 us, of the 32 x 32 blocks only those that still change and lie on or
+// below the diagonal (88 us with every block and a division; 114 us when every wave computes the
+// root); factor and inverse on the host, with the copies to and from it, took 7 ms per 256 rows.
 __global__ __launch_bounds__(1024) void k_chol_inverse(const double* __restrict__ A, int lda, int nb, int k0,
                                                        double* __restrict__ X, int ldx, double* __restrict__ LiT,
                                                        int* __restrict__ info) {
@@ -46,35 +56,36 @@ __global__ __launch_bounds__(1024) void k_chol_inverse(const double* __restrict_
             T[a][b] = (i < nb && j <= i) ? A[static_cast<size_t>(i) * lda + j] : (i == j ? 1.0 : 0.0);
         }
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll 1
         for (int kk = 0; kk < 32; ++kk) {
             const int k = 32 * kb + kk, par = kk & 1;
             if (tx == kk) {
 #pragma unroll
-                for (int a = 0; a < 4; ++a) cb[par][ty + 32 * a] = T[a][kb];
+                for (int a = kb; a < 4; ++a) cb[par][ty + 32 * a] = T[a][kb];
                 // the pivot's reciprocal root, by the one wave that holds it
                 if (ty == kk) {
                     if (!(T[kb][kb] > 0.0)) atomicMin(info, k0 + k);
-                    rb[par] = 1.0 / sqrt(T[kb][kb]);
+                    rb[par] = rsqrt_refined(T[kb][kb]);
                 }
             }
             if (ty == kk)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) vb[par][tx + 32 * b] = T[kb][b];
+                for (int b = 0; b <= kb; ++b) vb[par][tx + 32 * b] = T[kb][b];
             __syncthreads();
             const double r = rb[par];
             double l[4], w[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) l[a] = cb[par][ty + 32 * a] * r;
+            for (int a = kb; a < 4; ++a) l[a] = cb[par][ty + 32 * a] * r;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const int j = tx + 32 * b;
                 w[b] = (j < k ? vb[par][j] : cb[par][j]) * r;
             }
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = kb; a < 4; ++a)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
+                for (int b = 0; b <= a; ++b) {
                     const int i = ty + 32 * a, j = tx + 32 * b;
                     if (i > k)
                         T[a][b] = j == k ? -l[a] * r : fma(-l[a], w[b], T[a][b]);
@@ -82,6 +93,7 @@ __global__ __launch_bounds__(1024) void k_chol_inverse(const double* __restrict_
                         T[a][b] = j < k ? w[b] : r;
                 }
         }
+    }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
