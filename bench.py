@@ -360,9 +360,9 @@ def main():
     achieved = flops_per_launch / (ms_per_launch * 1e-3) / 1e12
     roofline = {"bound": "mfma", "achieved": round(achieved, 3), "peak": PEAK[headline], "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK[headline], 4), "traffic": None,
-                "kernel": ({"fp64": "k_ht_mfma<double>", "fp32": "k_ht_mfma<float>", "bf16x3": "k_ht_bf3"}[headline]
+                "kernel": ({"fp64": "k_ht_f64", "fp32": "k_ht_f32", "bf16x3": "k_ht_bf3"}[headline]
                            + " (half-transform X_Q = B_Q C)") if dom == "HT" else
-                          ({"fp64": "k_kgemm_mfma<double>", "fp32": "k_kgemm_mfma<float>", "bf16x3": "k_kgemm_bf3"}[headline]
+                          ({"fp64": "k_kc_f64", "fp32": "k_kc_f32", "bf16x3": "k_kgemm_bf3"}[headline]
                            + " (K = sum_Q X_Q X_Q^T)"),
                 "launches_per_build": nlaunch / args.steps, "ms_per_launch": round(ms_per_launch, 4),
                 "algorithmic_flops_per_launch": flops_per_launch}

@@ -184,12 +184,14 @@ __device__ __forceinline__ void ht_body(const double* __restrict__ BQ, const int
     }
 }
 
-// Bound by the FP64 MFMA pipes (91 % busy at 2.3 GHz, where a library product of 8192^3 reaches
-// 72.6 TFLOP/s): 3000 Q at nbf 1500 / 300 columns take 60.4 ms (67 TFLOP/s of the 2 nbf^2 ncol
-// products) against 76.1 ms through LDS with 128 x 320 tiles and a barrier per 8 rows of the sum;
+// Bound by the FP64 MFMA pipes (90 % busy at 2.3 GHz, where a library product of 8192^3 reaches
+// 72.6 TFLOP/s): 2000 Q at nbf 1500 / 300 columns take 39.5 ms (68 TFLOP/s of the 2 nbf^2 ncol
+// products) against 50.7 through LDS with 128 x 320 tiles and a barrier per 8 rows of the sum;
 // nbf 576 / 120 columns / 2784 Q 3.8 ms against 5.8.  Columns are cut into near-equal groups of at
 // most 80, in 16s: 80 columns cost 5 blocks, not two 64s.  Four waves per workgroup: the column groups
-// of one row block mostly share a CU's vector cache (one wave per workgroup: 62.1 ms).
+// of one row block mostly share a CU's vector cache (one wave per workgroup: 3 % slower).  64 x 128 and
+// 64 x 160 with one wave per SIMD were 8 % slower and spilled; waves that draw their items from counters fill
+// the slots that uneven waves leave empty (a quarter at nbf 413) and were 3-7 % slower all the same.
 template <int RT, int NC>
 __global__ __launch_bounds__(256, 2) void k_ht_f64(
     const double* __restrict__ B, const int* __restrict__ tidx, int nT, int ntp, int nq, const double* __restrict__ CA,
