@@ -227,8 +227,9 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc);
 int dfjk_finalize(dfjk_handle* h);
 
 /* Device memory that handles freed (dfjk_finalize, dfjk_destroy, a buffer that grew) is kept for the next
- * allocations of this library, 12 GiB at most over all handles and devices; it is given back when an
- * allocation fails and by this call. */
+ * allocations of this library, 12 GiB at most over all handles and devices, and so is the pinned staging of
+ * the host-array calls (256 MiB); both are given back by this call, device memory also when an allocation
+ * fails. */
 int dfjk_trim_memory(void);
 
 #ifdef __cplusplus

@@ -174,6 +174,67 @@ size_t device_free_bytes() {
     return free_b + dev_pool().held(dev);
 }
 
+// Pinned staging that handles gave back (idle: every call that fills it waits for the stream), kept for the
+// next ones, at most kPinPool bytes: allocating and freeing a few MB costs 2 ms of a handle's first call with
+// host arrays.
+constexpr size_t kPinPool = size_t(256) << 20;
+class PinPool {
+   public:
+    // at least need bytes (*cap of them), or nullptr: no pinned memory
+    char* take(size_t need, size_t* cap) {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            size_t best = free_.size();
+            for (size_t i = 0; i < free_.size(); ++i)
+                if (free_[i].second >= need && (best == free_.size() || free_[i].second < free_[best].second)) best = i;
+            if (best < free_.size()) {
+                char* p = free_[best].first;
+                *cap = free_[best].second;
+                total_ -= *cap;
+                free_.erase(free_.begin() + best);
+                return p;
+            }
+        }
+        // whole powers of two from 4 MiB on, so that the arrays of a call's return fit where its inputs did
+        size_t size = size_t(4) << 20;
+        while (size < need) size *= 2;
+        char* p = nullptr;
+        if (hipHostMalloc(reinterpret_cast<void**>(&p), size, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        *cap = size;
+        return p;
+    }
+    void give(char* p, size_t cap) {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (total_ + cap <= kPinPool) {
+                free_.emplace_back(p, cap);
+                total_ += cap;
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    void trim() {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (auto& f : free_) (void)hipHostFree(f.first);
+        free_.clear();
+        total_ = 0;
+    }
+
+   private:
+    std::mutex mu_;
+    std::vector<std::pair<char*, size_t>> free_;
+    size_t total_ = 0;
+};
+// never destroyed: the runtime may be gone when static objects are
+PinPool& pin_pool() {
+    static PinPool* p = new PinPool;
+    return *p;
+}
+
 // A second stream of a handle, with the events that order it.
 struct SideQueue {
     int dev = -1;
@@ -2357,16 +2418,14 @@ bool pin_room(dfjk_handle* h, const std::vector<HostCopy>& x) {
     for (const HostCopy& c : x) need += c.n * sizeof(double);
     if (need > kPinBytes) return false;
     if (need > h->io_pin_cap) {
-        if (h->io_pin) hcheck(hipHostFree(h->io_pin), "hipHostFree");
+        if (h->io_pin) {
+            hcheck(hipStreamSynchronize(h->stream), "staging");  // an upload may still read it
+            pin_pool().give(h->io_pin, h->io_pin_cap);
+        }
         h->io_pin = nullptr;
         h->io_pin_cap = 0;
-        const size_t cap = std::max<size_t>(need, size_t(1) << 20);
-        if (hipHostMalloc(reinterpret_cast<void**>(&h->io_pin), cap, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            h->io_pin = nullptr;
-            return false;
-        }
-        h->io_pin_cap = cap;
+        h->io_pin = pin_pool().take(need, &h->io_pin_cap);
+        if (!h->io_pin) return false;
     }
     return true;
 }
@@ -2789,7 +2848,7 @@ int dfjk_destroy(dfjk_handle* h) {
         if (h->hB) (void)hipHostFree(h->hB);
         if (h->cmap_pin) (void)hipHostFree(h->cmap_pin);
         if (h->sign_pin) (void)hipHostFree(h->sign_pin);
-        if (h->io_pin) (void)hipHostFree(h->io_pin);
+        if (h->io_pin) pin_pool().give(h->io_pin, h->io_pin_cap);
         if (h->ev_cmap) (void)hipEventDestroy(h->ev_cmap);
         delete h;
         if (cs) (void)hipStreamDestroy(cs);
@@ -3220,7 +3279,10 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc) {
 }
 
 int dfjk_trim_memory(void) {
-    return guarded([&] { dev_pool().trim(); });
+    return guarded([&] {
+        dev_pool().trim();
+        pin_pool().trim();
+    });
 }
 
 int dfjk_finalize(dfjk_handle* h) {
