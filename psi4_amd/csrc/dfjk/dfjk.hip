@@ -1389,11 +1389,20 @@ const float* ensure_B32(dfjk_handle* h) {
     return h->dB32.as<float>();
 }
 // tile-transposed FP32 copy, read by the BF16 half-transform for blocks used as (J, I)
+// (and the plain one with it, where that is missing too)
 void ensure_B32T(dfjk_handle* h) {
     if (!h->dB32T.p) {
-        require_copy_room(b_doubles(h) * sizeof(float));
-        float* p = h->dB32T.get<float>(b_doubles(h));
-        launch_to_f32_t(h->dB.as<double>(), p, b_doubles(h), h->stream);
+        const size_t n = b_doubles(h);
+        const bool both = !h->dB32.p;
+        require_copy_room((both ? 2 : 1) * n * sizeof(float));
+        try {
+            float* plain = both ? h->dB32.get<float>(n) : nullptr;
+            launch_to_f32_t(h->dB.as<double>(), plain, h->dB32T.get<float>(n), n, h->stream);
+        } catch (...) {  // no copy without its contents
+            if (both) h->dB32.release();
+            h->dB32T.release();
+            throw;
+        }
     }
 }
 void invalidate_copies(dfjk_handle* h) {
@@ -2029,8 +2038,8 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
                                  "not exist yet; run one dfjk_compute_device at this precision first");
         // J reads the FP32 copy in both mixed modes (2^-24 relative; a BF16 hi + lo pair's
         // 2^-17 would make the J error of a density change dominate its K error)
-        if (prec != DFJK_PREC_FP64) ensure_B32(h);
         if (prec == DFJK_PREC_BF16X3 && doK) ensure_B32T(h);
+        if (prec != DFJK_PREC_FP64) ensure_B32(h);
     }
 
     // J workspace in core: the symmetrised tile-packed density, d_Q, the d_Q partials per
@@ -2247,13 +2256,14 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
             hipEvent_t e0 = tm.begin();
             if (prec != DFJK_PREC_FP64) {
                 float* c = wk.get<float>(h->ws_stage32, qs * qblk);
-                launch_to_f32(st, c, nel, s);
                 b32 = c;
-            }
-            if (prec == DFJK_PREC_BF16X3 && doK) {
-                float* c = wk.get<float>(h->ws_stage32t, qs * qblk);
-                launch_to_f32_t(st, c, nel, s);
-                b32t = c;
+                if (prec == DFJK_PREC_BF16X3 && doK) {
+                    float* ct = wk.get<float>(h->ws_stage32t, qs * qblk);
+                    launch_to_f32_t(st, c, ct, nel, s);
+                    b32t = ct;
+                } else {
+                    launch_to_f32(st, c, nel, s);
+                }
             }
             tm.end(T_OTHER, e0);
         }

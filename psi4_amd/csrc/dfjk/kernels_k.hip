@@ -774,13 +774,25 @@ __global__ void k_to_f32(const double* __restrict__ src, float* __restrict__ dst
          i += static_cast<size_t>(gridDim.x) * blockDim.x)
         dst[i] = static_cast<float>(src[i]);
 }
-// Same, each 32x32 tile transposed: dst[t][r][c] = src[t][c][r] (the half-transform reads these
-// for the blocks it uses in the transposed orientation).
-__global__ void k_to_f32_t(const double* __restrict__ src, float* __restrict__ dst, size_t n) {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const size_t e = i % TILE2, base = i - e;
-        dst[i] = static_cast<float>(src[base + (e % TILE) * TILE + e / TILE]);
+// FP32 with each 32x32 tile transposed, dstT[t][r][c] = src[t][c][r] (the half-transform reads these
+// for the blocks it uses in the transposed orientation), and with dst the plain FP32 copy too, from one
+// read of src.  The tile is turned in LDS, so both sides move whole lines: bound by HBM, 3.9 GB in 1.6
+// ms with both copies (apart 1.0 + 1.55, the transposed one reading every line twice).
+__global__ __launch_bounds__(256) void k_to_f32_t(const double* __restrict__ src, float* __restrict__ dst,
+                                                  float* __restrict__ dstT, size_t ntile) {
+    __shared__ float T[TILE][TILE + 1];
+    const int r = threadIdx.x >> 3, c = 4 * (threadIdx.x & 7);
+    for (size_t t = blockIdx.x; t < ntile; t += gridDim.x) {
+        const size_t o = t * TILE2 + 4 * threadIdx.x;
+        const double2 a = *reinterpret_cast<const double2*>(src + o), b = *reinterpret_cast<const double2*>(src + o + 2);
+        const v4f_t v = {static_cast<float>(a.x), static_cast<float>(a.y), static_cast<float>(b.x),
+                         static_cast<float>(b.y)};
+        if (dst) *reinterpret_cast<v4f_t*>(dst + o) = v;
+        __syncthreads();  // the tile before has been read
+#pragma unroll
+        for (int k = 0; k < 4; ++k) T[r][c + k] = v[k];
+        __syncthreads();
+        *reinterpret_cast<v4f_t*>(dstT + o) = v4f_t{T[c][r], T[c + 1][r], T[c + 2][r], T[c + 3][r]};
     }
 }
 
@@ -901,9 +913,11 @@ void launch_kgemm_bf3(const uint16_t* Ah, const uint16_t* Al, const uint16_t* Bh
 void launch_to_f32(const double* src, float* dst, size_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_to_f32, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
 }
-void launch_to_f32_t(const double* src, float* dst, size_t n, hipStream_t s) {
+void launch_to_f32_t(const double* src, float* dst, float* dstT, size_t n, hipStream_t s) {
     require(n % TILE2 == 0, "to_f32_t");
-    hipLaunchKernelGGL(k_to_f32_t, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_to_f32_t, dim3(static_cast<unsigned>(std::min<size_t>(n / TILE2, 8192))), dim3(256), 0, s, src,
+                       dst, dstT, n / TILE2);
 }
 void launch_pack_cT_bf(const double* src, int ldsrc, int nbf, const int* cmap, uint16_t* hi, uint16_t* lo, int nbfp,
                        int ldc, hipStream_t s) {

@@ -35,8 +35,9 @@ void launch_kgemm_bf3(const uint16_t* Ah, const uint16_t* Al, const uint16_t* Bh
 
 // Precision copies and operand packing (cmap: destination column -> source column or -1).
 void launch_to_f32(const double* src, float* dst, size_t n, hipStream_t s);
-// FP32 with every 32x32 tile transposed (the blocks the BF16 half-transform reads as (J,I)).
-void launch_to_f32_t(const double* src, float* dst, size_t n, hipStream_t s);
+// FP32 with every 32x32 tile transposed (the blocks the BF16 half-transform reads as (J,I)) and, with dst,
+// the plain FP32 copy beside it.
+void launch_to_f32_t(const double* src, float* dst, float* dstT, size_t n, hipStream_t s);
 void launch_pack_cT_bf(const double* src, int ldsrc, int nbf, const int* cmap, uint16_t* hi, uint16_t* lo, int nbfp,
                        int ldc, hipStream_t s);
 // s[i] = +1 / -1 if Cr[:,i] is bitwise +/- Cl[:,(i + shift) % ncol], else 0.
