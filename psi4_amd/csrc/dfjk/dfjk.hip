@@ -87,12 +87,6 @@ void copy_settled(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, 
     hcheck(hipMemcpy(dst, src, bytes, kind), what);
     hcheck(hipDeviceSynchronize(), what);
 }
-void copy2d_settled(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width, size_t rows,
-                    hipMemcpyKind kind, hipStream_t s, const char* what) {
-    hcheck(hipStreamSynchronize(s), what);
-    hcheck(hipMemcpy2D(dst, dpitch, src, spitch, width, rows, kind), what);
-    hcheck(hipDeviceSynchronize(), what);
-}
 
 // Device memory that handles gave back, kept for the next allocation of about the same size: at most
 // kPoolBytes in all.  hipMalloc costs 0.1-0.4 ms, and 30 ms per GB once the process has cycled through
