@@ -12,6 +12,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -1481,6 +1482,11 @@ struct PairIn {
     int ncol = 0;
     double *D = nullptr, *J = nullptr, *K = nullptr;
 };
+// do two arrays of na and nb doubles share memory?
+bool overlap(const double* a, size_t na, const double* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return a && b && x < y + nb * sizeof(double) && y < x + na * sizeof(double);
+}
 // Two structured non-symmetric forms are recognised (bitwise column tests on the device) and kept
 // symmetric:
 //  * signed: every column of Cr is +/- the same column of Cl (the incremental
@@ -2606,11 +2612,18 @@ void compute_impl(dfjk_handle* h, int n, const double* const* Cl, const double* 
         p.D = dD;
         p.J = dJ;
         p.K = dK;
-        // a pair that reads or writes what an earlier one of its batch writes waits for it
+        // a pair that reads or writes what an earlier one of its batch writes, or writes what one reads (every D of
+        // a batch may be written before any C is packed), waits for it
         bool clash = false;
-        for (const PairIn& o : batch)
-            for (const double* w : {o.D, o.J, o.K})
-                clash |= w && (w == p.cl || w == p.cr || w == p.D || w == p.J || w == p.K);
+        const size_t csz = static_cast<size_t>(h->nbf) * p.ncol;
+        for (const PairIn& o : batch) {
+            const size_t osz = static_cast<size_t>(h->nbf) * o.ncol;
+            for (const double* w : {o.D, o.J, o.K}) {
+                clash |= overlap(w, nn, p.cl, csz) || overlap(w, nn, p.cr, csz);
+                for (const double* v : {p.D, p.J, p.K}) clash |= overlap(w, nn, v, nn);
+            }
+            for (const double* v : {p.D, p.J, p.K}) clash |= overlap(v, nn, o.cl, osz) || overlap(v, nn, o.cr, osz);
+        }
         const bool alone = arena || h->precision != DFJK_PREC_FP64 || !h->do_K || !p.K;
         if (alone || clash || (!batch.empty() && (p.J == nullptr) != (batch[0].J == nullptr))) flush();
         batch.push_back(p);
