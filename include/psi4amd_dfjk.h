@@ -165,7 +165,7 @@ int dfjk_get_Bw_dense(dfjk_handle* h, int q0, int q1, double* out);
  * n density pairs; Cr == NULL means lr_symmetric (C_right = C_left, jk.cc:597-602).
  * Cl[i], Cr[i]: nbf x ncol[i] row-major.  D/J/K outputs: nbf x nbf (any may be NULL).
  * J and K are overwritten unless accumulate != 0 (then J += ..., K += ...).  The pairs take effect in
- * order: an output may lie where another pair's array is or was. */
+ * order, and D, J, K of a pair too: an output may lie where another pair's array is or was. */
 int dfjk_compute(dfjk_handle* h, int n, const double* const* Cl, const double* const* Cr, const int* ncol,
                  double* const* D, double* const* J, double* const* K, int accumulate);
 int dfjk_compute_device(dfjk_handle* h, int n, const double* const* Cl, const double* const* Cr, const int* ncol,

@@ -1687,7 +1687,15 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     // D of symmetric pairs comes from the columns packed for d_Q, and its partial sums lie behind K's: two
     // launches less ((H2O)4 with host arrays: 112 -> 107 us)
     bool d_packed = h->do_J && !accumulate;
-    for (int p = 0; p < np; ++p) d_packed &= pr[p].J && form[p].sym && !form[p].is_signed();
+    // outputs of a pair that share memory are written one after the other: D, J, K
+    bool apart = true;
+    const size_t nn = static_cast<size_t>(nbf) * nbf;
+    for (int p = 0; p < np; ++p) {
+        d_packed &= pr[p].J && form[p].sym && !form[p].is_signed();
+        apart &= !overlap(pr[p].D, nn, pr[p].J, nn) && !overlap(pr[p].D, nn, pr[p].K, nn) &&
+                 !overlap(pr[p].J, nn, pr[p].K, nn);
+    }
+    d_packed &= apart;
     if (!d_packed) {
         hipEvent_t e0 = tm.begin();
         const size_t mark = wk.used;
@@ -1825,7 +1833,6 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     double* P = wk.get<double>(h->ws_P, psize);
     int ncross = 0;
     for (int p = 0; p < np; ++p) ncross += form[p].cross ? 1 : 0;
-    const size_t nn = static_cast<size_t>(nbf) * nbf;
     double* M = ncross ? wk.get<double>(h->ws_M, ncross * nn) : nullptr;
     int rt = ht_row_tiles(nT, qblk, ncb);
     const size_t dq = static_cast<size_t>(ht_row_groups(nT, 1)) * ncb;  // d partials per Q, at most
@@ -1907,8 +1914,12 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
             side.join();
         else
             j_pass(s);
-        ju = prepare_j_unpack(g, Jpart, jstride, jn, jout, np, nbf, 1.0, accumulate, s);
-        pju = &ju;  // its sums are taken along by the first reduction below
+        if (apart) {
+            ju = prepare_j_unpack(g, Jpart, jstride, jn, jout, np, nbf, 1.0, accumulate, s);
+            pju = &ju;  // its sums are taken along by the first reduction below
+        } else {
+            launch_j_unpack(g, Jpart, jstride, jn, jout, np, nbf, 1.0, accumulate, s);
+        }
         tm.end(T_J, ej);
     }
     hipEvent_t e2 = tm.begin();

@@ -1,5 +1,5 @@
-"""Device calls whose arrays overlap: the pairs of a call are taken in order, as if each were finished before the
-next is begun.
+"""Device calls whose arrays overlap: the pairs of a call are taken in order, and so are the outputs D, J, K of a
+pair, as if each were finished before the next is begun.
 
 The reference replays a call on a numpy copy of the same memory.  Tolerance: arrays that a pair reads may be
 results of an earlier one, so an error bound would have to follow the chain; the products of at most two
@@ -71,3 +71,11 @@ def test_outputs_that_reach_into_the_next_input(jk):
     pairs = [{"L": 0, "R": NN, "ncol": 17, "D": 2 * NN, "J": 3 * NN, "K": 4 * NN},
              {"L": 5 * NN - 100, "R": 6 * NN, "ncol": 17, "D": NN - 300, "J": 7 * NN, "K": 8 * NN}]
     _run(jk, 9 * NN, pairs)
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_outputs_of_one_pair_in_one_array(jk, accumulate):
+    """J and K added up in one array, and D, J and K all written to one array (K stays)."""
+    announce(f"outputs of a pair in one array, accumulate {accumulate}")
+    _run(jk, 5 * NN, [{"L": 0, "ncol": 9, "D": NN, "J": 2 * NN, "K": 2 * NN},
+                      {"L": 3 * NN, "ncol": 9, "D": 4 * NN, "J": 4 * NN, "K": 4 * NN}], accumulate)
