@@ -25,6 +25,7 @@
 #include "../ints/basis_build.hpp"
 #include "../ints/ints.hpp"
 #include "../ints/hostlinalg.hpp"
+#include "host_copies.hpp"
 #include "kernels.hpp"
 #include "kernels_f32.hpp"
 #include "kernels_f64.hpp"
@@ -2429,11 +2430,6 @@ void reset_timers(dfjk_handle* h) {
 // an idle device each, copy_settled: an (H2O)4 build took 147 us with them, 109 with these).  Up to kPinBytes per direction and
 // call; larger transfers, or no pinned memory, take copy_settled.
 constexpr size_t kPinBytes = size_t(64) << 20;
-struct HostCopy {
-    double* dev;
-    double* host;
-    size_t n;  // doubles
-};
 bool pin_room(dfjk_handle* h, const std::vector<HostCopy>& x) {
     size_t need = 0;
     for (const HostCopy& c : x) need += c.n * sizeof(double);
@@ -2449,18 +2445,6 @@ bool pin_room(dfjk_handle* h, const std::vector<HostCopy>& x) {
         if (!h->io_pin) return false;
     }
     return true;
-}
-// one copy per run of adjacent device arrays
-template <class F>
-void for_runs(const std::vector<HostCopy>& x, F&& f) {
-    size_t off = 0;
-    for (size_t i = 0; i < x.size();) {
-        size_t j = i + 1, n = x[i].n;
-        while (j < x.size() && x[j].dev == x[j - 1].dev + x[j - 1].n) n += x[j++].n;
-        f(x[i].dev, off, n * sizeof(double));
-        off += n * sizeof(double);
-        i = j;
-    }
 }
 // (the staging is free: every call that fills it ends by waiting for the stream)
 void upload_arrays(dfjk_handle* h, const std::vector<HostCopy>& x, const char* what) {
@@ -2512,7 +2496,7 @@ void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool 
             const size_t csz = static_cast<size_t>(h->nbf) * ncol;
             for (const HostCopy& e : upl)
                 if (e.host == c && e.n == csz) return e.dev;
-            upl.push_back({raw, const_cast<double*>(c), csz});
+            upl.push_back({raw, const_cast<double*>(c), csz, h->ws_craw.p});
             raw += csz;
             return upl.back().dev;
         };
@@ -2528,8 +2512,8 @@ void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool 
                 if (!host) return;
                 dev = g;
                 g += nn;
-                if (wanted) down.push_back({dev, host, nn});
-                if (add) upl.push_back({dev, host, nn});
+                if (wanted) down.push_back({dev, host, nn, h->ws_out.p});
+                if (add) upl.push_back({dev, host, nn, h->ws_out.p});
             };
             place(batch[i].D, pr[i].D, true, false);
             place(batch[i].J, pr[i].J, h->do_J, accumulate);
@@ -2681,19 +2665,19 @@ void compute_wk_impl(dfjk_handle* h, int n, const double* const* Cl, const doubl
         if (!device) {
             double* raw = h->ws_craw.get<double>(2 * csz);
             gW = h->ws_out.get<double>(nn);
-            std::vector<HostCopy> upl{{raw, const_cast<double*>(cl), csz}};
+            std::vector<HostCopy> upl{{raw, const_cast<double*>(cl), csz, h->ws_craw.p}};
             cl = raw;
             if (cr) {
-                upl.push_back({raw + csz, const_cast<double*>(cr), csz});
+                upl.push_back({raw + csz, const_cast<double*>(cr), csz, h->ws_craw.p});
                 cr = raw + csz;
             }
-            if (accumulate) upl.push_back({gW, dW, nn});
+            if (accumulate) upl.push_back({gW, dW, nn, h->ws_out.p});
             upload_arrays(h, upl, "upload");
         }
         compute_wk_pair(h, cl, cr, ncol[i], gW, accumulate);
         // lr_symmetric: MemDFJK::compute_JK hermitivitizes wK (MemDFJK.cc:101-107)
         if (!cr) launch_hermitivitize(gW, h->nbf, h->nbf, h->stream);
-        if (!device) download_arrays(h, {{gW, dW, nn}}, "download wK");
+        if (!device) download_arrays(h, {{gW, dW, nn, h->ws_out.p}}, "download wK");
     }
     finish_timers(h);
 }
