@@ -170,7 +170,7 @@ size_t device_free_bytes() {
     return free_b + dev_pool().held(dev);
 }
 
-// Pinned staging that handles gave back (idle: every call that fills it waits for the stream), kept for the
+// Pinned staging that handles gave back (idle: a call that fills it waits for the stream, see StagingWait), kept for the
 // next ones, at most kPinPool bytes: allocating and freeing a few MB costs 2 ms of a handle's first call with
 // host arrays.
 constexpr size_t kPinPool = size_t(256) << 20;
@@ -2446,7 +2446,15 @@ bool pin_room(dfjk_handle* h, const std::vector<HostCopy>& x) {
     }
     return true;
 }
-// (the staging is free: every call that fills it ends by waiting for the stream)
+// A call that fills the staging does not end, by an exception either, before its uploads have read it: the next
+// call, or the handle that the staging goes to, fills it again.
+struct StagingWait {
+    dfjk_handle* h;
+    bool filled;
+    ~StagingWait() {
+        if (filled) (void)hipStreamSynchronize(h->stream);
+    }
+};
 void upload_arrays(dfjk_handle* h, const std::vector<HostCopy>& x, const char* what) {
     if (!pin_room(h, x)) {
         for (const HostCopy& c : x) copy_settled(c.dev, c.host, c.n * sizeof(double), hipMemcpyHostToDevice, h->stream, what);
@@ -2486,6 +2494,7 @@ void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool 
     const int np = static_cast<int>(batch.size());
     std::vector<PairIn> pr(batch);
     std::vector<HostCopy> down;
+    StagingWait staging{h, !device};
     if (!device) {
         // operands to the device, an array that several pairs share once
         size_t csum = 0;
@@ -2542,6 +2551,7 @@ void run_batch(dfjk_handle* h, std::vector<PairIn>& batch, int accumulate, bool 
         for (int i = 0; i < np; ++i) compute_pair(h, pr[i], form[i], accumulate, wk);
     }
     if (!device) download_arrays(h, down, "download");
+    staging.filled = false;  // waited for
 }
 
 // arena: null for the allocating entry points, else the device address of this device's
@@ -2662,6 +2672,7 @@ void compute_wk_impl(dfjk_handle* h, int n, const double* const* Cl, const doubl
         const double* cl = Cl[i];
         const double* cr = Cr ? Cr[i] : nullptr;
         double* gW = dW;
+        StagingWait staging{h, !device};
         if (!device) {
             double* raw = h->ws_craw.get<double>(2 * csz);
             gW = h->ws_out.get<double>(nn);
@@ -2678,6 +2689,7 @@ void compute_wk_impl(dfjk_handle* h, int n, const double* const* Cl, const doubl
         // lr_symmetric: MemDFJK::compute_JK hermitivitizes wK (MemDFJK.cc:101-107)
         if (!cr) launch_hermitivitize(gW, h->nbf, h->nbf, h->stream);
         if (!device) download_arrays(h, {{gW, dW, nn, h->ws_out.p}}, "download wK");
+        staging.filled = false;
     }
     finish_timers(h);
 }
