@@ -196,6 +196,7 @@ class JK {
         }
         if (!initialized_) throw std::runtime_error("JK: initialize() must be called before compute()");
         // outputs are (re)allocated unless accumulating into existing ones of the right count
+        auto zero = [](Arr& a) { std::fill(a.mutable_data(), a.mutable_data() + a.size(), 0.0); };
         if (!accumulate_ || J_.size() != n || (do_wK_ && wK_.size() != n)) {
             D_.clear();
             J_.clear();
@@ -206,7 +207,6 @@ class JK {
                 J_.push_back(Arr({nbf_, nbf_}));
                 K_.push_back(Arr({nbf_, nbf_}));
                 // what compute does not overwrite starts from zero
-                auto zero = [&](Arr& a) { std::fill(a.mutable_data(), a.mutable_data() + a.size(), 0.0); };
                 if (accumulate_ || !do_J_) zero(J_.back());
                 if (accumulate_ || !do_K_) zero(K_.back());
                 if (do_wK_) {
@@ -224,18 +224,31 @@ class JK {
             pj[i] = J_[i].mutable_data();
             pk[i] = K_[i].mutable_data();
         }
+        int rc = DFJK_OK;
+        bool have_jk = false;
         {
             py::gil_scoped_release nogil;
-            check(dfjk_compute(h_, static_cast<int>(n), pl.data(), lr_symmetric ? nullptr : pr.data(), ncol.data(),
-                               pd.data(), do_J_ ? pj.data() : nullptr, do_K_ ? pk.data() : nullptr,
-                               accumulate_ ? 1 : 0));
-            if (do_wK_) {
+            rc = dfjk_compute(h_, static_cast<int>(n), pl.data(), lr_symmetric ? nullptr : pr.data(), ncol.data(),
+                              pd.data(), do_J_ ? pj.data() : nullptr, do_K_ ? pk.data() : nullptr, accumulate_ ? 1 : 0);
+            have_jk = rc == DFJK_OK;
+            if (have_jk && do_wK_) {
                 std::vector<double*> pw(n);
                 for (size_t i = 0; i < n; ++i) pw[i] = wK_[i].mutable_data();
-                check(dfjk_compute_wK(h_, static_cast<int>(n), pl.data(), lr_symmetric ? nullptr : pr.data(),
-                                      ncol.data(), pw.data(), accumulate_ ? 1 : 0));
+                rc = dfjk_compute_wK(h_, static_cast<int>(n), pl.data(), lr_symmetric ? nullptr : pr.data(), ncol.data(),
+                                     pw.data(), accumulate_ ? 1 : 0);
             }
         }
+        if (rc != DFJK_OK && !accumulate_) {
+            // what a failed build leaves to be read is zero, not memory that nothing has written
+            for (size_t i = 0; i < n; ++i) {
+                if (!have_jk) {
+                    zero(J_[i]);
+                    zero(K_[i]);
+                }
+                if (do_wK_) zero(wK_[i]);
+            }
+        }
+        check(rc);
     }
 
     // Device-pointer variant (torch tensors): pointers as integers.

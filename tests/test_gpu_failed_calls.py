@@ -49,3 +49,17 @@ def test_the_call_after_a_refused_one(gpu_available):
         a = np.einsum("qmn,mn->q", np.abs(B), np.abs(C) @ np.abs(C).T)
         tol = 2 * (NBF * NBF + NAUX + 14) * 2.0 ** -53 * np.einsum("q,qmn->mn", a, np.abs(B))
         assert np.all(np.abs(jk.J()[0] - np.einsum("q,qmn->mn", d, B)) <= tol)
+
+
+def test_outputs_of_a_refused_call_are_zero(gpu_available):
+    """J and K hold zeros after a refused call, not memory that nothing has written."""
+    announce("J and K after a refused call")
+    jk = _handle()
+    rng = np.random.default_rng(1)
+    for _ in range(3):
+        jk.C_clear()
+        jk.C_left_add(rng.standard_normal((NBF, 12)))
+        jk.compute()               # results that the next arrays' memory may still hold
+        assert jk.J()[0].any()
+        _refused(jk, rng, 11)
+        assert not jk.J()[0].any() and not jk.K()[0].any()
