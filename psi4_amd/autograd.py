@@ -84,8 +84,9 @@ class _SCFEnergy2e(torch.autograd.Function):
         _sync()
         jk.energy_adjoint_device(C.data_ptr(), C.shape[1], dC.data_ptr() if want_C else 0,
                                  dB.data_ptr() if want_B else 0)
-        # E.backward() passes 1: no pass over dE/dB (as large as B) for that
-        if float(gE) != 1.0:
+        # E.backward() passes 1: no pass over dE/dB (as large as B) for that, unless the gradients are to be
+        # differentiated in gE themselves (create_graph)
+        if gE.requires_grad or float(gE) != 1.0:
             if want_C:
                 dC.mul_(gE)
             if want_B:
