@@ -282,11 +282,11 @@ SideQueues& side_queues() {
     return *p;
 }
 
-// Growable device buffer.  At least 1 MiB: the builds of a small system then fit what the first one
-// allocated, whatever their precision and form (an allocation costs as much as such a build).
+// Growable device buffer of at least `least` bytes.
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    size_t least = 256;
     int dev = 0;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
@@ -299,7 +299,7 @@ struct DevBuf {
     }
     template <class T>
     T* get(size_t count) {
-        const size_t need = std::max<size_t>(count * sizeof(T), size_t(1) << 20);
+        const size_t need = std::max(count * sizeof(T), least);
         if (need > bytes) {
             release();
             hcheck(hipGetDevice(&dev), "hipGetDevice");
@@ -323,6 +323,16 @@ struct DevBuf {
     T* as() const {
         return static_cast<T*>(p);
     }
+};
+// A workspace array of a handle: the builds of a small system then mostly fit what the first one allocated,
+// whatever their precision and form (an allocation costs as much as such a build).  A handle holds a dozen of them,
+// so with 1 MiB and tables of 1 MiB too the smallest handle (nbf 8) took 18.0 MiB, now 3.2.
+struct WsBuf : DevBuf {
+    WsBuf() { least = size_t(256) << 10; }
+};
+// An array that lives for one step of the set-up; its block goes to the next step by way of the pool.
+struct TmpBuf : DevBuf {
+    TmpBuf() { least = size_t(1) << 20; }
 };
 
 inline int round_up(int a, int b) { return (a + b - 1) / b * b; }
@@ -423,7 +433,7 @@ struct dfjk_handle {
     hipStream_t cstream = nullptr;      // copy stream (default priority, ordered by events)
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
     SideQueue side;                     // streaming passes beside MFMA-bound kernels (see SideStream)
-    DevBuf ws_stage[2], ws_stage32, ws_stage32t;
+    WsBuf ws_stage[2], ws_stage32, ws_stage32t;
     // range-separated exchange: Bw = M (P|erf(omega r)/r|mn), same layout and fit as B
     DevBuf dBw;
     double bw_omega = -1.0;         // omega dBw was built for (< 0: none)
@@ -445,8 +455,8 @@ struct dfjk_handle {
     double bw_alpha = 1.0, bw_beta = 0.0;
     std::vector<double> fit_M;      // host metric factor, kept for rebuilding Bw after an omega change
     // workspace
-    DevBuf ws_craw, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_out, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
-    DevBuf ws_CB, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
+    WsBuf ws_craw, ws_D, ws_W, ws_dpart, ws_d, ws_Jpart, ws_XL, ws_XR, ws_P, ws_out, ws_G, ws_sign, ws_c32, ws_cbf, ws_cmap, ws_CA, ws_CD, ws_M;
+    WsBuf ws_CB, ws_red, ws_Y, ws_PC, ws_gam, ws_dc;
     // column map of the half-transform: the device copy is re-uploaded (from pinned memory,
     // asynchronously) only when it changes
     std::vector<int> cmap_dev;          // what ws_cmap holds
@@ -726,7 +736,7 @@ std::vector<double> device_metric_factor(dfjk_handle* h, const std::vector<doubl
     constexpr int NB = kCholBlock;
     const hipStream_t s = h->stream;
     const size_t nn = static_cast<size_t>(n) * n;
-    DevBuf dA, dP, dPT, dT, dL, dinfo;
+    TmpBuf dA, dP, dPT, dT, dL, dinfo;
     h->dM_ready = false;
     double* A = dA.get<double>(nn);
     double* X = h->ws_G.get<double>(nn);
@@ -797,7 +807,7 @@ std::vector<double> device_metric_eigen(dfjk_handle* h, const std::vector<double
     const size_t nn = static_cast<size_t>(n) * n;
     const hipStream_t s = h->stream;
     h->dM_ready = false;
-    DevBuf dA, dS, dRT, dw, de, df, dinfo;
+    TmpBuf dA, dS, dRT, dw, de, df, dinfo;
     double* A = dA.get<double>(nn);
     double* w = dw.get<double>(n);
     double* e = de.get<double>(n);
@@ -867,7 +877,7 @@ std::vector<double> metric_factor(dfjk_handle* h, bool want_host) {
     // (P|Q) on the device when the kernels cover the auxiliary shells (then it stays there for
     // the factorisation), else on the host
     const bool host_factor = h->fitting == DFJK_FIT_CHOLESKY && std::getenv("PSI4AMD_HOST_FACTOR");
-    DevBuf dJ;
+    TmpBuf dJ;
     std::vector<double> Jm;
     const bool on_dev = !host_factor && gpu_metric(h, dJ);
     if (!on_dev) {
@@ -906,7 +916,7 @@ void fit_on_device(dfjk_handle* h, const std::vector<double>& M, const std::vect
     double* dM = h->ws_G.get<double>(static_cast<size_t>(na) * na);
     if (!h->dM_ready)
         copy_settled(dM, M.data(), M.size() * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload metric factor");
-    DevBuf dMF;
+    TmpBuf dMF;
     double* MF = dMF.get<double>(fit_packed_size(na));
     launch_fit_pack(dM, na, MF, h->stream);
     // chunk of columns so that the staging buffer stays <= ~1 GiB
@@ -950,7 +960,7 @@ std::vector<int64_t> tile_dst(const dfjk_handle* h);
 // Device copies of the shell tables of a "primary" basis pb (and an auxiliary basis ab), the
 // solid-harmonic rows l = 0..4 and the host engine's Boys grid; fills the table fields of a.
 struct IntTables {
-    DevBuf ps, as, pe, pc, ae, ac, c2s, boys;
+    TmpBuf ps, as, pe, pc, ae, ac, c2s, boys;
 };
 void upload_int_tables(const Basis& pb, const Basis* ab, IntTables& t, ThreeIndexArgs& a) {
     auto shells = [](const Basis& b, std::vector<GpuShell>& sh, std::vector<double>& e, std::vector<double>& c) {
@@ -1044,7 +1054,7 @@ bool gpu_schwarz(dfjk_handle* h, double* fun_max) {
     ThreeIndexArgs a;
     IntTables tabs;
     upload_int_tables(pb, nullptr, tabs, a);
-    DevBuf d_pairs, d_out;
+    TmpBuf d_pairs, d_out;
     d_pairs.get<int2>(std::max<size_t>(1, pall.size()));
     copy_settled(d_pairs.p, pall.data(), pall.size() * sizeof(int2), hipMemcpyHostToDevice, h->stream, "upload pairs");
     const size_t nn = static_cast<size_t>(pb.nbf) * pb.nbf;
@@ -1082,7 +1092,7 @@ void run_three_index(dfjk_handle* h, const Basis& pb, const Basis& ab, const std
     ThreeIndexArgs a;
     IntTables tabs;
     upload_int_tables(pb, &ab, tabs, a);
-    DevBuf d_dst, d_pairs, d_afun;
+    TmpBuf d_dst, d_pairs, d_afun;
     auto up = [&](DevBuf& b, const void* src, size_t bytes) {
         b.get<char>(bytes);
         copy_settled(b.p, src, bytes, hipMemcpyHostToDevice, h->stream, "upload integral tables");
@@ -1180,7 +1190,7 @@ void fit_device_A(dfjk_handle* h, const std::vector<double>& M, const double* A,
     double* dM = h->ws_G.get<double>(static_cast<size_t>(na) * na);
     if (!h->dM_ready)
         copy_settled(dM, M.data(), M.size() * sizeof(double), hipMemcpyHostToDevice, h->stream, "upload metric factor");
-    DevBuf dMF;
+    TmpBuf dMF;
     double* MF = dMF.get<double>(fit_packed_size(na));
     launch_fit_pack(dM, na, MF, h->stream);
     if (!host_dst) {
