@@ -228,10 +228,14 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc);
 int dfjk_finalize(dfjk_handle* h);
 
 /* Device memory that handles freed (dfjk_finalize, dfjk_destroy, a buffer that grew) is kept for the next
- * allocations of this library, 12 GiB at most over all handles and devices, and so is the pinned staging of
- * the host-array calls (256 MiB); both are given back by this call, device memory also when an allocation
- * fails. */
+ * allocations of this library: over all handles and devices 12 GiB at most, and no more than 1 GiB or an eighth of the
+ * device memory that would be free otherwise, whichever is more, when a block comes in.  So is the pinned staging of the
+ * host-array calls (256 MiB).  Both are given back by this call, device memory also when an allocation of
+ * this library fails. */
 int dfjk_trim_memory(void);
+/* The device memory kept so, in bytes, instead of the 12 GiB; 0: freed memory goes back to the device at once (a
+ * process that shares its card).  What is held beyond it is given back by the call. */
+int dfjk_set_memory_pool(size_t bytes);
 
 #ifdef __cplusplus
 }

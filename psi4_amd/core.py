@@ -20,6 +20,7 @@ PREC_BF16X3 = _core.PREC_BF16X3
 FIT_CHOLESKY = _core.FIT_CHOLESKY
 FIT_EIGEN = _core.FIT_EIGEN
 trim_memory = _core.trim_memory
+set_memory_pool = _core.set_memory_pool
 
 _SUPPORTED = ("DF", "MEM_DF")
 

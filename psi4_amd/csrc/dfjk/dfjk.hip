@@ -90,16 +90,20 @@ void copy_settled(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, 
     hcheck(hipDeviceSynchronize(), what);
 }
 
-// Device memory that handles gave back, kept for the next allocation of about the same size: at most
-// kPoolBytes in all.  hipMalloc costs 0.1-0.4 ms, and 30 ms per GB once the process has cycled through
-// the card's memory (freed pages are cleared before they are handed out again): a set-up of
-// (H2O)16 allocates 3.4 GB, which took 105 of its 121 ms in such a process.  A block enters the pool
-// when the device is idle, as hipFree would leave it, so any stream and thread may take it.  Blocks
-// are given back oldest first when the bound is reached, all of them when an allocation fails, and by
-// dfjk_trim_memory; free-memory decisions count them as free.  The bound takes the whole workspace of a
-// build (8 GiB of X and its partial sums), so that a new handle's first build waits for no cleared
-// pages: with 4 GiB, nbf 1500 / naux 6000 after other handles took 1.55 s instead of 0.2.
+// Device memory that handles gave back, kept for the next allocation of about the same size.  hipMalloc
+// costs 0.1-0.4 ms, and 30 ms per GB once the process has cycled through the card's memory (freed pages are
+// cleared before they are handed out again): a set-up of (H2O)16 allocates 3.4 GB, which took 105 of its 121 ms
+// in such a process.  A block enters the pool when the device is idle, as hipFree would leave it, so any stream
+// and thread may take it.  At most kPoolBytes over all devices, or what dfjk_set_memory_pool says, and of that no
+// more than kPoolAlways or 1/kPoolShare of what would be free without the pool, whichever is more: on a card that
+// others fill (torch's allocator, a second process) the pool gives way at the next block that comes in.  Blocks
+// are given back oldest first, all of them when an allocation of this library fails, and by dfjk_trim_memory;
+// free-memory decisions count them as free.  The bound takes the whole workspace of a build (8 GiB of X and its
+// partial sums), so that a new handle's first build waits for no cleared pages: with 4 GiB, nbf 1500 / naux 6000
+// after other handles took 1.55 s instead of 0.2.
 constexpr size_t kPoolBytes = size_t(12) << 30;
+constexpr size_t kPoolAlways = size_t(1) << 30;
+constexpr int kPoolShare = 8;
 class DevPool {
    public:
     // a block of at least need bytes on device dev (its size in *got), or nullptr
@@ -120,13 +124,16 @@ class DevPool {
     }
     void give(void* p, size_t bytes, int dev) {
         int cur = -1;
-        if (bytes <= kPoolBytes && hipGetDevice(&cur) == hipSuccess && cur == dev &&
-            hipDeviceSynchronize() == hipSuccess) {
+        if (hipGetDevice(&cur) == hipSuccess && cur == dev && hipDeviceSynchronize() == hipSuccess) {
             std::lock_guard<std::mutex> lock(mu_);
-            while (total_ + bytes > kPoolBytes) drop_oldest();
-            blocks_.push_back({p, bytes, dev});
-            total_ += bytes;
-            return;
+            const size_t most = bound(bytes, dev);
+            const bool keep = bytes <= most;
+            while (total_ + (keep ? bytes : 0) > most) drop_oldest();
+            if (keep) {
+                blocks_.push_back({p, bytes, dev});
+                total_ += bytes;
+                return;
+            }
         }
         (void)hipFree(p);
     }
@@ -134,11 +141,14 @@ class DevPool {
         std::lock_guard<std::mutex> lock(mu_);
         while (!blocks_.empty()) drop_oldest();
     }
+    void set_limit(size_t bytes) {
+        std::lock_guard<std::mutex> lock(mu_);
+        limit_ = bytes;
+        while (total_ > limit_) drop_oldest();
+    }
     size_t held(int dev) {
         std::lock_guard<std::mutex> lock(mu_);
-        size_t n = 0;
-        for (const Block& b : blocks_) n += b.dev == dev ? b.bytes : 0;
-        return n;
+        return held_on(dev);
     }
 
    private:
@@ -147,6 +157,22 @@ class DevPool {
         size_t bytes;
         int dev;
     };
+    size_t held_on(int dev) const {
+        size_t n = 0;
+        for (const Block& b : blocks_) n += b.dev == dev ? b.bytes : 0;
+        return n;
+    }
+    // What the pool may hold once a block of `bytes` on the current device dev comes in.  The device is asked for
+    // its free memory when a block of 64 MiB or more does (at every block, it cost a set-up 2 %).
+    size_t bound(size_t bytes, int dev) {
+        if (bytes >= size_t(64) << 20) {
+            size_t free_b = 0, all = 0;
+            share_ = kPoolAlways;
+            if (hipMemGetInfo(&free_b, &all) == hipSuccess)
+                share_ = std::max(share_, (free_b + held_on(dev) + bytes) / kPoolShare);
+        }
+        return std::min(limit_, share_);
+    }
     void drop_oldest() {
         (void)hipFree(blocks_.front().p);
         total_ -= blocks_.front().bytes;
@@ -154,7 +180,7 @@ class DevPool {
     }
     std::mutex mu_;
     std::vector<Block> blocks_;
-    size_t total_ = 0;
+    size_t total_ = 0, limit_ = kPoolBytes, share_ = kPoolAlways;
 };
 // never destroyed: the runtime may be gone when static objects are
 DevPool& dev_pool() {
@@ -3310,6 +3336,10 @@ int dfjk_get_out_of_core(dfjk_handle* h, int* ooc) {
         if (!ooc) fail(DFJK_ERR_ARG, "null output");
         *ooc = h->ooc ? 1 : 0;
     });
+}
+
+int dfjk_set_memory_pool(size_t bytes) {
+    return guarded([&] { dev_pool().set_limit(bytes); });
 }
 
 int dfjk_trim_memory(void) {

@@ -444,7 +444,9 @@ PYBIND11_MODULE(_core, m) {
     m.attr("FIT_CHOLESKY") = static_cast<int>(DFJK_FIT_CHOLESKY);
     m.attr("FIT_EIGEN") = static_cast<int>(DFJK_FIT_EIGEN);
     m.def("trim_memory", [] { check(dfjk_trim_memory()); },
-          "give back the device memory kept from finished JK objects (4 GiB at most)");
+          "give back the device memory (12 GiB at most) and the pinned staging (256 MiB) kept from finished JK objects");
+    m.def("set_memory_pool", [](size_t bytes) { check(dfjk_set_memory_pool(bytes)); }, py::arg("bytes"),
+          "bytes of device memory that may be kept from finished JK objects (12 GiB; 0: none)");
     py::class_<JK, std::shared_ptr<JK>>(m, "JK", py::dynamic_attr())
         .def_static("build_JK", &JK::build, py::arg("basis"), py::arg("aux"), py::arg("do_wK") = false,
                     py::arg("doubles") = static_cast<size_t>(256000000))

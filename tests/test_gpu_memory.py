@@ -40,3 +40,50 @@ def test_small_handles_are_small(gpu_available):
     print(f"  {each:.2f} MiB per handle", flush=True)
     assert each < 4.0
     del first, held
+
+
+def test_the_pool_keeps_to_its_setting(gpu_available):
+    """A handle with 0.5 GiB of B leaves it behind for the next one by default, and nothing with a pool of 0 bytes."""
+    from psi4_amd.core import set_memory_pool, trim_memory
+    announce("a finished handle of 0.5 GiB, pool of 0 bytes and by default")
+    gc.collect()
+    trim_memory()
+    size = 68 * 990 * 8192             # naux x tile pairs of 44 x 32 functions x 8 KiB
+    try:
+        for pool, kept in ((0, False), (12 << 30, True)):
+            set_memory_pool(pool)
+            before = _free()
+            jk = _handle(44 * 32, 68)
+            assert before - _free() > size
+            del jk
+            gc.collect()
+            assert (before - _free() > size // 2) == kept
+        set_memory_pool(1 << 20)       # what is held beyond a new bound goes back
+        assert before - _free() < size // 2
+    finally:
+        set_memory_pool(12 << 30)
+
+
+def test_the_pool_gives_way_on_a_full_card(gpu_available):
+    """With about 16 GiB free, 3 GiB of a finished handle are more than an eighth of it and go back to the device."""
+    import torch
+
+    from psi4_amd.core import trim_memory
+    announce("a finished handle of 3 GiB with 16 GiB free")
+    gc.collect()
+    trim_memory()
+    torch.cuda.empty_cache()
+    rest = _free() - (16 << 30)
+    if rest < 0:
+        pytest.skip("less than 16 GiB free on this device")
+    fill = torch.empty(rest, dtype=torch.uint8, device="cuda")
+    try:
+        before = _free()
+        jk = _handle(1408, 400)        # 44 x 45 / 2 tiles of 8 KiB per Q: 3.02 GiB
+        assert before - _free() > 3 << 30
+        del jk
+        gc.collect()
+        assert before - _free() < 1 << 30
+    finally:
+        del fill
+        torch.cuda.empty_cache()
