@@ -27,6 +27,16 @@ def _sync():
     torch.cuda.current_stream().synchronize()
 
 
+def _empty(shape, device):
+    """A float64 device array; where torch finds no memory, the memory kept from finished JK objects is given back."""
+    try:
+        return torch.empty(shape, dtype=torch.float64, device=device)
+    except torch.OutOfMemoryError:
+        from .core import trim_memory
+        trim_memory()
+        return torch.empty(shape, dtype=torch.float64, device=device)
+
+
 def _tensor_twin(jk, nbf, naux):
     """Tensor-level JK of jk's shape that holds a caller-supplied B (made once, kept on jk)."""
     twin = getattr(jk, "_autograd_twin", None)
@@ -80,7 +90,7 @@ class _SCFEnergy2e(torch.autograd.Function):
         dB = None
         if want_B:
             info = jk.info()                 # the twin: its whole auxiliary range is in use
-            dB = torch.empty((info["naux"], info["nbf"], info["nbf"]), dtype=torch.float64, device=C.device)
+            dB = _empty((info["naux"], info["nbf"], info["nbf"]), C.device)
         _sync()
         jk.energy_adjoint_device(C.data_ptr(), C.shape[1], dC.data_ptr() if want_C else 0,
                                  dB.data_ptr() if want_B else 0)

@@ -843,14 +843,27 @@ std::vector<double> device_metric_eigen(dfjk_handle* h, const std::vector<double
     else
         copy_settled(A, Jm.data(), nn * sizeof(double), hipMemcpyHostToDevice, s, "upload metric");
     rocblas_handle rb = nullptr;
-    if (rocblas_create_handle(&rb) != rocblas_status_success) fail(DFJK_ERR_DEVICE, "rocblas_create_handle failed");
+    // the library's own workspace comes from the device, not from the pool: with the memory that is kept
+    // there given back, a call that found none is made again (it fails before it touches A)
+    auto with_memory = [](auto&& call) {
+        rocblas_status st = call();
+        if (st == rocblas_status_memory_error) {
+            (void)hipGetLastError();  // the failed allocation's status
+            dev_pool().trim();
+            st = call();
+        }
+        return st;
+    };
+    if (with_memory([&] { return rocblas_create_handle(&rb); }) != rocblas_status_success)
+        fail(DFJK_ERR_DEVICE, "rocblas_create_handle failed");
     struct RbGuard {
         rocblas_handle r;
         ~RbGuard() { rocblas_destroy_handle(r); }
     } guard{rb};
     if (rocblas_set_stream(rb, s) != rocblas_status_success) fail(DFJK_ERR_DEVICE, "rocblas_set_stream failed");
     // the metric is symmetric, so its row-major storage is also its column-major storage
-    const rocblas_status st = rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, n, A, n, w, e, info);
+    const rocblas_status st = with_memory(
+        [&] { return rocsolver_dsyevd(rb, rocblas_evect_original, rocblas_fill_upper, n, A, n, w, e, info); });
     if (st != rocblas_status_success)
         fail(DFJK_ERR_DEVICE, std::string("rocsolver_dsyevd: ") + rocblas_status_to_string(st));
     std::vector<double> a(n);
