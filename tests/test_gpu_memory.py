@@ -87,3 +87,39 @@ def test_the_pool_gives_way_on_a_full_card(gpu_available):
     finally:
         del fill
         torch.cuda.empty_cache()
+
+
+def test_two_threads_share_the_pools(gpu_available):
+    """Handles made, used and dropped by two threads at once: memory, staging and side queues go from one to the other.
+    Every build of every thread has to finish, whatever kind of error would stop it.  J against numpy at the
+    rounding of its sums, on sums of absolute values."""
+    import threading
+
+    announce("two threads, six handles each")
+    shapes = [(100, 90, 20), (61, 90, 20), (150, 70, 33), (24, 116, 5), (256, 250, 24), (97, 40, 8)]
+    done, errors = [], []
+
+    def work(t):
+        try:
+            for i in range(len(shapes)):
+                nbf, naux, ncol = shapes[(i + 3 * t) % len(shapes)]
+                jk = _handle(nbf, naux)
+                jk.fill_synthetic(nbf)
+                B = jk.get_B_dense(0, naux)
+                C = np.random.default_rng(i).standard_normal((nbf, ncol))
+                jk.C_left_add(C)
+                jk.compute()
+                flat, D = B.reshape(naux, -1), (C @ C.T).reshape(-1)
+                Da = (np.abs(C) @ np.abs(C).T).reshape(-1)
+                tol = 2 * (nbf * nbf + naux + ncol + 2) * 2.0 ** -53 * ((np.abs(flat) @ Da) @ np.abs(flat))
+                assert np.all(np.abs(jk.J()[0].reshape(-1) - (flat @ D) @ flat) <= tol)
+                done.append((t, i))
+        except Exception as e:  # noqa: BLE001
+            errors.append((t, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors and sorted(done) == [(t, i) for t in range(2) for i in range(len(shapes))]
