@@ -2828,11 +2828,7 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
         if (h->ooc) hcheck(hipEventRecord(h->ev_free[blk & 1], s), "record");
         launch_dpart_reduce(dpart, nq, nrg, ncb, dr, dvec + qa, h->naux, s);
         launch_adj_z(CB, X, nT, ncb, nq, dvec + qa, Z, epart + static_cast<size_t>(qa - q0) * nzw, s);
-        // dE/dC beside dE/dB, which is bound by its writes
-        SideStream side(h);
-        if (dEdC)
-            launch_adj_dc(X, Z, nT, ncb, nk, nq, nsp, part, blk > 0 ? 1 : 0,
-                          gam && worth_side_stream(h, static_cast<double>(nn) * nq * sizeof(double)) ? side.fork() : s);
+        if (dEdC) launch_adj_dc(X, Z, nT, ncb, nk, nq, nsp, part, blk > 0 ? 1 : 0, s);
         const int ga = std::max(qa, uq0), gb = std::min(qa + nq, uq1);
         if (gam && ga < gb) {
             double* out = gam_host ? Gb : gam_dev + static_cast<size_t>(ga - uq0) * nn;
@@ -2842,7 +2838,6 @@ void adjoint_impl(dfjk_handle* h, const double* dC, int nocc, double* E, double*
                 copy_settled(gam_host + static_cast<size_t>(ga - uq0) * nn, Gb, nn * (gb - ga) * sizeof(double),
                              hipMemcpyDeviceToHost, s, "download dE/dB");
         }
-        side.join();
     }
     if (dEdC) launch_adj_dc_reduce(part, nsp, nT, ncb, nbf, nocc, 4.0, dEdC, s);
     if (E) {
