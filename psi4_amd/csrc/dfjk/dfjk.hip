@@ -2087,7 +2087,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     }
     const size_t qs = static_cast<size_t>(h->ntp) * TILE2;  // elements per Q
     const size_t xq = static_cast<size_t>(f32 ? nbfp : xrows) * ldc;  // X elements per Q
-    const size_t esz = prec == DFJK_PREC_FP64 ? 8 : 4;       // FP64, FP32, or BF16 hi+lo
+    constexpr size_t esz = 4;                                // FP32, or BF16 hi + lo
 
     // resident lower-precision copies (in core); the fixed-workspace entry point allocates
     // none, so an earlier allocating compute at this precision must have made them
@@ -2198,23 +2198,25 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
         nsplit = std::min(choose_nsplit(ntile, std::min(nq_total, 65535)), cap_split);
         P = wk.get<double>(h->ws_P, static_cast<size_t>(nsplit) * ntile * 16384);
     }
-    // contraction passes over k: (kbeg, kend, alpha, column offsets of the two operands)
+    // BF16x3: contraction passes over k (FP32 has segs): (kbeg, kend, alpha, column offsets of the two operands).
+    // Padding columns of X are zero: each pass stops at the contraction's k-step after the last real
+    // column of its group.
     struct Pass {
         int kbeg, kend;
         double alpha;
         size_t offl, offr;
     };
-    // padding columns of X are zero: each pass stops at the contraction's k-step after
-    // the last real column of its group
-    const int kstep = 32;
     std::vector<Pass> passes;
-    if (signed_sym) {
-        if (!plus.empty()) passes.push_back({0, round_up(static_cast<int>(plus.size()), kstep), 1.0, 0, 0});
-        passes.push_back({kplus, kplus + round_up(static_cast<int>(minus.size()), kstep), -1.0, 0, 0});
-    } else if (cross) {
-        passes.push_back({0, round_up(half, kstep), 1.0, 0, static_cast<size_t>(wcross)});
-    } else {
-        passes.push_back({0, std::min(ldc, round_up(ncol, kstep)), 1.0, 0, 0});
+    if (doK && !f32) {
+        const int kstep = 32;
+        if (signed_sym) {
+            if (!plus.empty()) passes.push_back({0, round_up(static_cast<int>(plus.size()), kstep), 1.0, 0, 0});
+            passes.push_back({kplus, kplus + round_up(static_cast<int>(minus.size()), kstep), -1.0, 0, 0});
+        } else if (cross) {
+            passes.push_back({0, round_up(half, kstep), 1.0, 0, static_cast<size_t>(wcross)});
+        } else {
+            passes.push_back({0, std::min(ldc, round_up(ncol, kstep)), 1.0, 0, 0});
+        }
     }
     float* c32 = nullptr;
     uint16_t *cth_l = nullptr, *ctl_l = nullptr, *cth_r = nullptr, *ctl_r = nullptr;
@@ -2233,7 +2235,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
                 cg.g[0] = ColGroup{dCl, nullptr, dmap, ncol, ncol, 0, ncb1};
             }
             launch_pack_frag32(cg, nbf, nbfp, c32, s);
-        } else if (prec == DFJK_PREC_BF16X3) {
+        } else {
             uint16_t* a = wk.get<uint16_t>(h->ws_cbf, 4 * csz);
             cth_l = a;
             ctl_l = a + csz;
@@ -2367,7 +2369,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
                 launch_kc_f32(reinterpret_cast<const float*>(XL), xq, ncb, h->nT, nq, segs, upper, P, blk > 0 ? 1 : 0, s);
                 h->n_kgemm += 1;
             }
-            for (size_t ip = 0; !f32 && ip < passes.size(); ++ip) {
+            for (size_t ip = 0; ip < passes.size(); ++ip) {
                 const Pass& pp = passes[ip];
                 const int acc = (blk > 0 || ip > 0) ? 1 : 0;
                 uint16_t* xl = reinterpret_cast<uint16_t*>(XL) + pp.offl * 16;
