@@ -1393,13 +1393,13 @@ void initialize_basis(dfjk_handle* h) {
 }
 
 // ---------------------------------------------------------------- compute
-// Q-splits of the contraction: at least about 2048 workgroups, a multiple of the 8 XCDs
+// Q-splits of the BF16x3 contraction: at least about 2048 workgroups, a multiple of the 8 XCDs
 // when the batch allows (the contraction maps each split to one XCD).  Among up to three
 // times that many splits that keep >= 32 Q per split, the one whose workgroups fill each
-// XCD's 64 slots (32 CUs x 2 workgroups) in the most nearly whole rounds is taken: the
-// last round of a launch otherwise runs part-empty (e.g. 78 tiles x 32 splits leave 2.5 %
-// of the rounds idle, 72 splits 0.3 %; measured 70.2 -> 68.8 ms for the FP64 contraction
-// at nbf 1500 / naux 6000).
+// XCD's 64 slots (32 CUs x 2 workgroups) in the most nearly whole rounds is taken, so that the
+// last round of a launch does not run part-empty (78 tiles x 32 splits leave 2.5 % of the
+// rounds idle, 72 splits 0.3 %).  At the power limit that is not seen: an increment at nbf 1500 /
+// naux 4000 takes 51.3 ms with the first or the best of those splits, and at nbf 576 they are the same.
 int choose_nsplit(int ntile, int nbatch) {
     const int target = g_kgemm_wgs;
     int ns0 = std::max(1, (target + ntile - 1) / ntile);
@@ -1829,7 +1829,7 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         Jpart = wk.get<double>(h->ws_Jpart, np * jstride);
     };
     if (doJ) {
-        dvec = wk.get<double>(h->ws_d, static_cast<size_t>(np) * ldd);  // at absolute Q (the adjoint reads it)
+        dvec = wk.get<double>(h->ws_d, static_cast<size_t>(np) * ldd);  // at absolute Q
         if (!h->ooc)
             size_j2(nq_total, wk.fixed() ? static_cast<int>(std::max<size_t>(
                                                h->ntp, std::min<size_t>(4096, wk.left() / 8 / (TILE2 * sizeof(double)))))
@@ -2110,7 +2110,7 @@ void compute_pair(dfjk_handle* h, const PairIn& in, const PairForm& form, int ac
     int jchunk = 0, jnchunk = 0, qchunk = 0;
     if (doJ) {
         W = wk.get<double>(h->ws_W, qs);
-        dvec = wk.get<double>(h->ws_d, h->naux);  // d_Q at its absolute Q (the adjoint reads it afterwards)
+        dvec = wk.get<double>(h->ws_d, h->naux);  // d_Q at its absolute Q
         if (!h->ooc) {
             dpart = wk.get<double>(h->ws_dpart, static_cast<size_t>(h->ntp) * h->naux);
             // about 4096 workgroups for the second pass (fewer chunks in a fixed workspace)
