@@ -1619,7 +1619,9 @@ std::vector<PairForm> classify_pairs(dfjk_handle* h, const PairIn* pr, int np, W
 }
 
 // dfjk_compute_device_noalloc, before any launch: the buffers of fixed size, one K split and one
-// auxiliary function's X must fit the scratch array (X blocks and splits then adapt to the rest).
+// auxiliary function's X must fit the scratch array (X blocks and splits then adapt to the rest).  The
+// sizes are those of the BF16x3 path, whose panels (up to 320 columns) and 128 x 128 blocks are padded most; FP64 and FP32
+// need less of each, so what this lets through fits them too.
 void require_scratch(const dfjk_handle* h, int ncol, const Work& wk) {
     if (h->ooc) fail(DFJK_ERR_STATE, "dfjk_compute_device_noalloc needs B in core");
     const int nbf = h->nbf, xrows = (h->nT + 3) / 4 * 128;
@@ -1811,10 +1813,39 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     for (int p = 0; p < np; ++p) njp += h->do_J && pr[p].J ? 1 : 0;
     const bool doJ = njp > 0;
     if (doJ && njp != np) fail(DFJK_ERR_INTERNAL, "J wanted for some pairs of a batch only");
+    const size_t qs = static_cast<size_t>(h->ntp) * TILE2;
+    // Fixed workspace: the bytes of one split per pass (and the cross form's M) and of one Q of X with its d
+    // partials; J's partials and the further splits leave that much.
+    size_t least_p = 0, least_x = 0;
+    // A general pair's sides are transformed one after the other where the arena does not hold both at once (many
+    // more columns than functions: the partner columns of the left side are then not stored either)
+    ColGroups left;
+    if (wk.fixed()) {
+        auto bytes = [&](int nc) { return static_cast<size_t>(nbfp) * 16 * nc * sizeof(double); };
+        for (int k = 0; k < 2; ++k)
+            least_p += (pass[k].size() + (k == 0 && d_packed && pr[0].D ? 1 : 0)) * kc_blocks(nT, k == 0) * 4096 * sizeof(double);
+        if (form[0].cross) least_p += nn * sizeof(double);
+        const size_t pad = 4096;  // alignment
+        auto one_q = [&](int nc) { return bytes(nc) + static_cast<size_t>(ht_row_groups(nT, 1)) * nc * sizeof(double) + pad; };
+        least_x = one_q(cg.ncb);
+        if (form[0].general() &&
+            2 * bytes(cg.ncb) + (h->naux + qs) * sizeof(double) + least_p + least_x + pad > wk.left()) {
+            left = cg;
+            left.n = 1;
+            left.ncb = left.g[0].ncb;
+            cg.n = 1;
+            cg.ncb = left.ncb;
+            cg.g[0] = cg.g[1];
+            cg.g[0].cb0 = dr.cb0[0] = pass[1][0].kb = 0;
+            least_x = one_q(cg.ncb) + bytes(cg.ncb);
+        }
+    }
     const int ncb = cg.ncb, nkx = 2 * ncb;
-    const size_t csz = static_cast<size_t>(nbfp) * 16 * ncb, xq = csz, qs = static_cast<size_t>(h->ntp) * TILE2;
+    const size_t csz = static_cast<size_t>(nbfp) * 16 * ncb, xq = csz;
+    double* CL = left.n ? wk.get<double>(h->ws_CA, csz) : nullptr;
     double* CA = wk.get<double>(h->ws_CA, csz);
     double* CD = doJ ? wk.get<double>(h->ws_CD, csz) : nullptr;
+    if (CL) launch_pack_frag(left, nbf, nbfp, CL, nullptr, s);
     launch_pack_frag(cg, nbf, nbfp, CA, CD, s);
 
     double *dvec = nullptr, *Jpart = nullptr;
@@ -1828,15 +1859,19 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         jstride = static_cast<size_t>(jn) * qs;
         Jpart = wk.get<double>(h->ws_Jpart, np * jstride);
     };
+    auto spare = [&](size_t later) { return wk.left() > later ? wk.left() - later : 0; };
     if (doJ) {
         dvec = wk.get<double>(h->ws_d, static_cast<size_t>(np) * ldd);  // at absolute Q
-        if (!h->ooc)
-            size_j2(nq_total, wk.fixed() ? static_cast<int>(std::max<size_t>(
-                                               h->ntp, std::min<size_t>(4096, wk.left() / 8 / (TILE2 * sizeof(double)))))
-                                         : 4096);
+        int want_wg = 4096;
+        if (wk.fixed()) {
+            const size_t most = spare(least_p + least_x) / (qs * sizeof(double));  // chunks
+            want_wg = static_cast<int>(std::max<size_t>(
+                h->ntp, std::min({size_t(4096), wk.left() / 8 / (TILE2 * sizeof(double)), most * h->ntp})));
+        }
+        if (!h->ooc) size_j2(nq_total, want_wg);
     }
     // Q-blocks
-    const size_t per_q = xq * sizeof(double);
+    const size_t per_q = xq * sizeof(double) * (CL ? 2 : 1);
     int qblk = std::min(nq_total, 65535);
     size_t budget = 0;
     if (!wk.fixed()) {
@@ -1864,9 +1899,11 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         poff[k] = psize;
         for (const Pass& ps : pass[k]) {
             int nsp = kc_choose_splits(nT, k == 0, kc_steps(qblk, ps.nk), nseg, kc_most_splits(nblk * nseg, budget));
-            if (wk.fixed())
+            if (wk.fixed()) {
+                const size_t one = static_cast<size_t>(nblk) * 4096 * sizeof(double) * nseg;
                 nsp = static_cast<int>(std::max<size_t>(
-                    1, std::min<size_t>(nsp, wk.left() / 4 / (static_cast<size_t>(nblk) * 4096 * sizeof(double) * nseg))));
+                    1, std::min({static_cast<size_t>(nsp), wk.left() / 4 / one, 1 + spare(least_p + least_x) / one})));
+            }
             segs[k].s[segs[k].n++] = KcSeg{segs[k].nsplit, nsp, ps.ka, ps.kb, ps.nk, ps.alpha};
             segs[k].nsplit += nsp;
         }
@@ -1897,6 +1934,7 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
     }
     const int nrg = ht_row_groups(nT, rt);
     double* X = wk.get<double>(h->ws_XL, xq * qblk);
+    double* XA = CL ? wk.get<double>(h->ws_XL, xq * qblk) : X;  // the contraction's row operand
     // one partial per Q (one pair, 16 columns, one row group) is d_Q itself
     const bool d_whole = doJ && np == 1 && ncb == 1 && nrg == 1;
     double* dpart = doJ && !d_whole ? wk.get<double>(h->ws_dpart, dq * qblk) : nullptr;
@@ -1934,8 +1972,9 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         }
         hipEvent_t e0 = tm.begin();
         launch_ht_f64(g, b64, nq, CA, CD, ncb, rt, X, d_whole ? dvec + qa : dpart, h->dZero.p, s);
+        if (CL) launch_ht_f64(g, b64, nq, CL, nullptr, ncb, rt, XA, nullptr, h->dZero.p, s);
         tm.end(T_HT, e0);
-        h->n_ht += 1;
+        h->n_ht += CL ? 2 : 1;
         if (doJ) {
             hipEvent_t ej = tm.begin();
             if (!d_whole) launch_dpart_reduce(dpart, nq, nrg, ncb, dr, dvec + qa, ldd, s);
@@ -1950,7 +1989,7 @@ void compute_f64(dfjk_handle* h, const PairIn* pr, const std::vector<PairForm>& 
         hipEvent_t e1 = tm.begin();
         for (int k = 0; k < 2; ++k)
             if (segs[k].n) {
-                launch_kc_f64(X, X, xq, nkx, nT, nq, segs[k], k == 0, P + poff[k], blk > 0 ? 1 : 0, s);
+                launch_kc_f64(XA, X, xq, nkx, nT, nq, segs[k], k == 0, P + poff[k], blk > 0 ? 1 : 0, s);
                 h->n_kgemm += 1;
             }
         tm.end(T_KGEMM, e1);
